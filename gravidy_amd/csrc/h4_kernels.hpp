@@ -278,16 +278,28 @@ __host__ __device__ inline uint32_t pick_iw(uint32_t nact, uint32_t fill16 = DEF
     return best;
 }
 
+// Active particles per work item of the exact kernel for nact active ones.
+// Few get a workgroup each: the ordered add chain bounds it (n = 16385:
+// nact 256 88 us, 117 us with 3 per workgroup; both 170 us at 1024).  More
+// share one, 3 chains on one wave and its term waves busier (nact 4096: 391
+// against 631 us).  From EXACT_WIDE on, one lane per particle fills the CUs
+// (n = 65536: 16.0 ms at any nact up to 65536, against 0.356 us times nact).
+constexpr uint32_t EXACT_WIDE = 45056;
+__host__ __device__ inline uint32_t exact_iw(uint32_t nact) {
+    return nact <= 768 ? 1u : nact < EXACT_WIDE ? 3u : (uint32_t)BS;
+}
+
 // ---------------------------------------------------------------------------
 // Pair terms
 // ---------------------------------------------------------------------------
 
-// Hermite4CPU::force_calculation (Hermite4CPU.cpp:55-82), operation for
-// operation: no contraction, IEEE sqrt and division, same association.
-__device__ __forceinline__ void pair_exact(const double pi[6], double xj,
-                                           double yj, double zj, double vxj,
-                                           double vyj, double vzj, double mj,
-                                           double e2, double fo[6]) {
+// The six terms one pair adds in Hermite4CPU::force_calculation
+// (Hermite4CPU.cpp:55-82), operation for operation: no contraction, IEEE
+// sqrt and division, same association.
+__device__ __forceinline__ void terms_exact(const double pi[6], double xj,
+                                            double yj, double zj, double vxj,
+                                            double vyj, double vzj, double mj,
+                                            double e2, double tm[6]) {
 #pragma clang fp contract(off)
     double rx = xj - pi[0];
     double ry = yj - pi[1];
@@ -306,12 +318,12 @@ __device__ __forceinline__ void pair_exact(const double pi[6], double xj,
 
     double rv = rx * vx + ry * vy + rz * vz;
 
-    fo[0] += (rx * mr3inv);
-    fo[1] += (ry * mr3inv);
-    fo[2] += (rz * mr3inv);
-    fo[3] += (vx * mr3inv - (3 * rv) * rx * mr5inv);
-    fo[4] += (vy * mr3inv - (3 * rv) * ry * mr5inv);
-    fo[5] += (vz * mr3inv - (3 * rv) * rz * mr5inv);
+    tm[0] = (rx * mr3inv);
+    tm[1] = (ry * mr3inv);
+    tm[2] = (rz * mr3inv);
+    tm[3] = (vx * mr3inv - (3 * rv) * rx * mr5inv);
+    tm[4] = (vy * mr3inv - (3 * rv) * ry * mr5inv);
+    tm[5] = (vz * mr3inv - (3 * rv) * rz * mr5inv);
 }
 
 // The FP64 pair loop works with s = sqrt(3) / r and q = s^2 = 3 / r^2:

@@ -191,11 +191,11 @@ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_
     ClPlan pl;
     pl.cmaj = 0;
     if (exact) {
-        pl.iw = BS;
+        pl.iw = exact_iw(nact);
         pl.S = 1;
         pl.tpc = ntiles(e, c);
-        pl.n_it = (nact + BS - 1) / BS;
-        pl.rows = pl.n_it * BS;
+        pl.n_it = (nact + pl.iw - 1) / pl.iw;
+        pl.rows = pl.n_it * pl.iw;
         pl.lanes = 1;
         pl.grid = e.grid;
     } else {
@@ -669,45 +669,174 @@ __device__ __forceinline__ void reduce_subgroups(double fo[6], double *red) {
     }
 }
 
-// FP64_EXACT: one lane per active i, j ascending over the cluster, j == i
-// skipped, exactly Hermite4CPU::update_acc_jrk (Hermite4CPU.cpp:309-336).
-// Writes f[i] directly.  Workgroups stride over the plan's i tiles.
+// FP64_EXACT: the pair terms of Hermite4CPU::update_acc_jrk
+// (Hermite4CPU.cpp:309-336) added in its order, j ascending, j == i skipped.
+// The order makes every component of a particle's sum a chain of n - 1
+// dependent FP64 adds (5.5 ns each on the part), but the terms (some 80
+// instructions, with an IEEE square root and division) do not depend on each
+// other.  One lane per active particle that computes and adds takes 161-235
+// ns per j whatever nact is, until its waves fill the SIMDs; with the terms
+// spread over waves and one wave adding them, an update takes (n = 1024)
+// nact 32: 247 -> 12.6 us, 1024: 250 -> 16 us; (n = 16385) 256: 3870 -> 88
+// us, 4096: 3930 -> 390 us, 16385: 3960 -> 1476 us.
+constexpr uint32_t XW = BS / 64 - 1;  // waves that compute terms; the last one adds them
+
+// Doubles of LDS of an item of IX particles over j tiles of TJ: two buffers
+// of 6 IX rows.  A row's stride of 4 dwords mod 64 lets the adding lanes,
+// one row each, read 16 bytes at a time without bank conflicts, and a wave's
+// term stores are 64 consecutive doubles.
+template <uint32_t IX, uint32_t TJ>
+constexpr uint32_t exact_lds() {
+    return 2 * 6 * IX * (TJ + 2);
+}
+
+// IX active particles against the whole cluster in j tiles of TJ: XW waves
+// compute tile t's terms into one LDS buffer (one pair per lane and unit of
+// one particle x 64 j) while lane 6 x + q of the remaining wave adds
+// component q of particle x of tile t - 1 from the other, in j order.  The
+// adding wave is another one of the four from one workgroup of a CU to the
+// next, so that they do not share a SIMD.  The skipped
+// term (j == i) is stored as +0.0, which leaves every sum as it is (a sum
+// that starts at +0.0 is never -0.0).
+template <uint32_t IX, uint32_t TJ>
+__device__ __forceinline__ void exact_item(const Soa &s, const uint32_t *mv, uint32_t nact,
+                                           uint32_t it, uint32_t j_begin, uint32_t n, double e2,
+                                           double *lds) {
+    constexpr uint32_t TS = TJ + 2, NJ = TJ / 64, UPW = IX * NJ / XW;
+    static_assert(IX * NJ % XW == 0 && 6 * IX <= 64 && TJ % 16 == 0, "units over the term waves");
+    const uint32_t w = ((threadIdx.x >> 6) + (blockIdx.x >> 8)) % (BS / 64);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t k0 = it * IX;
+    const uint32_t tiles = (n + TJ - 1) / TJ;
+    const bool adds = w == XW;
+    // term waves: unit u = w UPW + k is particle u / NJ, j sub-tile u % NJ
+    uint32_t iu[UPW], js[UPW];
+    double pi[UPW][6];
+    double4 ja[UPW], jb[UPW];
+    double acc = 0.0;
+    if (!adds) {
+#pragma unroll
+        for (uint32_t k = 0; k < UPW; ++k) {
+            const uint32_t u = w * UPW + k, a = k0 + u / NJ;
+            iu[k] = mv[a < nact ? a : nact - 1];
+            js[k] = (u % NJ) * 64 + lane;
+            load_predictor(s, iu[k], pi[k]);
+            const uint32_t j = j_begin + min(js[k], n - 1);
+            ja[k] = s.pp[j];
+            jb[k] = s.pv[j];
+        }
+    }
+    for (uint32_t t = 0; t <= tiles; ++t) {
+        if (!adds) {
+            if (t < tiles) {
+                double *buf = lds + (t & 1u) * (6 * IX * TS);
+#pragma unroll
+                for (uint32_t k = 0; k < UPW; ++k) {
+                    const double4 a = ja[k], b = jb[k];
+                    const uint32_t j = t * TJ + js[k];
+                    if (t + 1 < tiles) {  // the next tile's records, under this one's terms
+                        const uint32_t jn = j_begin + min(j + TJ, n - 1);
+                        ja[k] = s.pp[jn];
+                        jb[k] = s.pv[jn];
+                    }
+                    double tm[6];
+                    terms_exact(pi[k], a.x, a.y, a.z, b.x, b.y, b.z, a.w, e2, tm);
+                    double *row = buf + 6 * ((w * UPW + k) / NJ) * TS + js[k];
+                    const bool me = j_begin + j == iu[k];
+                    if (__ballot(me))  // (one tile in n / TJ)
+                        for (uint32_t q = 0; q < 6; ++q) tm[q] = me ? 0.0 : tm[q];
+                    for (uint32_t q = 0; q < 6; ++q) row[q * TS] = tm[q];
+                }
+            }
+        } else if (t > 0 && lane < 6 * IX) {
+            const double *row = lds + ((t - 1) & 1u) * (6 * IX * TS) + lane * TS;
+            const uint32_t jn = min(TJ, n - (t - 1) * TJ);
+            constexpr uint32_t U = 16;  // terms in flight from LDS ahead of the adds
+            if (jn == TJ) {
+                double2 cur[U / 2], nxt[U / 2];
+                const double2 *r2 = reinterpret_cast<const double2 *>(row);
+                for (uint32_t k = 0; k < U / 2; ++k) cur[k] = r2[k];
+#pragma unroll
+                for (uint32_t j = 0; j < TJ; j += U) {
+                    if (j + U < TJ)
+                        for (uint32_t k = 0; k < U / 2; ++k) nxt[k] = r2[(j + U) / 2 + k];
+                    for (uint32_t k = 0; k < U / 2; ++k) {
+                        acc += cur[k].x;
+                        acc += cur[k].y;
+                    }
+                    for (uint32_t k = 0; k < U / 2; ++k) cur[k] = nxt[k];
+                }
+            } else {
+                for (uint32_t j = 0; j < jn; ++j) acc += row[j];
+            }
+        }
+        __syncthreads();
+    }
+    if (adds && lane < 6 * IX) {
+        const uint32_t a = k0 + lane / 6;
+        if (a < nact) s.f[lane % 6][mv[a]] = acc;
+    }
+}
+
+// One lane per active particle (BS of them per item), its own adds the
+// chain.
+__device__ __forceinline__ void exact_item_wide(const Soa &s, const uint32_t *mv, uint32_t nact,
+                                                uint32_t it, uint32_t j_begin, uint32_t n,
+                                                double e2, double4 *tile) {
+    const double4 *sp = tile, *sv = tile + JT;
+    const uint32_t k = it * BS + threadIdx.x;
+    const bool act = k < nact;
+    const uint32_t i = act ? mv[k] : mv[0];
+    const uint32_t j_end = j_begin + n;
+    double pi[6];
+    load_predictor(s, i, pi);
+    double fo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (uint32_t j0 = j_begin; j0 < j_end; j0 += JT) {
+        __syncthreads();
+        load_jtile(s, j0, tile);
+        __syncthreads();
+        const uint32_t jn = min((uint32_t)JT, j_end - j0);
+        for (uint32_t jj = 0; jj < jn; ++jj) {
+            const double4 a = sp[jj], b = sv[jj];
+            if (j0 + jj != i) {
+                double tm[6];
+                terms_exact(pi, a.x, a.y, a.z, b.x, b.y, b.z, a.w, e2, tm);
+                for (int q = 0; q < 6; ++q) fo[q] += tm[q];
+            }
+        }
+    }
+    __syncthreads();  // the next item may write the tile as its term buffer
+    if (act)
+        for (int q = 0; q < 6; ++q) s.f[q][i] = fo[q];
+}
+
+// Workgroups stride over the plan's items (exact_iw particles each) and
+// write f[i] directly.
 __global__ __launch_bounds__(BS) void k_update_exact(Soa s, Ens e, const uint32_t *move,
                                                     double e2) {
-    __shared__ double4 tile[2 * JT];
-    const double4 *sp = tile, *sv = tile + JT;
+    constexpr uint32_t L1 = exact_lds<1, 192>(), L3 = exact_lds<3, 64>();
+    constexpr uint32_t LX = L1 > L3 ? L1 : L3, LM = LX > 8 * JT ? LX : 8 * JT;
+    __shared__ __align__(32) double lds[LM];
     const bool single = e.K == 1;
     unsigned long long total = 0;
+    ClPlan pl0{};
     if (single)
-        (void)plan_single(e, 1u, total);
+        pl0 = plan_single(e, 1u, total);
     else
         total = e.ctl->items;
     for (unsigned long long item = blockIdx.x; item < total; item += gridDim.x) {
         const uint32_t c = single ? 0u : find_cluster(e.items_pre, e.K, item);
         const uint32_t it = (uint32_t)(item - (single ? 0ull : e.items_pre[c]));
-        const uint32_t nact = e.cs[c].nact;
-        const uint32_t *mv = move + e.off[c];
-        const uint32_t j_begin = e.off[c], j_end = e.off[c] + e.cnt[c];
-        uint32_t k = it * BS + threadIdx.x;
-        bool act = k < nact;
-        uint32_t i = act ? mv[k] : mv[0];
-        double pi[6];
-        load_predictor(s, i, pi);
-        double fo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        for (uint32_t j0 = j_begin; j0 < j_end; j0 += JT) {
-            __syncthreads();
-            load_jtile(s, j0, tile);
-            __syncthreads();
-            uint32_t jn = min((uint32_t)JT, j_end - j0);
-            for (uint32_t jj = 0; jj < jn; ++jj) {
-                double4 a = sp[jj];
-                double4 b = sv[jj];
-                if (j0 + jj != i)
-                    pair_exact(pi, a.x, a.y, a.z, b.x, b.y, b.z, a.w, e2, fo);
-            }
-        }
-        if (act)
-            for (int q = 0; q < 6; ++q) s.f[q][i] = fo[q];
+        const uint32_t iw = single ? pl0.iw : e.plan[c].iw;
+        const uint32_t nact = e.cs[c].nact, off = e.off[c], n = e.cnt[c];
+        const uint32_t *mv = move + off;
+        // (every item ends with a barrier after its last read of lds)
+        if (iw == 1)
+            exact_item<1, 192>(s, mv, nact, it, off, n, e2, lds);
+        else if (iw == 3)
+            exact_item<3, 64>(s, mv, nact, it, off, n, e2, lds);
+        else
+            exact_item_wide(s, mv, nact, it, off, n, e2, reinterpret_cast<double4 *>(lds));
     }
 }
 
@@ -2019,12 +2148,16 @@ int configure_launch(h4h_ctx *ctx) {
 
 uint32_t finish_grid(h4h_ctx *ctx) { return std::min<uint32_t>(1024, std::max<uint32_t>(64, ctx->nblk)); }
 
+// Workgroups of the exact update for up to n active particles: its items
+// stride over them, and up to 3 are resident on each CU.
+uint32_t exact_grid(uint32_t n) { return std::min<uint32_t>(n, 1024); }
+
 // Pair kernel of the current precision over the plan's items.  compact:
 // the step's selection wrote the active particles' records.
 int launch_update(h4h_ctx *ctx, bool compact = false) {
     if (ctx->precision == H4H_FP64_EXACT) {
-        hipLaunchKernelGGL(k_update_exact, dim3(ctx->e.grid), dim3(BS), 0, ctx->stream, ctx->s,
-                           ctx->e, ctx->move, ctx->e2);
+        hipLaunchKernelGGL(k_update_exact, dim3(exact_grid(ctx->n)), dim3(BS), 0, ctx->stream,
+                           ctx->s, ctx->e, ctx->move, ctx->e2);
     } else {
         auto *kern = ctx->precision == H4H_MIXED ? k_update_mixed : k_update_fp64;
         hipLaunchKernelGGL(kern, dim3(ctx->e.grid), dim3(BS), 0, ctx->stream, ctx->s, ctx->e,
@@ -3372,7 +3505,7 @@ int h4h_update_acc_jrk_static(const double *d_p6, const float *d_pm, uint32_t n,
                        d_move, nact, move, s, tab);
     H4H_LAUNCHED();
     if (precision == H4H_FP64_EXACT) {
-        hipLaunchKernelGGL(k_update_exact, dim3(grid), dim3(BS), 0, st, s, e, move, e2);
+        hipLaunchKernelGGL(k_update_exact, dim3(exact_grid(nact)), dim3(BS), 0, st, s, e, move, e2);
     } else {
         auto *kern = precision == H4H_MIXED ? k_update_mixed : k_update_fp64;
         hipLaunchKernelGGL(kern, dim3(grid), dim3(BS), 0, st, s, e, move, partial, e2, 0u);
