@@ -289,6 +289,37 @@ __host__ __device__ inline uint32_t exact_iw(uint32_t nact) {
     return nact <= 768 ? 1u : nact < EXACT_WIDE ? 3u : (uint32_t)BS;
 }
 
+// Work items of the energy of n particles: i blocks of ENERGY_I particles
+// against the j chunks of jc particles from the block's first one on, in
+// wgs contiguous runs.  The chunk is the largest of 256 ... 16 that gives
+// 2048 items, so that a small system's pairs are spread over the CUs too
+// (n = 1024: 96 items of 16, not 6 of 256); small items go two to a
+// workgroup (fewer workgroup sums to add on the host; n = 4096: 52 us with
+// 1024 workgroups), and 2048 workgroups, 8 per CU, take 16 items or more
+// each (n = 131072: 3783 -> 3714 us, but n = 65536: 1125 -> 1134 us).
+constexpr uint32_t ENERGY_GRID = 2048;  // most workgroups of one cluster
+constexpr uint32_t ENERGY_I = 512;
+struct EnergyItems {
+    uint32_t jc;      // particles per j chunk
+    uint32_t chunks;  // j chunks
+    uint32_t wgs;     // workgroups
+    uint64_t items;
+};
+__host__ __device__ inline EnergyItems energy_items(uint32_t n) {
+    EnergyItems e;
+    const uint64_t nb = ((uint64_t)n + ENERGY_I - 1) / ENERGY_I;
+    for (e.jc = JT;; e.jc /= 2) {
+        e.chunks = (uint32_t)(((uint64_t)n + e.jc - 1) / e.jc);
+        e.items = nb * e.chunks - (ENERGY_I / e.jc) * (nb * (nb - 1) / 2);
+        if (e.items >= 2048 || e.jc == 16) break;
+    }
+    e.wgs = e.items >= 16 * ENERGY_GRID ? ENERGY_GRID
+            : e.items >= 2048           ? 1024u
+            : e.items >= 512            ? (uint32_t)(e.items / 2)
+                                        : (uint32_t)(e.items < 256 ? e.items : 256);
+    return e;
+}
+
 // ---------------------------------------------------------------------------
 // Pair terms
 // ---------------------------------------------------------------------------

@@ -59,7 +59,7 @@ int fail(int code, const std::string &msg) {
 
 constexpr uint32_t DEFAULT_GRID = 2048;       // persistent workgroups
 constexpr uint32_t DEFAULT_MAX_SPLIT = 1024;  // largest j split
-constexpr uint32_t ENERGY_GRID = 1024;
+constexpr uint32_t ENERGY_OUT = 8 * ENERGY_GRID;  // workgroup sums of one energy launch
 
 // ---------------------------------------------------------------------------
 // Cluster geometry helpers
@@ -1873,12 +1873,12 @@ __global__ void k_set_times_from_tmin(Ens e, double itime) {
 // cluster, NbodyUtils::get_energy (NbodyUtils.cpp:427-529).  1/|r_ij| from
 // v_rsq_f64 and one Newton step (relative error below 2^-47 and of one
 // sign, against the reference's division by sqrt): a lane sums
-// m_j / |r_ij| over one j tile in plain FP64 (at most 256 terms of one
+// 2 m_j / |r_ij| over one j chunk in plain FP64 (at most 256 terms of one
 // sign, so at most 256 roundings of the partial sum: 3e-14 relative),
-// multiplies by m_i and adds that into its Neumaier-compensated sum; then
-// per workgroup, then over workgroups in index order (deterministic for a
-// fixed grid).  A coincident pair (r = 0) makes the Newton step NaN; such
-// a tile is summed again with 1/0 = inf, so coincident particles give -inf
+// multiplies by m_i / 2 and adds that into its Neumaier-compensated sum;
+// then per workgroup, then over workgroups in index order (deterministic
+// for a fixed n).  A coincident pair (r = 0) makes the Newton step NaN; such
+// a chunk is summed again with 1/0 = inf, so coincident particles give -inf
 // as in the reference.
 // ---------------------------------------------------------------------------
 
@@ -1917,72 +1917,108 @@ __device__ __forceinline__ void block_sum2(double &a, double &b, double *red) {
     }
 }
 
-// Items are pairs of (i tile, j tile) with j tile >= i tile of the cluster
-// at device offset off, numbered row by row;
-// out[4*block] = {epot, epot_comp, ekin, ekin_comp}.
-// Cluster c0 + blockIdx.y of the cluster tables offs / cnts; workgroup
-// blockIdx.x takes the tile pairs blockIdx.x, + stride, + 2 stride, ...
-// (stride >= gridDim.x: a launch with fewer workgroups than stride has the
-// same per-workgroup sums as one with stride workgroups, the others' being
-// zero), and writes its four sums at out[4 (blockIdx.y gridDim.x +
-// blockIdx.x)].
+// Cluster c0 + blockIdx.y of the cluster tables offs / cnts: items are pairs
+// of an i block (ENERGY_I particles, EI per lane) and a j chunk (jc
+// particles, EnergyItems) that reaches past the block's first particle,
+// numbered row by row (i block by i block), a contiguous run of them per
+// workgroup; out[4 (blockIdx.y gridDim.x + blockIdx.x)] = {epot, epot_comp,
+// ekin, ekin_comp} of the run.
+//
+// VALU bound at 14 issue slots per pair (3 sub, 3 for r^2, 4 for v_rsq_f64,
+// 4 for the Newton step and the sum) if each j record read from LDS serves
+// EI pairs: one pair per read took the 16 cycles that a CU's LDS needs to
+// return a broadcast double4 to a wave as often as its SIMDs took 60 to use
+// it, four SIMDs per LDS (N = 262144: 1.72e12 pairs/s).
+constexpr uint32_t EI = ENERGY_I / BS;
+
+__device__ __forceinline__ double energy_term(const double4 &q, double xi, double yi, double zi,
+                                              double sum, bool guard) {
+    const double rx = q.x - xi, ry = q.y - yi, rz = q.z - zi;
+    const double r2 = __builtin_fma(rx, rx, __builtin_fma(ry, ry, rz * rz));
+    const double y = __builtin_amdgcn_rsq(r2);
+    double w = __builtin_fma(-(r2 * y), y, 3.0);  // y w = 2 / r
+    if (guard && !(r2 > 0.0)) w = INFINITY;       // (y is +inf there too)
+    return __builtin_fma(q.w * y, w, sum);
+}
+
 __global__ __launch_bounds__(BS) void k_energy(Soa s, const uint32_t *offs, const uint32_t *cnts,
-                                              uint32_t c0, uint32_t stride, double *out) {
+                                              uint32_t c0, double *out) {
 #pragma clang fp contract(off)
-    __shared__ double4 sr[JT];
+    __shared__ double4 sr[2][JT];
     __shared__ double red[2 * (BS / 64)];
     const uint32_t off = offs[c0 + blockIdx.y], n = cnts[c0 + blockIdx.y];
-    const uint32_t nt = (n + BS - 1) / BS;
-    const uint64_t items = (uint64_t)nt * (nt + 1) / 2;
+    const EnergyItems ei = energy_items(n);
+    const uint32_t R = ENERGY_I / ei.jc;  // a row starts R chunks after the one before
     double ep = 0.0, epc = 0.0, ek = 0.0, ekc = 0.0;
-    // Row `it` holds nt - it items.  (it, rem) locate the current item and
-    // advance by stride per iteration, so the walk is O(nt) in total.
-    uint32_t it = 0;
-    uint64_t rem = blockIdx.x;
-    for (uint64_t item = blockIdx.x; item < items; item += stride) {
-        while (rem >= (uint64_t)(nt - it)) {
-            rem -= (nt - it);
-            ++it;
+    if (blockIdx.x < ei.wgs) {
+        const uint64_t first = ei.items * blockIdx.x / ei.wgs;
+        const uint64_t last = ei.items * (blockIdx.x + 1) / ei.wgs;
+        uint32_t row = 0;
+        uint64_t rem = first;
+        while (rem >= ei.chunks - row * R) {
+            rem -= ei.chunks - row * R;
+            ++row;
         }
-        uint32_t jt = it + (uint32_t)rem;
-        rem += stride;
-        uint32_t li = it * BS + threadIdx.x;
-        uint32_t lj0 = jt * JT;
-        __syncthreads();
-        {
-            uint32_t j = off + lj0 + threadIdx.x;
-            if (lj0 + threadIdx.x < n)
-                sr[threadIdx.x] = make_double4(s.r[0][j], s.r[1][j], s.r[2][j], s.m[j]);
-        }
-        __syncthreads();
-        if (li < n) {
-            uint32_t i = off + li;
-            double xi = s.r[0][i], yi = s.r[1][i], zi = s.r[2][i], mi = s.m[i];
-            uint32_t jn = min((uint32_t)JT, n - lj0);
-            uint32_t jb = (jt == it) ? threadIdx.x + 1 : 0;
-            auto tile_sum = [&](bool guard) {
-                double sum = 0.0;
-                for (uint32_t jj = jb; jj < jn; ++jj) {
-                    double4 q = sr[jj];
-                    double rx = q.x - xi;
-                    double ry = q.y - yi;
-                    double rz = q.z - zi;
-                    double r2 = __builtin_fma(rx, rx, __builtin_fma(ry, ry, rz * rz));
-                    double y = __builtin_amdgcn_rsq(r2);
-                    double e = __builtin_fma(-r2, y * y, 1.0);
-                    double rinv = __builtin_fma(y * e, 0.5, y);
-                    if (guard && !(r2 > 0.0)) rinv = INFINITY;
-                    sum = __builtin_fma(q.w, rinv, sum);
+        auto load_j = [&](uint32_t ch) {  // (past the end: zero mass, far away)
+            const uint32_t lj = ch * ei.jc + threadIdx.x, j = off + lj;
+            if (threadIdx.x < ei.jc && lj < n)
+                return make_double4(s.r[0][j], s.r[1][j], s.r[2][j], s.m[j]);
+            return make_double4(PAD_POS, PAD_POS, PAD_POS, 0.0);
+        };
+        double xi[EI], yi[EI], zi[EI], mi[EI];
+        double4 nj = load_j(row * R + (uint32_t)rem);
+        bool fresh = true;  // a new row's i particles are to be loaded
+        for (uint64_t item = first; item < last; ++item) {
+            const uint32_t ch = row * R + (uint32_t)rem;
+            const uint32_t li0 = row * ENERGY_I + threadIdx.x;
+            double4 *tile = sr[item & 1];
+            tile[threadIdx.x] = nj;
+            if (fresh)
+                for (uint32_t k = 0; k < EI; ++k) {
+                    const uint32_t li = li0 + k * BS, i = off + li;
+                    const bool in = li < n;
+                    xi[k] = in ? s.r[0][i] : -PAD_POS;
+                    yi[k] = in ? s.r[1][i] : -PAD_POS;
+                    zi[k] = in ? s.r[2][i] : -PAD_POS;
+                    mi[k] = in ? s.m[i] : 0.0;
+                    if (rem == 0 && in) {  // the row's first item counts its kinetic energy
+                        const double vx = s.v[0][i], vy = s.v[1][i], vz = s.v[2][i];
+                        const double vv2 = vx * vx + vy * vy + vz * vz;
+                        neumaier(ek, ekc, 0.5 * mi[k] * vv2);
+                    }
                 }
-                return sum;
-            };
-            double tile = tile_sum(false);
-            if (isnan(tile)) tile = tile_sum(true);
-            if (jb < jn) neumaier(ep, epc, -(mi * tile));
-            if (jt == it) {
-                double vx = s.v[0][i], vy = s.v[1][i], vz = s.v[2][i];
-                double vv2 = vx * vx + vy * vy + vz * vz;
-                neumaier(ek, ekc, 0.5 * mi * vv2);
+            // the next item, its j chunk requested under this one's pairs
+            const bool diag = rem < R;
+            fresh = ++rem >= ei.chunks - row * R;
+            if (fresh) {
+                rem = 0;
+                ++row;
+            }
+            if (item + 1 < last) nj = load_j(row * R + (uint32_t)rem);
+            __syncthreads();  // (the other tile's readers passed the last one)
+            double sum[EI];
+            for (uint32_t k = 0; k < EI; ++k) sum[k] = 0.0;
+            if (!diag) {
+#pragma unroll 4
+                for (uint32_t jj = 0; jj < ei.jc; ++jj) {
+                    const double4 q = tile[jj];
+#pragma unroll
+                    for (uint32_t k = 0; k < EI; ++k)
+                        sum[k] = energy_term(q, xi[k], yi[k], zi[k], sum[k], false);
+                }
+            }
+            for (uint32_t k = 0; k < EI; ++k) {
+                const uint32_t li = li0 + k * BS, jd = li + 1;
+                const uint32_t jb = jd > ch * ei.jc ? jd - ch * ei.jc : 0u;  // j > i
+                if (diag)
+                    for (uint32_t jj = jb; jj < ei.jc; ++jj)
+                        sum[k] = energy_term(tile[jj], xi[k], yi[k], zi[k], sum[k], false);
+                if (isnan(sum[k])) {
+                    sum[k] = 0.0;
+                    for (uint32_t jj = jb; jj < ei.jc; ++jj)
+                        sum[k] = energy_term(tile[jj], xi[k], yi[k], zi[k], sum[k], true);
+                }
+                if (li < n) neumaier(ep, epc, -(0.5 * mi[k] * sum[k]));
             }
         }
     }
@@ -2044,7 +2080,6 @@ struct h4h_ctx {
     double *staging = nullptr;   // n * 8 doubles
     double *partial = nullptr;   // j-split partials
     size_t partial_len = 0;
-    double *eout = nullptr;      // energy per-workgroup sums
     uint32_t *move = nullptr;
     // cluster tables
     uint32_t *d_off = nullptr, *d_cnt = nullptr, *d_hoff = nullptr, *d_bcl = nullptr;
@@ -2058,7 +2093,9 @@ struct h4h_ctx {
     uint32_t *d_tune = nullptr;  // [64] tuning table
     double *hist_t = nullptr;
     uint32_t *hist_n = nullptr;
-    // pinned host mirrors
+    // pinned host memory: energy per-workgroup sums, mirrors
+    double *pinned = nullptr;
+    double *eout = nullptr;
     RunCtl *ctl_host = nullptr;
     ClState *cs_host = nullptr;
     double *hist_t_host = nullptr;
@@ -2380,13 +2417,17 @@ int download_scalar(h4h_ctx *ctx, const double *src, double *dst) {
 
 bool valid_precision(int p) { return p == H4H_FP64 || p == H4H_FP64_EXACT || p == H4H_MIXED; }
 
+// Workgroup sums the energy buffer of a context holds: one system's, or
+// ENERGY_OUT for an ensemble.
+size_t eout_len(const h4h_ctx *ctx) { return ctx->K > 1 ? ENERGY_OUT : ENERGY_GRID; }
+
 // Energies of clusters c0 .. c0 + count - 1, in launches of as many
-// clusters as fit the ENERGY_GRID x 4 sums of eout: per cluster the
-// workgroups that have tile pairs (at most ENERGY_GRID, item stride
-// ENERGY_GRID as in a launch of ENERGY_GRID workgroups for that cluster
-// alone), then a host Neumaier sum of its workgroup sums in order.
+// clusters as fit the sums of eout (64 clusters of 1024 to 32768 particles:
+// 4 launches; 48, each waited for, with a buffer for one system's
+// workgroups), then per cluster a host Neumaier sum of its workgroup sums
+// in order.  The workgroups write their sums, 32 bytes each, to the pinned
+// host buffer themselves, which takes no copy call.
 int energies_of(h4h_ctx *ctx, uint32_t c0, uint32_t count, double *ekin, double *epot) {
-    std::vector<double> h(ENERGY_GRID * 4);
     // Neumaier sum of the per-workgroup (sum, compensation) pairs (an
     // infinite sum leaves the compensation alone, as on the device).
     auto add = [](double &s, double &c2, double x) {
@@ -2399,28 +2440,24 @@ int energies_of(h4h_ctx *ctx, uint32_t c0, uint32_t count, double *ekin, double 
         }
         s = t;
     };
-    auto wgs = [&](uint32_t c) {
-        const uint64_t nt = (ctx->cnt[c] + BS - 1) / BS;
-        return (uint32_t)std::min<uint64_t>(ENERGY_GRID, nt * (nt + 1) / 2);
-    };
+    auto wgs = [&](uint32_t c) { return energy_items(ctx->cnt[c]).wgs; };
+    const size_t most = eout_len(ctx);
     for (uint32_t b0 = c0; b0 < c0 + count;) {
         uint32_t gx = wgs(b0), kb = 1;
         while (b0 + kb < c0 + count) {
             const uint32_t g2 = std::max(gx, wgs(b0 + kb));
-            if ((uint64_t)(kb + 1) * g2 > ENERGY_GRID) break;
+            if ((uint64_t)(kb + 1) * g2 > most) break;
             gx = g2;
             ++kb;
         }
         hipLaunchKernelGGL(k_energy, dim3(gx, kb), dim3(BS), 0, ctx->stream, ctx->s, ctx->d_off,
-                           ctx->d_cnt, b0, (uint32_t)ENERGY_GRID, ctx->eout);
+                           ctx->d_cnt, b0, ctx->eout);
         H4H_LAUNCHED();
-        H4H_HIP(hipMemcpyAsync(h.data(), ctx->eout, (size_t)kb * gx * 4 * sizeof(double),
-                               hipMemcpyDeviceToHost, ctx->stream));
         H4H_HIP(hipStreamSynchronize(ctx->stream));
         for (uint32_t k = 0; k < kb; ++k) {
             double sp = 0.0, cp = 0.0, sk = 0.0, ck = 0.0;
-            const double *hk = h.data() + (size_t)k * gx * 4;
-            for (uint32_t b = 0; b < gx; ++b) {
+            const double *hk = ctx->eout + (size_t)k * gx * 4;
+            for (uint32_t b = 0; b < wgs(b0 + k); ++b) {
                 add(sp, cp, hk[4 * b + 0]);
                 add(sp, cp, hk[4 * b + 1]);
                 add(sk, ck, hk[4 * b + 2]);
@@ -2494,7 +2531,6 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     size_t np = ctx->n_dev;
     bool ok = hipMalloc(&ctx->state, np * N_SOA * sizeof(double)) == hipSuccess &&
               hipMalloc(&ctx->staging, (size_t)ctx->n * 8 * sizeof(double)) == hipSuccess &&
-              hipMalloc(&ctx->eout, ENERGY_GRID * 4 * sizeof(double)) == hipSuccess &&
               hipMalloc(&ctx->move, np * sizeof(uint32_t)) == hipSuccess &&
               hipMalloc(&ctx->d_off, K * sizeof(uint32_t)) == hipSuccess &&
               hipMalloc(&ctx->d_cnt, K * sizeof(uint32_t)) == hipSuccess &&
@@ -2511,11 +2547,17 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
               hipMalloc(&ctx->hist_t, HIST_CAP * sizeof(double)) == hipSuccess &&
               hipMalloc(&ctx->hist_n, HIST_CAP * sizeof(uint32_t)) == hipSuccess;
     if (!ok) return cleanup(fail(H4H_ENOMEM, "device allocation failed"));
-    ok = hipHostMalloc(&ctx->ctl_host, sizeof(RunCtl), hipHostMallocDefault) == hipSuccess &&
-         hipHostMalloc(&ctx->cs_host, K * sizeof(ClState), hipHostMallocDefault) == hipSuccess &&
-         hipHostMalloc(&ctx->hist_t_host, HIST_CAP * sizeof(double), hipHostMallocDefault) == hipSuccess &&
-         hipHostMalloc(&ctx->hist_n_host, HIST_CAP * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess;
-    if (!ok) return cleanup(fail(H4H_ENOMEM, "pinned allocation failed"));
+    // One pinned allocation for all host mirrors (each costs ~0.2 ms).
+    static_assert(sizeof(RunCtl) % 8 == 0 && sizeof(ClState) % 8 == 0, "carved in doubles");
+    const size_t eo = eout_len(ctx) * 4, ct = sizeof(RunCtl) / 8, cst = K * sizeof(ClState) / 8;
+    if (hipHostMalloc(&ctx->pinned, (eo + ct + cst + HIST_CAP + HIST_CAP / 2) * sizeof(double),
+                      hipHostMallocDefault) != hipSuccess)
+        return cleanup(fail(H4H_ENOMEM, "pinned allocation failed"));
+    ctx->eout = ctx->pinned;
+    ctx->ctl_host = reinterpret_cast<RunCtl *>(ctx->eout + eo);
+    ctx->cs_host = reinterpret_cast<ClState *>(ctx->eout + eo + ct);
+    ctx->hist_t_host = ctx->eout + eo + ct + cst;
+    ctx->hist_n_host = reinterpret_cast<uint32_t *>(ctx->hist_t_host + HIST_CAP);
     for (int k = 0; k < 4; ++k)
         if (hipEventCreate(&ctx->ev[k]) != hipSuccess)
             return cleanup(fail(H4H_EHIP, "hipEventCreate failed"));
@@ -2741,15 +2783,13 @@ int h4h_destroy(h4h_ctx *ctx) {
     drop_graph(ctx);
     for (int k = 0; k < 4; ++k)
         if (ctx->ev[k]) (void)hipEventDestroy(ctx->ev[k]);
-    void *dev[] = {ctx->state, ctx->staging, ctx->partial, ctx->eout, ctx->move, ctx->d_off,
+    void *dev[] = {ctx->state, ctx->staging, ctx->partial, ctx->move, ctx->d_off,
                    ctx->d_cnt, ctx->d_hoff, ctx->d_bcl, ctx->d_cs, ctx->d_plan, ctx->d_pre,
                    ctx->d_ctl, ctx->d_dirty, ctx->d_bmin, ctx->d_arec, ctx->d_tune, ctx->hist_t,
                    ctx->hist_n};
     for (void *p : dev)
         if (p) (void)hipFree(p);
-    void *host[] = {ctx->ctl_host, ctx->cs_host, ctx->hist_t_host, ctx->hist_n_host};
-    for (void *p : host)
-        if (p) (void)hipHostFree(p);
+    if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return H4H_OK;
