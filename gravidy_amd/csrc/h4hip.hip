@@ -52,10 +52,6 @@ int fail(int code, const std::string &msg) {
 #ifndef H4_MIXED_UNROLL
 #define H4_MIXED_UNROLL 2
 #endif
-// Waves of the one-workgroup step's pair loop for active sets under 64.
-#ifndef H4_SMALL_NARROW_WAVES
-#define H4_SMALL_NARROW_WAVES 8
-#endif
 
 constexpr uint32_t DEFAULT_GRID = 2048;       // persistent workgroups
 constexpr uint32_t DEFAULT_MAX_SPLIT = 1024;  // largest j split
@@ -1044,32 +1040,28 @@ __device__ __forceinline__ double magnitude(double x, double y, double z) {
     return sqrt(x * x + y * y + z * z);
 }
 
-// NbodyUtils::normalize_dt (NbodyUtils.cpp:371-424), bounds as arguments.
-__device__ __forceinline__ double normalize_dt(double new_dt, double old_dt,
-                                               double t, double dt_min,
-                                               double dt_max) {
+// Whether block time t is commensurate with twice the step (the condition of
+// NbodyUtils::normalize_dt for doubling it).
+__device__ __forceinline__ bool dt_doubles(double old_dt, double t) {
 #pragma clang fp contract(off)
-    if (new_dt <= old_dt / 8) {
-        new_dt = dt_min;
-    } else if (old_dt / 8 < new_dt && new_dt <= old_dt / 4) {
-        new_dt = old_dt / 8;
-    } else if (old_dt / 4 < new_dt && new_dt <= old_dt / 2) {
-        new_dt = old_dt / 4;
-    } else if (old_dt / 2 < new_dt && new_dt <= old_dt) {
-        new_dt = old_dt / 2;
-    } else if (old_dt < new_dt && new_dt <= old_dt * 2) {
-        new_dt = old_dt;
-    } else if (2 * old_dt < new_dt) {
-        double val = t / (2 * old_dt);
-        new_dt = (ceil(val) == val) ? 2.0 * old_dt : old_dt;
-    } else {
-        new_dt = old_dt;
-    }
-    if (new_dt < dt_min)
-        new_dt = dt_min;
-    else if (new_dt > dt_max)
-        new_dt = dt_max;
-    return new_dt;
+    const double val = t / (2 * old_dt);
+    return ceil(val) == val;
+}
+
+// NbodyUtils::normalize_dt (NbodyUtils.cpp:371-424), bounds as arguments;
+// doubles() gives dt_doubles(old_dt, t).
+template <class F>
+__device__ __forceinline__ double normalize_dt(double new_dt, double old_dt, F doubles,
+                                               double dt_min, double dt_max) {
+#pragma clang fp contract(off)
+    // (selects from the last branch to the first; NaN keeps the old step)
+    double res = old_dt;
+    if (2 * old_dt < new_dt) res = doubles() ? 2.0 * old_dt : old_dt;
+    res = old_dt / 2 < new_dt && new_dt <= old_dt ? old_dt / 2 : res;
+    res = old_dt / 4 < new_dt && new_dt <= old_dt / 2 ? old_dt / 4 : res;
+    res = old_dt / 8 < new_dt && new_dt <= old_dt / 4 ? old_dt / 8 : res;
+    new_dt = new_dt <= old_dt / 8 ? dt_min : res;
+    return new_dt < dt_min ? dt_min : new_dt > dt_max ? dt_max : new_dt;
 }
 
 // Hermite4CPU::correction_pos_vel (Hermite4CPU.cpp:370-411) with
@@ -1106,7 +1098,133 @@ __device__ __forceinline__ double correct_vals(const double o[6], const double f
     double abs_a1_22 = abs_a1_2 * abs_a1_2;
     double normal_dt = sqrt(eta * ((abs_a1 * abs_a1_2 + abs_j12) /
                                    (abs_j1 * abs_a1_3 + abs_a1_22)));
-    return normalize_dt(normal_dt, dt1, itime, dt_min, dt_max);
+    return normalize_dt(normal_dt, dt1, [&] { return dt_doubles(dt1, itime); }, dt_min, dt_max);
+}
+
+// Lane exchanges by DPP (a few cycles; a ds_bpermute shuffle takes ~100):
+// CTRL is the DPP control, BANK the banks of four lanes that take it (the
+// others keep `old`).
+template <int CTRL, int BANK = 0xf>
+__device__ __forceinline__ double dpp(double old, double x) {
+    const unsigned long long o = __builtin_bit_cast(unsigned long long, old);
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)o, (int)(uint32_t)u,
+                                                              CTRL, 0xf, BANK, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(
+        (int)(uint32_t)(o >> 32), (int)(uint32_t)(u >> 32), CTRL, 0xf, BANK, false);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;     // quad_perm 1,0,3,2 and 2,3,0,1
+constexpr int DPP_QUADS = 0x141, DPP_EIGHTS = 0x140;  // row_half_mirror, row_mirror
+template <int K>
+__device__ __forceinline__ double quad_lane(double x) {  // lane K of each quad
+    return dpp<K * 0x55>(x, x);
+}
+// The value of lane ^ 4: row_shl:4 into banks 0 and 2, row_shr:4 into 1 and 3.
+__device__ __forceinline__ double xor4(double x) {
+    return dpp<0x114, 0xa>(dpp<0x104, 0x5>(x, x), x);
+}
+// Swaps the odd rows of 16 lanes (ROWS = 1; the upper half of 32: ROWS = 2)
+// of x with the even ones of y: an even row has then x of itself (a) and of
+// its odd neighbour (b), an odd row y of its even neighbour (a) and of
+// itself (b).
+template <int ROWS>
+__device__ __forceinline__ void swap_rows(double x, double y, double &a, double &b) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const unsigned long long t = __builtin_bit_cast(unsigned long long, y);
+    uint32_t l0, l1, h0, h1;
+    if constexpr (ROWS == 1) {
+        const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)t, false, false);
+        const auto hi =
+            __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(t >> 32), false, false);
+        l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+    } else {
+        const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)t, false, false);
+        const auto hi =
+            __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(t >> 32), false, false);
+        l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+    }
+    a = __builtin_bit_cast(double, ((unsigned long long)h0 << 32) | l0);
+    b = __builtin_bit_cast(double, ((unsigned long long)h1 << 32) | l1);
+}
+// v_min_f64 as it is (fmin also quiets both operands: two more instructions
+// each time; a NaN loses either way).
+__device__ __forceinline__ double vmin(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Minimum over the wave (all lanes active; every lane gets it).
+__device__ __forceinline__ double wave_min(double x) {
+    double a, b;
+    x = vmin(x, dpp<DPP_XOR1>(x, x));
+    x = vmin(x, dpp<DPP_XOR2>(x, x));
+    x = vmin(x, dpp<DPP_QUADS>(x, x));   // (the quads are uniform by now,
+    x = vmin(x, dpp<DPP_EIGHTS>(x, x));  // and the eights)
+    swap_rows<1>(x, x, a, b);
+    x = vmin(a, b);
+    swap_rows<2>(x, x, a, b);
+    return vmin(a, b);
+}
+
+// The corrector of one particle on 8 consecutive lanes of a wave (all lanes
+// active): lane c + 4 vel has component c (0..2; lane 3 repeats 2) of the
+// position and a2 (vel = 0) or of the velocity and a3 (vel = 1).  The same
+// operations as correct_vals, value by value, so the same bits; on one lane
+// they are ~600 instructions, 18 of them IEEE divisions and square roots one
+// after the other (5900 cycles in a one-workgroup step), here a chain of two
+// divisions and two square roots.
+struct Corr8 {
+    double dt1, den, k1, k2;
+    bool doubles;
+};
+// What depends on the step and the block time only.
+__device__ __forceinline__ Corr8 corr8_coef(double dt1, double itime, bool vel) {
+#pragma clang fp contract(off)
+    const double dt2 = dt1 * dt1;
+    const double dt3 = dt2 * dt1;
+    const double dt4 = dt2 * dt2;
+    const double dt5 = dt4 * dt1;
+    Corr8 k;
+    k.dt1 = dt1;
+    k.den = vel ? dt3 : dt2;
+    k.k1 = (vel ? dt3 : dt4) / (vel ? 6.0 : 24.0);
+    k.k2 = (vel ? dt4 : dt5) / (vel ? 24.0 : 120.0);
+    k.doubles = dt_doubles(dt1, itime);
+    return k;
+}
+// o0, o1 and f0, f1: component c of the old and new acceleration and jerk;
+// pr: of the predicted position or velocity.  x: the corrected one, ad: a2
+// or a3 of the component; returns the new step (every lane).
+__device__ __forceinline__ double corr8(const Corr8 &k, bool vel, double o0, double o1, double f0,
+                                        double f1, double pr, double eta, double dt_min,
+                                        double dt_max, double &x, double &ad) {
+#pragma clang fp contract(off)
+    const double dt1 = k.dt1;
+    const double n2 = -6 * (o0 - f0) - dt1 * (4 * o1 + 2 * f1);
+    const double n3 = 12 * (o0 - f0) + 6 * dt1 * (o1 + f1);
+    ad = (vel ? n3 : n2) / k.den;
+    const double other = xor4(ad);
+    const double a2 = vel ? other : ad, a3 = vel ? ad : other;
+    x = pr + k.k1 * a2 + k.k2 * a3;
+    // squared lengths: acceleration and jerk (vel = 0); a3 and the second
+    // derivative at the new time (vel = 1), one square root per lane
+    const double a1_2 = a2 + dt1 * a3;
+    const double p = vel ? a3 : f0, q = vel ? a1_2 : f1;
+    const double p2 = p * p, q2 = q * q;
+    const double sp = quad_lane<0>(p2) + quad_lane<1>(p2) + quad_lane<2>(p2);
+    const double sq = quad_lane<0>(q2) + quad_lane<1>(q2) + quad_lane<2>(q2);
+    const double m = sqrt((threadIdx.x & 1u) ? sq : sp);
+    const double mp = quad_lane<0>(m), mq = quad_lane<1>(m);
+    const double op = dpp<DPP_QUADS>(mp, mp), oq = dpp<DPP_QUADS>(mq, mq);
+    const double abs_a1 = vel ? op : mp, abs_j1 = vel ? oq : mq;
+    const double abs_a1_3 = vel ? mp : op, abs_a1_2 = vel ? mq : oq;
+    const double abs_j12 = abs_j1 * abs_j1;
+    const double abs_a1_22 = abs_a1_2 * abs_a1_2;
+    const double normal_dt = sqrt(eta * ((abs_a1 * abs_a1_2 + abs_j12) /
+                                         (abs_j1 * abs_a1_3 + abs_a1_22)));
+    return normalize_dt(normal_dt, dt1, [&] { return k.doubles; }, dt_min, dt_max);
 }
 
 // The corrector of particle i at block time itime, given its new forces
@@ -1510,11 +1628,15 @@ __global__ __launch_bounds__(BS) void k_tail(Ens e) {
 // Small systems: whole block steps in one workgroup
 // ---------------------------------------------------------------------------
 
-constexpr uint32_t SB = 1024;         // threads of k_small_run, and the largest N it takes
+constexpr uint32_t SN = 1024;            // largest N k_small_run takes
+constexpr uint32_t SB = 512;             // its threads
+constexpr uint32_t SP = SN / SB;         // particles per thread
+constexpr uint32_t SW = SB / 64;         // waves
+constexpr uint32_t SC = SN / 64;         // chunks of 64 particles
 constexpr uint32_t SMALL_MAX_ACT = 256;  // largest active set k_small_run takes
-static_assert(SB % JT == 0 && SB / JT <= SB / 64, "block minima from the wave minima");
-static_assert(H4_SMALL_NARROW_WAVES >= 1 && H4_SMALL_NARROW_WAVES <= SB / 64,
-              "pair waves of the one-workgroup step");
+// Columns of a context's state from r[0] on (create_impl lays them out).
+constexpr uint32_t COL_R = 0, COL_F = 7, COL_OLD = 13, COL_A2 = 19, COL_T = 25, COL_DT = 26;
+static_assert(SB % JT == 0 && SC == 16, "a row of 16 lanes holds the chunks");
 
 // p (a global-memory pointer), as a value the compiler cannot hoist out of
 // a loop: stores through it inside the loop address SGPR base + VGPR offset
@@ -1527,55 +1649,178 @@ __device__ __forceinline__ __attribute__((address_space(1))) T *in_loop(T *p) {
     return (__attribute__((address_space(1))) T *)p;
 }
 
-// Number of threads of the workgroup with `flag` set, and (for those) the
-// count below them in thread order.  Ends with a barrier.
-__device__ __forceinline__ uint32_t small_count(bool flag, uint32_t *wcnt, uint32_t &below) {
-    const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
-    const unsigned long long mask = __ballot(flag);
-    if (lane == 0) wcnt[w] = (uint32_t)__popcll(mask);
-    __syncthreads();
-    uint32_t total = 0;
-    below = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-    for (uint32_t k = 0; k < SB / 64; ++k) {
-        const uint32_t c = wcnt[k];
-        below += k < w ? c : 0u;
-        total += c;
-    }
-    return total;
+// Sum of c over the 16 lanes of the row.
+__device__ __forceinline__ uint32_t row_sum(uint32_t c) {
+    auto add = [&](int o) { c += (uint32_t)o; };
+    add(__builtin_amdgcn_update_dpp(0, (int)c, DPP_XOR1, 0xf, 0xf, false));
+    add(__builtin_amdgcn_update_dpp(0, (int)c, DPP_XOR2, 0xf, 0xf, false));
+    add(__builtin_amdgcn_update_dpp(0, (int)c, DPP_QUADS, 0xf, 0xf, false));
+    add(__builtin_amdgcn_update_dpp(0, (int)c, DPP_EIGHTS, 0xf, 0xf, false));
+    return c;
 }
 
-// Minimum of v over the workgroup (every thread gets it).  Ends after a
-// barrier; wmin is free again after the next one.
-__device__ __forceinline__ double small_min(double v, double *wmin) {
-    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+// Number of particles of the workgroup with their flag set (particle
+// tid + k SB: flag[k] of thread tid), and (for those) the count below them
+// in particle order.  Ends after a barrier.
+__device__ __forceinline__ uint32_t small_count(const bool flag[SP], uint32_t *wcnt,
+                                                uint32_t below[SP]) {
+    const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
+    unsigned long long mask[SP];
+    for (uint32_t k = 0; k < SP; ++k) {
+        mask[k] = __ballot(flag[k]);
+        if (lane == 0) wcnt[k * SW + w] = (uint32_t)__popcll(mask[k]);
+    }
+    __syncthreads();
+    const uint32_t c = wcnt[lane % SC];
+    for (uint32_t k = 0; k < SP; ++k)
+        below[k] = row_sum(lane % SC < k * SW + w ? c : 0u) +
+                   (uint32_t)__popcll(mask[k] & ((1ull << lane) - 1ull));
+    return row_sum(c);
+}
+
+// Minimum over the workgroup (every thread gets it).  Ends after a barrier;
+// wmin is free again after the next one.
+__device__ __forceinline__ double small_min(const double x[SP], double *wmin) {
+    double v = x[0];
+    for (uint32_t k = 1; k < SP; ++k) v = vmin(v, x[k]);
+    v = wave_min(v);
     if (__lane_id() == 0) wmin[threadIdx.x >> 6] = v;
     __syncthreads();
-    double m = wmin[0];
-    for (uint32_t k = 1; k < SB / 64; ++k) m = fmin(m, wmin[k]);
-    return m;
+    return wave_min(wmin[__lane_id() % SW]);
 }
 
-// Block steps of systems of n <= SB particles, workgroup c of SB threads for
+// Pairs of particle i (record pi) with j = g, g + G, ... < n, added to fo;
+// MIXED: FP32 sums of 32 pairs at a time.
+template <bool MIXED>
+__device__ __forceinline__ void small_pairs(const double pi[6], uint32_t i, uint32_t g, uint32_t G,
+                                            uint32_t n, const double4 *lpp, const double4 *lpv,
+                                            double e2, uint32_t self_zero, double fo[6]) {
+    if constexpr (!MIXED) {
+        if (self_zero) {
+            // two j at a time (a missing second one without mass): most lanes
+            // have 2 to 16, and one at a time their latency is the phase
+#pragma unroll 2
+            for (uint32_t j = g; j < n; j += 2 * G) {
+                const uint32_t k = min(j + G, n - 1);
+                const double4 a = lpp[j], b = lpv[j], a2 = lpp[k], b2 = lpv[k];
+                pair_fp64(pi, a.x, a.y, a.z, b.x, b.y, b.z, a.w, e2, fo);
+                pair_fp64(pi, a2.x, a2.y, a2.z, b2.x, b2.y, b2.z, j + G < n ? a2.w : 0.0, e2, fo);
+            }
+        } else {
+            for (uint32_t j = g; j < n; j += G) {
+                const double4 a = lpp[j], b = lpv[j];
+                const bool me = j == i;
+                pair_fp64(pi, me ? pi[0] + 1.0 : a.x, a.y, a.z, b.x, b.y, b.z, me ? 0.0 : a.w, e2,
+                          fo);
+            }
+        }
+    } else {
+        const float e2f = (float)e2;
+        for (uint32_t j0 = g; j0 < n; j0 += 32 * G) {
+            const uint32_t j1 = min(n, j0 + 32 * G);
+            float t6[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (self_zero) {
+#pragma unroll 4
+                for (uint32_t j = j0; j < j1; j += G) {
+                    const double4 a = lpp[j], b = lpv[j];
+                    pair_mixed(pi, a.x, a.y, a.z, b.x, b.y, b.z, (float)a.w, e2f, t6);
+                }
+            } else {
+                for (uint32_t j = j0; j < j1; j += G) {
+                    const double4 a = lpp[j], b = lpv[j];
+                    const bool me = j == i;
+                    pair_mixed(pi, me ? pi[0] + 1.0 : a.x, a.y, a.z, b.x, b.y, b.z,
+                               me ? 0.f : (float)a.w, e2f, t6);
+                }
+            }
+            for (int k = 0; k < 6; ++k) fo[k] += (double)t6[k];
+        }
+    }
+}
+
+// Sums fo over the wave's lanes with the same slot (lane mod P, P < 64 a
+// power of two) and stores each slot's six sums at its row.  Swapping halves
+// and rows of 16 between two components leaves each half its own three and
+// each row one or two, so the later levels move 2 values instead of 6 (41
+// instructions at P = 1; 156 with all six carried through six levels).
+__device__ __forceinline__ void small_reduce(const double fo[6], uint32_t P, double *row) {
+    const uint32_t lane = __lane_id();
+    double a, b, u[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {  // lower half: components 0..2, upper: 3..5
+        swap_rows<2>(fo[k], fo[3 + k], a, b);
+        u[k] = a + b;
+    }
+    const uint32_t q = lane >= 32 ? 3u : 0u;
+    if (P == 32) {
+        for (int k = 0; k < 3; ++k) row[q + k] = u[k];
+        return;
+    }
+    swap_rows<1>(u[0], u[1], a, b);  // even rows: component q, odd: q + 1
+    double x = a + b;
+    swap_rows<1>(u[2], u[2], a, b);  // both: q + 2
+    double y = a + b;
+    // rotations by 8, 4, 2, 1 inside the rows: lane ^ 8, and so on (uniform
+    // under the larger ones by then)
+    if (P <= 8) {
+        x += dpp<0x128>(x, x);
+        y += dpp<0x128>(y, y);
+    }
+    if (P <= 4) {
+        x += dpp<0x124>(x, x);
+        y += dpp<0x124>(y, y);
+    }
+    if (P <= 2) {
+        x += dpp<0x122>(x, x);
+        y += dpp<0x122>(y, y);
+    }
+    if (P == 1) {
+        x += dpp<0x121>(x, x);
+        y += dpp<0x121>(y, y);
+    }
+    if ((lane & 15u) < P) {
+        const bool odd = (lane & 16u) != 0;
+        row[q + (odd ? 1u : 0u)] = x;
+        if (!odd) row[q + 2] = y;
+    }
+}
+
+// Block steps of systems of n <= SN particles, workgroup c of SB threads for
 // cluster c (a larger cluster's workgroup returns at once), up to max_run
 // steps per launch; clusters are independent, so the workgroups never wait
-// for each other.  Thread i owns particle i of its cluster and
-// keeps its position, velocity, forces, time and step in registers for the
+// for each other.  Thread t owns particles t and t + SB of its cluster and
+// keeps their position, velocity, forces, time and step in registers for the
 // whole launch; the threads exchange the predictor records and the active
 // list through LDS, and the state goes to HBM as it changes (stores
 // that nothing in the launch reads back).  Each step is the device loop's
 // step: predictor of all particles at the block time T, the particles with
 // t + dt = T (Hermite4::find_particles_to_move), their old forces, the pair
 // sums, the corrector and new step, the next block time min(t + dt) and the
-// loop tail (the record_tail of each step).  The active set of the next step is counted
-// before its predictor; when it is empty or larger than max_act the launch
-// ends and leaves that step to the multi-workgroup kernels.
+// loop tail (the record_tail of each step; the counters go out at the end).
+// The active set of the next step is counted before its predictor; when it
+// is empty or larger than max_act the launch ends and leaves that step to
+// the multi-workgroup kernels.
 //
-// Pair sums: P = nact rounded up to a power of two i slots over PT threads
-// (all SB for P >= 64, H4_SMALL_NARROW_WAVES waves below), G = PT / P lanes
-// per slot (lane g of slot p takes j = g, g + G, ...; P >= 64 puts one j per
-// wave, an LDS broadcast), reduced by shuffles inside a wave and in wave
-// order through LDS: a fixed order for a given nact.  The mixed path folds
-// its FP32 runs into FP64 every 32 pairs, as the main kernel does.  On exit
+// Pair sums: P = nact rounded up to a power of two i slots and G groups of
+// lanes; a lane of group g takes one slot and j = g, g + G, ...  P < 64:
+// G = SB / P, a wave's groups summed by halving (small_reduce: neighbouring
+// groups first, so a lane's group is its slot-free bits reversed), the waves'
+// sums in order through LDS.  P >= 64: G = 1024 / P in two passes, one j per
+// wave (an LDS broadcast), summed in group order.  A fixed order for a given
+// nact.  The mixed path folds its FP32 runs into FP64 every 32 pairs, as the
+// main kernel does.  The corrector of slot k runs on 8 lanes (corr8), slots
+// 0-7 on the first wave; waves without one take the minima of the particles
+// that are not active.  The next block time is the minimum over those and
+// the new steps; with at most 64 active particles every wave reads the new
+// steps itself and makes the next active list without another barrier: three
+// barriers per step.
+//
+// What bounds a step is the chain of these phases on one CU, at n = 1024 also
+// its pairs.  Cycles per step, of the form before (1024 threads, shuffles, a
+// one-lane corrector of 5900 cycles, counters read back from memory, 8
+// barriers) and of this one: n = 256 14300 and 7600, n = 1024 21400 and
+// 13900.  512 threads of two particles each have 256 registers: 1024 threads
+// spilled 62 around the pair loop, 5000 cycles of a step at n = 1024.  On exit
 // the predictor records of the last step and the per-block minima of t + dt
 // are stored for the kernels that follow.
 template <bool MIXED>
@@ -1584,45 +1829,63 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
                                                   double dt_min, double dt_max,
                                                   uint32_t self_zero) {
 #pragma clang fp contract(off)
-    __shared__ double4 lpp[SB], lpv[SB];  // predictor records
-    __shared__ __align__(16) double red[6 * SB];  // pair sums per (group, slot); corrector output
+    __shared__ double4 lpp[SN], lpv[SN];          // predictor records
+    __shared__ __align__(16) double red[6 * SN];  // pair sums per (group, slot)
     __shared__ double stg[7 * SMALL_MAX_ACT];     // old forces and step per active slot
-    __shared__ uint32_t lact[SB];          // active list
-    __shared__ uint32_t wcnt[SB / 64];
-    __shared__ double wmin[SB / 64];
+    __shared__ double outs[13 * SMALL_MAX_ACT];   // new forces, position, velocity, step
+    // t + dt (inf: active, or no particle), behind the sums of a step with
+    // P < 64
+    double *rest = red + 4 * SN;
+    static_assert(6 * 32 * SW <= 4 * SN, "sums of 32 slots");
+    __shared__ uint32_t lact[SN];                 // active list
+    __shared__ double wmin[SC], cmin[SW];         // minimum of rest per chunk
+    __shared__ unsigned long long wmask[SC];      // the particles that have it
+    __shared__ uint32_t wcnt[SC];
 
     const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid >> 6;
     const uint32_t c = blockIdx.x;
     ClState *cs = &e.cs[c];
     const uint32_t n = e.cnt[c];
-    if (n > SB) return;
+    if (n > SN) return;
     const uint32_t off = e.off[c];  // first particle of the cluster
-    const bool in = tid < n;
     if (max_act > SMALL_MAX_ACT) max_act = SMALL_MAX_ACT;
     if (cs->done) return;
     const double t_end = e.ctl->t_end, t_stop = e.ctl->t_stop;
     const unsigned long long max_steps = e.ctl->max_steps;
     unsigned long long steps = cs->steps;
+    unsigned long long inter = cs->interactions, nst = cs->nsteps;
     uint32_t hk = (uint32_t)(steps % e.hist_cap);  // history slot of the next step
     double T = cs->atime;
     // self_zero (set by the host, self_pair_is_zero): a particle's pair with
     // itself (r = 0, v = 0) has a finite weight m / e2^1.5 for every mass of
     // the context, so it adds exact zeros and the j loop needs no test for it.
 
-    double r[3] = {0.0, 0.0, 0.0}, v[3] = {0.0, 0.0, 0.0};
-    double f[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double ti = 0.0, dti = 0.0;
-    float mf = 0.0f;
-    if (in) {
-        const uint32_t gi = off + tid;
-        for (int k = 0; k < 3; ++k) {
-            r[k] = s.r[k][gi];
-            v[k] = s.v[k][gi];
+    bool in[SP], act[SP];
+    double r[SP][3], v[SP][3], f[SP][6], ti[SP], dti[SP], tdt[SP];
+    float mf[SP];
+#pragma unroll
+    for (uint32_t k = 0; k < SP; ++k) {
+        in[k] = tid + k * SB < n;
+        for (int q = 0; q < 3; ++q) r[k][q] = v[k][q] = 0.0;
+        for (int q = 0; q < 6; ++q) f[k][q] = 0.0;
+        ti[k] = dti[k] = 0.0;
+        mf[k] = 0.0f;
+        if (in[k]) {
+            const uint32_t gi = off + tid + k * SB;
+            for (int q = 0; q < 3; ++q) {
+                r[k][q] = s.r[q][gi];
+                v[k][q] = s.v[q][gi];
+            }
+            for (int q = 0; q < 6; ++q) f[k][q] = s.f[q][gi];
+            ti[k] = s.t[gi];
+            dti[k] = s.dt[gi];
+            mf[k] = (float)s.m[gi];
         }
-        for (int k = 0; k < 6; ++k) f[k] = s.f[k][gi];
-        ti = s.t[gi];
-        dti = s.dt[gi];
-        mf = (float)s.m[gi];
+        tdt[k] = in[k] ? ti[k] + dti[k] : (double)INFINITY;
+    }
+    if (tid < SC) {  // (chunks without a particle are never minimised)
+        wmin[tid] = INFINITY;
+        wmask[tid] = 0;
     }
     // The loop tail the cluster's last multi-workgroup step left comes
     // first; its next block time is the minimum of t + dt, which these
@@ -1632,219 +1895,257 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
         const double Tp = cs->tail_t;
         const uint32_t np = cs->tail_nact;
         steps = cs->tail_steps + 1;
-        const double mn = small_min(in ? ti + dti : (double)INFINITY, wmin);
-        const bool stop = loop_stops(*e.ctl, Tp, steps, mn);
+        const double mn = small_min(tdt, cmin);
+        const bool last = loop_stops(*e.ctl, Tp, steps, mn);
         if (tid == 0) {
-            record_tail(e, c, Tp, np, steps, mn, stop);
+            record_tail(e, c, Tp, np, steps, mn, last);
             cs->tail_pend = 0;
             e.ctl->ndirty[0] = e.ctl->ndirty[1] = 0;
         }
-        if (stop) return;  // (the block minima are the finish pass's)
+        if (last) return;  // (the block minima are the finish pass's)
+        inter += (unsigned long long)np * n;
+        nst += np;
         hk = (uint32_t)(steps % e.hist_cap);
         T = mn;
     }
-    bool act = in && fabs(T - (ti + dti)) < 2 * DBL_EPSILON;
-    uint32_t k_act;  // this particle's place in the active list
+    uint32_t k_act[SP];  // the particles' places in the active list
+    for (uint32_t k = 0; k < SP; ++k)
+        act[k] = in[k] && fabs(T - tdt[k]) < 2 * DBL_EPSILON;
     uint32_t nact = small_count(act, wcnt, k_act);
 
     uint32_t it = 0;
-    for (; it < max_run && nact >= 1 && nact <= max_act; ++it) {
+    bool stop = false;
+    double t_last = 0.0;
+    const size_t np = (size_t)e.nblk * JT;  // the state's columns are np apart
+    // Corrector lanes: slot k on lanes 8 (k % 8) ... + 7 of wave k / 8 (the
+    // first waves, which the SIMDs issue first, prepare it before their pairs).
+    const bool vel = (lane & 4u) != 0;
+    const uint32_t cc = min(lane & 3u, 2u), cq = cc + (vel ? 3u : 0u);
+    for (; !stop && it < max_run && nact >= 1 && nact <= max_act; ++it) {
         // Predictor of every particle at T; active list.
-        if (in) {
-            double4 a, b;
-            predict_vals(r, v, f, T - ti, mf, a, b);
-            lpp[tid] = a;
-            lpv[tid] = b;
-        }
-        if (act) {
-            lact[k_act] = tid;
-            for (int k = 0; k < 6; ++k) stg[k_act * 7 + k] = f[k];
-            stg[k_act * 7 + 6] = dti;
+#pragma unroll
+        for (uint32_t k = 0; k < SP; ++k) {
+            const uint32_t i = tid + k * SB;
+            if (in[k]) {
+                double4 a, b;
+                predict_vals(r[k], v[k], f[k], T - ti[k], mf[k], a, b);
+                lpp[i] = a;
+                lpv[i] = b;
+            }
+            if (act[k]) {
+                lact[k_act[k]] = i;
+                double *st = stg + 7 * k_act[k];
+                for (int q = 0; q < 6; ++q) st[q] = f[k][q];
+                st[6] = dti[k];
+            }
+            if (nact <= 32) rest[i] = act[k] ? (double)INFINITY : tdt[k];
         }
         __syncthreads();
 
-        // Pair sums of the active particles on PT threads: all SB when
-        // P >= 64 (one slot per lane), H4_SMALL_NARROW_WAVES waves when
-        // P < 64 (the same FP64 work per SIMD with fewer cross-lane and
-        // cross-wave sums).
         const uint32_t lp = nact > 1 ? 32u - (uint32_t)__clz(nact - 1) : 0u;
         const uint32_t P = 1u << lp;
-        const uint32_t PT = P < 64 ? 64u * H4_SMALL_NARROW_WAVES : SB;
-        const uint32_t G = PT >> lp;
-        const uint32_t slot = tid & (P - 1), g = tid >> lp;
-        const bool pt = tid < PT;  // (PT is a multiple of 64: wave-uniform)
-        const uint32_t i = lact[slot < nact ? slot : nact - 1];
-        double pi[6];
+        const bool corr = 8 * w < nact;  // this wave has corrector slots
+        Corr8 ck{};
+        double o0 = 0.0, o1 = 0.0, pr = 0.0;
+        auto corr_prepare = [&](uint32_t k) {
+            const double *st = stg + 7 * k;
+            const uint32_t ia = lact[k];
+            o0 = st[cc];
+            o1 = st[3 + cc];
+            ck = corr8_coef(st[6], T, vel);
+            pr = reinterpret_cast<const double *>(vel ? lpv + ia : lpp + ia)[cc];
+        };
+        if (corr) corr_prepare(min(8 * w + lane / 8, nact - 1));
+
+        // Pair sums.
         {
-            const double4 a = lpp[i], b = lpv[i];
-            pi[0] = a.x;
-            pi[1] = a.y;
-            pi[2] = a.z;
-            pi[3] = b.x;
-            pi[4] = b.y;
-            pi[5] = b.z;
-        }
-        double fo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (!pt) {
-        } else if constexpr (!MIXED) {
-            if (self_zero) {
-                for (uint32_t j = g; j < n; j += G) {
-                    const double4 a = lpp[j], b = lpv[j];
-                    pair_fp64(pi, a.x, a.y, a.z, b.x, b.y, b.z, a.w, e2, fo);
-                }
+            const uint32_t slot = tid & (P - 1);
+            const uint32_t i = lact[min(slot, nact - 1)];
+            double pi[6];
+            {
+                const double4 a = lpp[i], b = lpv[i];
+                pi[0] = a.x;
+                pi[1] = a.y;
+                pi[2] = a.z;
+                pi[3] = b.x;
+                pi[4] = b.y;
+                pi[5] = b.z;
+            }
+            double fo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+            if (P < 64) {
+                const uint32_t g = w * (64 >> lp) + (__brev(lane >> lp) >> (26 + lp));
+                small_pairs<MIXED>(pi, i, g, SB >> lp, n, lpp, lpv, e2, self_zero, fo);
+                small_reduce(fo, P, red + (w * P + slot) * 6);
             } else {
-                for (uint32_t j = g; j < n; j += G) {
-                    const double4 a = lpp[j], b = lpv[j];
-                    const bool me = j == i;
-                    pair_fp64(pi, me ? pi[0] + 1.0 : a.x, a.y, a.z, b.x, b.y, b.z,
-                              me ? 0.0 : a.w, e2, fo);
+                const uint32_t G = SN >> lp;
+                for (uint32_t g = tid >> lp; g < G; g += SB >> lp) {
+                    for (int k = 0; k < 6; ++k) fo[k] = 0.0;
+                    small_pairs<MIXED>(pi, i, g, G, n, lpp, lpv, e2, self_zero, fo);
+                    double2 *row = reinterpret_cast<double2 *>(red + (g * P + slot) * 6);
+                    row[0] = make_double2(fo[0], fo[1]);
+                    row[1] = make_double2(fo[2], fo[3]);
+                    row[2] = make_double2(fo[4], fo[5]);
+                }
+            }
+        }
+        __syncthreads();
+
+        auto rest_min = [&](uint32_t q, double x) {
+            const double m = wave_min(x);
+            const unsigned long long mask = __ballot(fabs(m - x) < 2 * DBL_EPSILON);
+            if (lane == 0) {
+                wmin[q] = m;
+                wmask[q] = mask;
+            }
+        };
+        const uint32_t chunks = (n + 63) / 64;
+        const uint32_t corr_waves = (nact + 7) / 8;  // (P < 64: at most 4 of SW)
+        if (corr) {
+            for (uint32_t k0 = 8 * w; k0 < nact; k0 += 8 * SW) {
+                const uint32_t k = min(k0 + lane / 8, nact - 1);
+                if (k0 != 8 * w) corr_prepare(k);
+                // groups in order: 8 (P < 64), else 1024 / P = 16, 8 or 4
+                double fq = 0.0;
+                const double *rk = red + k * 6 + cq;
+                const uint32_t ngrp = P < 64 ? SW : SN >> lp;
+                for (uint32_t q0 = 0; q0 < ngrp; q0 += 4) {
+#pragma unroll
+                    for (uint32_t q = 0; q < 4; ++q) fq += rk[(q0 + q) * P * 6];
+                }
+                if (!MIXED) fq *= PAIR_SCALE;
+                const double fx = xor4(fq);
+                double x, ad;
+                const double dtn = corr8(ck, vel, o0, o1, vel ? fx : fq, vel ? fq : fx, pr, eta,
+                                         dt_min, dt_max, x, ad);
+                if (k0 + lane / 8 < nact && (lane & 3u) < 3u) {
+                    double *out = outs + 13 * k;
+                    out[cq] = fq;
+                    out[6 + cq] = x;
+                    const uint32_t gi = off + lact[k];
+                    auto *col = in_loop(s.r[0]) + gi;  // one base: one SGPR pair
+                    col[(cq + (vel ? COL_R + 1 : COL_R)) * np] = x;  // (m between r and v)
+                    col[(cq + COL_F) * np] = fq;
+                    col[(cq + COL_OLD) * np] = vel ? o1 : o0;
+                    col[(cq + COL_A2) * np] = ad;
+                    if ((lane & 7u) == 0) {
+                        out[12] = dtn;
+                        col[COL_T * np] = T;
+                        col[COL_DT * np] = dtn;
+                    }
+                }
+            }
+        } else if (P < 64) {
+            for (uint32_t q = w - corr_waves; q < chunks; q += SW - corr_waves)
+                rest_min(q, rest[64 * q + lane]);
+        }
+        if (P >= 64)
+#pragma unroll
+            for (uint32_t k = 0; k < SP; ++k)
+                rest_min(k * SW + w, act[k] ? (double)INFINITY : tdt[k]);
+        __syncthreads();
+
+        // The owners take their corrected state.
+#pragma unroll
+        for (uint32_t k = 0; k < SP; ++k)
+            if (act[k]) {
+                const double *o = outs + 13 * k_act[k];
+                for (int q = 0; q < 6; ++q) f[k][q] = o[q];
+                for (int q = 0; q < 3; ++q) {
+                    r[k][q] = o[6 + q];
+                    v[k][q] = o[9 + q];
+                }
+                ti[k] = T;
+                dti[k] = o[12];
+                tdt[k] = T + o[12];
+            }
+
+        // Next block time (Hermite4::next_integration_time): the minimum over
+        // the not-active minima and the active slots' new times, and the
+        // particles that have it.  A time that is not the minimum but within
+        // find_particles_to_move's tolerance of it (steps below 2^-50) sends
+        // every wave to the counting below.
+        double mn;
+        bool close;
+        uint32_t cnt = 0;
+        if (nact <= 64) {
+            const double wv = wmin[lane % SC];
+            const uint32_t wc = (uint32_t)__popcll(wmask[lane % SC]);
+            const double x = lane < nact ? T + outs[13 * min(lane, nact - 1) + 12]
+                                         : (double)INFINITY;
+            mn = wave_min(vmin(x, wv));
+            close = __ballot((wv != mn && fabs(mn - wv) < 2 * DBL_EPSILON) ||
+                             (x != mn && fabs(mn - x) < 2 * DBL_EPSILON)) != 0;
+            const unsigned long long cm = __ballot(x == mn && lane < nact);
+            const unsigned long long at = __ballot(wv == mn);  // bit q: chunk q has the minimum
+            const uint32_t mine = wv == mn ? wc : 0u;
+            const uint32_t base = (uint32_t)__popcll(cm);
+            cnt = base + row_sum(mine);
+#pragma unroll
+            for (uint32_t k = 0; k < SP; ++k) {
+                const uint32_t q = k * SW + w;
+                const unsigned long long mask = wmask[q];
+                const uint32_t below = row_sum(lane % SC < q ? mine : 0u);
+                if (act[k]) {
+                    act[k] = (cm >> k_act[k]) & 1ull;
+                    k_act[k] = (uint32_t)__popcll(cm & ((1ull << k_act[k]) - 1ull));
+                } else {
+                    act[k] = ((at >> q) & 1ull) && ((mask >> lane) & 1ull);
+                    k_act[k] = base + below + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
                 }
             }
         } else {
-            const float e2f = (float)e2;
-            for (uint32_t j0 = g; j0 < n; j0 += 32 * G) {
-                const uint32_t j1 = min(n, j0 + 32 * G);
-                float t6[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                if (self_zero) {
-                    for (uint32_t j = j0; j < j1; j += G) {
-                        const double4 a = lpp[j], b = lpv[j];
-                        pair_mixed(pi, a.x, a.y, a.z, b.x, b.y, b.z, (float)a.w, e2f, t6);
-                    }
-                } else {
-                    for (uint32_t j = j0; j < j1; j += G) {
-                        const double4 a = lpp[j], b = lpv[j];
-                        const bool me = j == i;
-                        pair_mixed(pi, me ? pi[0] + 1.0 : a.x, a.y, a.z, b.x, b.y, b.z,
-                                   me ? 0.f : (float)a.w, e2f, t6);
-                    }
-                }
-                for (int k = 0; k < 6; ++k) fo[k] += (double)t6[k];
-            }
-        }
-        if (P < 64 && pt)
-            for (uint32_t o = P; o < 64; o <<= 1)
-                for (int k = 0; k < 6; ++k) fo[k] += __shfl_xor(fo[k], (int)o);
-        // P <= 64: wave w holds the sums of slots 0..P-1 in lanes 0..P-1
-        // (group w); P > 64: every lane holds one slot, group g.
-        const uint32_t ngrp = P <= 64 ? PT / 64 : G;
-        if (pt && (P > 64 || lane < P)) {
-            const uint32_t grp = P <= 64 ? w : g;
-            for (int k = 0; k < 6; ++k) red[(grp * P + slot) * 6 + k] = fo[k];
-        }
-        __syncthreads();
-
-        // Corrector of active slot tid (threads 0 .. nact-1, the first waves:
-        // each wave that holds an active slot runs the whole corrector).
-        double fn[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        double rn[3], vn[3], dtn = 0.0;
-        if (tid < nact) {
-            // groups in order; ngrp <= SB / 64 (unrolled: the loads issue together)
-#pragma unroll
-            for (uint32_t q = 0; q < SB / 64; ++q) {
-                const bool use = q < ngrp;
-                const double2 *rp =
-                    reinterpret_cast<const double2 *>(red + ((use ? q : 0u) * P + tid) * 6);
-                const double2 x0 = rp[0], x1 = rp[1], x2 = rp[2];
-                fn[0] = use ? fn[0] + x0.x : fn[0];
-                fn[1] = use ? fn[1] + x0.y : fn[1];
-                fn[2] = use ? fn[2] + x1.x : fn[2];
-                fn[3] = use ? fn[3] + x1.y : fn[3];
-                fn[4] = use ? fn[4] + x2.x : fn[4];
-                fn[5] = use ? fn[5] + x2.y : fn[5];
-            }
-            if (!MIXED)
-                for (int k = 0; k < 6; ++k) fn[k] *= PAIR_SCALE;
-            const uint32_t ia = lact[tid];  // within the cluster
-            const uint32_t gi = off + ia;
-            double o[6], pr[6], a2[3], a3[3];
-            for (int k = 0; k < 6; ++k) o[k] = stg[tid * 7 + k];
-            {
-                const double4 a = lpp[ia], b = lpv[ia];
-                pr[0] = a.x;
-                pr[1] = a.y;
-                pr[2] = a.z;
-                pr[3] = b.x;
-                pr[4] = b.y;
-                pr[5] = b.z;
-            }
-            dtn = correct_vals(o, fn, pr, stg[tid * 7 + 6], T, eta, dt_min, dt_max, rn, vn, a2,
-                               a3);
-            for (int k = 0; k < 6; ++k) {
-                in_loop(s.old[k])[gi] = o[k];
-                in_loop(s.f[k])[gi] = fn[k];
-            }
-            for (int k = 0; k < 3; ++k) {
-                in_loop(s.r[k])[gi] = rn[k];
-                in_loop(s.v[k])[gi] = vn[k];
-                in_loop(s.a2[k])[gi] = a2[k];
-                in_loop(s.a3[k])[gi] = a3[k];
-            }
-            in_loop(s.t)[gi] = T;
-            in_loop(s.dt)[gi] = dtn;
-        }
-        __syncthreads();  // red is read: the corrected state goes there for the owners
-        if (tid < nact) {
-            double *out = red + tid * 13;
-            for (int k = 0; k < 6; ++k) out[k] = fn[k];
-            for (int k = 0; k < 3; ++k) {
-                out[6 + k] = rn[k];
-                out[9 + k] = vn[k];
-            }
-            out[12] = dtn;
-        }
-        __syncthreads();
-        if (act) {
-            const double *in_ = red + k_act * 13;
-            for (int k = 0; k < 6; ++k) f[k] = in_[k];
-            for (int k = 0; k < 3; ++k) {
-                r[k] = in_[6 + k];
-                v[k] = in_[9 + k];
-            }
-            ti = T;
-            dti = in_[12];
+            mn = small_min(tdt, cmin);
+            close = true;
         }
 
-        // Next block time (Hermite4::next_integration_time) and loop tail.
-        const double mn = small_min(in ? ti + dti : (double)INFINITY, wmin);
+        // Loop tail.
         steps += 1;
-        const bool stop = T >= t_stop || steps >= max_steps || !(T < t_end) || !(mn > T);
+        stop = T >= t_stop || steps >= max_steps || !(T < t_end) || !(mn > T);
+        inter += (unsigned long long)nact * n;
+        nst += nact;
+        if (c == 0 && tid == 0) {
+            e.hist_t[hk] = T;
+            e.hist_n[hk] = nact;
+        }
+        t_last = T;
+        T = mn;
+        if (++hk == e.hist_cap) hk = 0;
+        if (close) {  // (uniform over the workgroup)
+            for (uint32_t k = 0; k < SP; ++k)
+                act[k] = in[k] && fabs(T - tdt[k]) < 2 * DBL_EPSILON;
+            cnt = small_count(act, wcnt, k_act);
+        }
+        nact = cnt;
+    }
+
+    // Loop state and predictor records of the last step made; per-block
+    // minima of t + dt.
+    if (it > 0) {
         if (tid == 0) {
-            if (c == 0) {
-                e.hist_t[hk] = T;
-                e.hist_n[hk] = nact;
-            }
-            cs->itime = T;
-            cs->atime = mn;
+            cs->itime = t_last;
+            cs->atime = T;
             cs->steps = steps;
-            cs->interactions += (unsigned long long)nact * n;
-            cs->nsteps += nact;
-            cs->small_steps += 1;
+            cs->interactions = inter;
+            cs->nsteps = nst;
+            cs->small_steps += it;
             if (stop) {
                 cs->done = 1;
                 atomicAdd(&e.ctl->ndone, 1u);
             }
         }
-        T = mn;
-        if (++hk == e.hist_cap) hk = 0;
-        if (stop) {
-            ++it;
-            break;
-        }
-        act = in && fabs(T - (ti + dti)) < 2 * DBL_EPSILON;
-        nact = small_count(act, wcnt, k_act);
-    }
-
-    // Predictor records of the last step made; per-block minima of t + dt.
-    if (it > 0 && in) {
-        s.pp[off + tid] = lpp[tid];
-        s.pv[off + tid] = lpv[tid];
+        for (uint32_t k = 0; k < SP; ++k)
+            if (in[k]) {
+                s.pp[off + tid + k * SB] = lpp[tid + k * SB];
+                s.pv[off + tid + k * SB] = lpv[tid + k * SB];
+            }
     }
     __syncthreads();  // wmin is rewritten below
-    double vb = in ? ti + dti : (double)INFINITY;
-    for (int o = 32; o > 0; o >>= 1) vb = fmin(vb, __shfl_xor(vb, o));
-    if (lane == 0) wmin[w] = vb;
+    for (uint32_t k = 0; k < SP; ++k) {
+        const double m = wave_min(tdt[k]);
+        if (lane == 0) wmin[k * SW + w] = m;
+    }
     __syncthreads();
-    constexpr uint32_t WPB = JT / 64;  // waves per block
+    constexpr uint32_t WPB = JT / 64;  // chunks per block
     if (tid < ntiles(e, c)) {
         double m = wmin[tid * WPB];
         for (uint32_t k = 1; k < WPB; ++k) m = fmin(m, wmin[tid * WPB + k]);
@@ -2225,7 +2526,7 @@ int launch_plan(h4h_ctx *ctx) {
     return H4H_OK;
 }
 
-// Whether the device can launch k_small_run (SB threads, 130 KiB of LDS).
+// Whether the device can launch k_small_run (SB threads, 157 KiB of LDS).
 bool small_fits(int device) {
     int lds = 0;
     if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
@@ -2240,12 +2541,12 @@ bool small_fits(int device) {
 }
 
 // Device loops of this context start each step slot with k_small_run: every
-// cluster has at most SB particles.  (With larger clusters beside them, the
+// cluster has at most SN particles.  (With larger clusters beside them, the
 // small clusters' runs of up to SMALL_RUN steps would hold up the larger
 // clusters' steps, which wait for the launch to end.)
 bool small_path(const h4h_ctx *ctx) {
     return ctx->small_ok && ctx->small_act > 0 && ctx->precision != H4H_FP64_EXACT &&
-           *std::max_element(ctx->cnt.begin(), ctx->cnt.end()) <= SB;
+           *std::max_element(ctx->cnt.begin(), ctx->cnt.end()) <= SN;
 }
 
 // Whether the pair loop of `precision` may add a particle's pair with itself
@@ -2610,7 +2911,11 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     for (int c = 0; c < 3; ++c) (void)take();
     s.pv = reinterpret_cast<double4 *>(take());
     for (int c = 0; c < 3; ++c) (void)take();
-    if (b != ctx->state + (size_t)np * N_SOA) return cleanup(fail(H4H_EINVAL, "state layout"));
+    if (b != ctx->state + (size_t)np * N_SOA || s.v[0] != s.r[0] + 4 * np ||
+        s.f[0] != s.r[0] + COL_F * np || s.old[0] != s.r[0] + COL_OLD * np ||
+        s.a2[0] != s.r[0] + COL_A2 * np || s.a3[0] != s.a2[0] + 3 * np ||
+        s.t != s.r[0] + COL_T * np || s.dt != s.r[0] + COL_DT * np)
+        return cleanup(fail(H4H_EINVAL, "state layout"));
     ok = hipMemcpyAsync(ctx->d_off, ctx->off.data(), K * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
          hipMemcpyAsync(ctx->d_cnt, ctx->cnt.data(), K * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
          hipMemcpyAsync(ctx->d_hoff, ctx->hoff.data(), K * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
