@@ -53,6 +53,9 @@ int fail(int code, const std::string &msg) {
 #define H4_MIXED_UNROLL 2
 #endif
 
+// Columns of a context's state from r[0] on (create_impl lays them out).
+constexpr uint32_t COL_R = 0, COL_F = 7, COL_OLD = 13, COL_A2 = 19, COL_T = 25, COL_DT = 26;
+
 constexpr uint32_t DEFAULT_GRID = 2048;       // persistent workgroups
 constexpr uint32_t DEFAULT_MAX_SPLIT = 1024;  // largest j split
 constexpr uint32_t ENERGY_OUT = 8 * ENERGY_GRID;  // workgroup sums of one energy launch
@@ -304,6 +307,145 @@ __device__ void plan_all(const Ens &e, uint32_t exact) {
 __global__ __launch_bounds__(BS) void k_plan(Ens e, uint32_t exact) { plan_all(e, exact); }
 
 // ---------------------------------------------------------------------------
+// Exchanges inside a wave
+// ---------------------------------------------------------------------------
+
+// Lane exchanges by DPP (a few cycles; a ds_bpermute shuffle takes ~100):
+// CTRL is the DPP control, BANK the banks of four lanes that take it (the
+// others keep `old`).
+template <int CTRL, int BANK = 0xf>
+__device__ __forceinline__ double dpp(double old, double x) {
+    const unsigned long long o = __builtin_bit_cast(unsigned long long, old);
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)o, (int)(uint32_t)u,
+                                                              CTRL, 0xf, BANK, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(
+        (int)(uint32_t)(o >> 32), (int)(uint32_t)(u >> 32), CTRL, 0xf, BANK, false);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;     // quad_perm 1,0,3,2 and 2,3,0,1
+constexpr int DPP_QUADS = 0x141, DPP_EIGHTS = 0x140;  // row_half_mirror, row_mirror
+template <int K>
+__device__ __forceinline__ double quad_lane(double x) {  // lane K of each quad
+    return dpp<K * 0x55>(x, x);
+}
+// The value of lane ^ 4: row_shl:4 into banks 0 and 2, row_shr:4 into 1 and 3.
+__device__ __forceinline__ double xor4(double x) {
+    return dpp<0x114, 0xa>(dpp<0x104, 0x5>(x, x), x);
+}
+// Swaps the odd rows of 16 lanes (ROWS = 1; the upper half of 32: ROWS = 2)
+// of x with the even ones of y: an even row has then x of itself (a) and of
+// its odd neighbour (b), an odd row y of its even neighbour (a) and of
+// itself (b).
+template <int ROWS>
+__device__ __forceinline__ void swap_rows(double x, double y, double &a, double &b) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const unsigned long long t = __builtin_bit_cast(unsigned long long, y);
+    uint32_t l0, l1, h0, h1;
+    if constexpr (ROWS == 1) {
+        const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)t, false, false);
+        const auto hi =
+            __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(t >> 32), false, false);
+        l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+    } else {
+        const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)t, false, false);
+        const auto hi =
+            __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(t >> 32), false, false);
+        l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+    }
+    a = __builtin_bit_cast(double, ((unsigned long long)h0 << 32) | l0);
+    b = __builtin_bit_cast(double, ((unsigned long long)h1 << 32) | l1);
+}
+// v_min_f64 as it is (fmin also quiets both operands: two more instructions
+// each time; a NaN loses either way).
+__device__ __forceinline__ double vmin(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Sum over the lane's group of L = 1, 4, 16 or 64 consecutive lanes (all
+// lanes of the wave active; every lane of the group gets it): lane ^ 1 first.
+__device__ __forceinline__ double lanes_sum(double x, uint32_t L) {
+    double a, b;
+    if (L >= 4) {
+        x += dpp<DPP_XOR1>(x, x);
+        x += dpp<DPP_XOR2>(x, x);
+    }
+    if (L >= 16) {
+        x += dpp<DPP_QUADS>(x, x);   // (the quads are uniform by now,
+        x += dpp<DPP_EIGHTS>(x, x);  // and the eights)
+    }
+    if (L >= 64) {
+        swap_rows<1>(x, x, a, b);
+        x = a + b;
+        swap_rows<2>(x, x, a, b);
+        x = a + b;
+    }
+    return x;
+}
+
+// Minimum over the wave (all lanes active; every lane gets it).
+__device__ __forceinline__ double wave_min(double x) {
+    double a, b;
+    x = vmin(x, dpp<DPP_XOR1>(x, x));
+    x = vmin(x, dpp<DPP_XOR2>(x, x));
+    x = vmin(x, dpp<DPP_QUADS>(x, x));   // (the quads are uniform by now,
+    x = vmin(x, dpp<DPP_EIGHTS>(x, x));  // and the eights)
+    swap_rows<1>(x, x, a, b);
+    x = vmin(a, b);
+    swap_rows<2>(x, x, a, b);
+    return vmin(a, b);
+}
+
+// Sums fo over the wave's lanes with the same slot (lane mod P, P < 64 a
+// power of two) and stores each slot's six sums at its row.  Swapping halves
+// and rows of 16 between two components leaves each half its own three and
+// each row one or two, so the later levels move 2 values instead of 6 (41
+// instructions at P = 1; 156 with all six carried through six levels).
+__device__ __forceinline__ void slot_sums(const double fo[6], uint32_t P, double *row) {
+    const uint32_t lane = __lane_id();
+    double a, b, u[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {  // lower half: components 0..2, upper: 3..5
+        swap_rows<2>(fo[k], fo[3 + k], a, b);
+        u[k] = a + b;
+    }
+    const uint32_t q = lane >= 32 ? 3u : 0u;
+    if (P == 32) {
+        for (int k = 0; k < 3; ++k) row[q + k] = u[k];
+        return;
+    }
+    swap_rows<1>(u[0], u[1], a, b);  // even rows: component q, odd: q + 1
+    double x = a + b;
+    swap_rows<1>(u[2], u[2], a, b);  // both: q + 2
+    double y = a + b;
+    // rotations by 8, 4, 2, 1 inside the rows: lane ^ 8, and so on (uniform
+    // under the larger ones by then)
+    if (P <= 8) {
+        x += dpp<0x128>(x, x);
+        y += dpp<0x128>(y, y);
+    }
+    if (P <= 4) {
+        x += dpp<0x124>(x, x);
+        y += dpp<0x124>(y, y);
+    }
+    if (P <= 2) {
+        x += dpp<0x122>(x, x);
+        y += dpp<0x122>(y, y);
+    }
+    if (P == 1) {
+        x += dpp<0x121>(x, x);
+        y += dpp<0x121>(y, y);
+    }
+    if ((lane & 15u) < P) {
+        const bool odd = (lane & 16u) != 0;
+        row[q + (odd ? 1u : 0u)] = x;
+        if (!odd) row[q + 2] = y;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Predictor / active selection / save old (one workgroup per JT block)
 // ---------------------------------------------------------------------------
 
@@ -427,7 +569,7 @@ __global__ __launch_bounds__(BS) void k_select(Soa s, Ens e, uint32_t flags, dou
         const uint32_t b0 = single ? 0u : e.off[c] / JT, nb = single ? e.nblk : ntiles(e, c);
         double mn = INFINITY;
         for (uint32_t k = threadIdx.x; k < nb; k += BS) mn = fmin(mn, e.bmin[b0 + k]);
-        for (int o = 32; o > 0; o >>= 1) mn = fmin(mn, __shfl_xor(mn, o));
+        mn = wave_min(mn);
         if (__lane_id() == 0) wmin[threadIdx.x >> 6] = mn;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -630,39 +772,45 @@ __device__ __forceinline__ void tile_pairs(const double pi[6], uint32_t i,
     }
 }
 
-// Sums fo over the BS/IW j sub-groups of each i slot: shuffles across the
-// sub-groups inside a wave (lane bits >= log2(IW)), then LDS across the
-// BS/64 waves in wave order.  The fixed tree makes it deterministic.  On
-// return lanes threadIdx.x < IW hold the sums of slot threadIdx.x.
+// j sub-group of thread t of an IW-slot group: with IW < 64 slots a wave
+// holds 64 / IW sub-groups, numbered by their lane bits reversed so that
+// slot_sums adds neighbouring ones first.
 template <int IW>
-__device__ __forceinline__ void reduce_subgroups(double fo[6], double *red) {
+__device__ __forceinline__ uint32_t subgroup(uint32_t t) {
     if constexpr (IW < 64) {
-#pragma unroll
-        for (int o = IW; o < 64; o <<= 1)
-            for (int c = 0; c < 6; ++c) fo[c] += __shfl_xor(fo[c], o);
+        constexpr uint32_t bits = IW == 4 ? 4 : 2;
+        static_assert((IW << bits) == 64, "IW is 4 or 16");
+        return (t >> 6) * (64 / IW) + (__brev((t & 63u) / IW) >> (32 - bits));
+    } else {
+        return t / IW;
     }
+}
+
+// Sums fo over the BS/IW j sub-groups of each i slot (thread t of BS): in
+// the wave (slot_sums), then over the waves in order through red.  The fixed
+// tree makes it deterministic.  IW < BS: leaves, after a barrier, sum q of
+// slot k for subgroup_sum; IW = BS: fo already is the slot's.
+template <int IW>
+__device__ __forceinline__ void reduce_subgroups(const double fo[6], double *red, uint32_t t) {
     if constexpr (IW < BS) {
-        constexpr uint32_t W = BS / 64;            // waves
-        constexpr uint32_t SL = IW < 64 ? IW : 64;  // slots held per wave
-        uint32_t lane = __lane_id();
-        uint32_t w = threadIdx.x >> 6;
+        const uint32_t w = t >> 6;
         __syncthreads();
-        if (lane < SL) {
-            // wave w holds slots (w*64 .. w*64+63) % IW when IW >= 64
-            uint32_t slot = (IW >= 64) ? (threadIdx.x % IW) : lane;
-            uint32_t grp = (IW >= 64) ? (threadIdx.x / IW) : w;
-            for (int c = 0; c < 6; ++c) red[(grp * IW + slot) * 6 + c] = fo[c];
+        if constexpr (IW < 64) {
+            slot_sums(fo, IW, red + (w * IW + t % IW) * 6);
+        } else {
+            static_assert(IW == 64, "one slot per lane");
+            for (int c = 0; c < 6; ++c) red[t * 6 + c] = fo[c];
         }
         __syncthreads();
-        if (threadIdx.x < IW) {
-            constexpr uint32_t NG = (IW >= 64) ? BS / IW : W;
-            for (int c = 0; c < 6; ++c) {
-                double acc = red[threadIdx.x * 6 + c];
-                for (uint32_t g = 1; g < NG; ++g) acc += red[(g * IW + threadIdx.x) * 6 + c];
-                fo[c] = acc;
-            }
-        }
     }
+}
+
+// Sum q of slot k over the waves, in order (IW < BS).
+template <int IW>
+__device__ __forceinline__ double subgroup_sum(const double *red, uint32_t k, uint32_t q) {
+    double acc = red[k * 6 + q];
+    for (uint32_t g = 1; g < BS / 64; ++g) acc += red[(g * IW + k) * 6 + q];
+    return acc;
 }
 
 // FP64_EXACT: the pair terms of Hermite4CPU::update_acc_jrk
@@ -847,7 +995,7 @@ __device__ __forceinline__ void update_item(const Soa &s, const ClPlan &pl, uint
                                             uint32_t nact, double *partial, double e2,
                                             double4 *lA, double4 *lB, double *red) {
     const uint32_t il = threadIdx.x % IW;
-    const uint32_t js = threadIdx.x / IW;
+    const uint32_t js = subgroup<IW>(threadIdx.x);
     uint32_t k = it * IW + il;
     bool act = k < nact;
     uint32_t t0 = jt_begin + sc * pl.tpc;
@@ -929,17 +1077,30 @@ __device__ __forceinline__ void update_item(const Soa &s, const ClPlan &pl, uint
             tile(lA, tt);
         }
     }
-    reduce_subgroups<IW>(fo, red);
-    if (threadIdx.x < IW && act) {
-        constexpr double scale = MIXED ? 1.0 : PAIR_SCALE;  // pair_fp64's 3 sqrt(3)
-        if (pl.S == 1) {
-            for (int q = 0; q < 6; ++q) s.f[q][i] = fo[q] * scale;
-        } else {
-            // partial_at(pl, q, sc, k), with the layout's strides
-            const size_t kst = pl.cmaj ? pl.S : 1u, cst = pl.cmaj ? 1u : pl.rows;
+    reduce_subgroups<IW>(fo, red, threadIdx.x);
+    constexpr double scale = MIXED ? 1.0 : PAIR_SCALE;  // pair_fp64's 3 sqrt(3)
+    // partial_at(pl, q, sc, k), with the layout's strides
+    const size_t kst = pl.cmaj ? pl.S : 1u, cst = pl.cmaj ? 1u : pl.rows;
+    const size_t qs = (size_t)pl.S * pl.rows;
+    if constexpr (IW == BS) {
+        if (act) {
             double *pq = partial + (size_t)sc * cst + (size_t)k * kst;
-            const size_t qs = (size_t)pl.S * pl.rows;
-            for (int q = 0; q < 6; ++q) pq[q * qs] = fo[q] * scale;
+            if (pl.S == 1)
+                for (int q = 0; q < 6; ++q) s.f[q][i] = fo[q] * scale;
+            else
+                for (int q = 0; q < 6; ++q) pq[q * qs] = fo[q] * scale;
+        }
+    } else {
+        // one thread per slot and component (consecutive slots on
+        // consecutive threads)
+        for (uint32_t x = threadIdx.x; x < 6 * IW; x += BS) {
+            const uint32_t q = x / IW, sl = x % IW, ks = it * IW + sl;
+            if (ks >= nact) continue;
+            const double f = subgroup_sum<IW>(red, sl, q) * scale;
+            if (pl.S == 1)
+                s.f[0][(size_t)q * (s.f[1] - s.f[0]) + mv[ks]] = f;  // (columns equally spaced)
+            else
+                partial[(size_t)sc * cst + (size_t)ks * kst + q * qs] = f;
         }
     }
 }
@@ -1099,73 +1260,6 @@ __device__ __forceinline__ double correct_vals(const double o[6], const double f
     double normal_dt = sqrt(eta * ((abs_a1 * abs_a1_2 + abs_j12) /
                                    (abs_j1 * abs_a1_3 + abs_a1_22)));
     return normalize_dt(normal_dt, dt1, [&] { return dt_doubles(dt1, itime); }, dt_min, dt_max);
-}
-
-// Lane exchanges by DPP (a few cycles; a ds_bpermute shuffle takes ~100):
-// CTRL is the DPP control, BANK the banks of four lanes that take it (the
-// others keep `old`).
-template <int CTRL, int BANK = 0xf>
-__device__ __forceinline__ double dpp(double old, double x) {
-    const unsigned long long o = __builtin_bit_cast(unsigned long long, old);
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)o, (int)(uint32_t)u,
-                                                              CTRL, 0xf, BANK, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(
-        (int)(uint32_t)(o >> 32), (int)(uint32_t)(u >> 32), CTRL, 0xf, BANK, false);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;     // quad_perm 1,0,3,2 and 2,3,0,1
-constexpr int DPP_QUADS = 0x141, DPP_EIGHTS = 0x140;  // row_half_mirror, row_mirror
-template <int K>
-__device__ __forceinline__ double quad_lane(double x) {  // lane K of each quad
-    return dpp<K * 0x55>(x, x);
-}
-// The value of lane ^ 4: row_shl:4 into banks 0 and 2, row_shr:4 into 1 and 3.
-__device__ __forceinline__ double xor4(double x) {
-    return dpp<0x114, 0xa>(dpp<0x104, 0x5>(x, x), x);
-}
-// Swaps the odd rows of 16 lanes (ROWS = 1; the upper half of 32: ROWS = 2)
-// of x with the even ones of y: an even row has then x of itself (a) and of
-// its odd neighbour (b), an odd row y of its even neighbour (a) and of
-// itself (b).
-template <int ROWS>
-__device__ __forceinline__ void swap_rows(double x, double y, double &a, double &b) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-    const unsigned long long t = __builtin_bit_cast(unsigned long long, y);
-    uint32_t l0, l1, h0, h1;
-    if constexpr (ROWS == 1) {
-        const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)t, false, false);
-        const auto hi =
-            __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(t >> 32), false, false);
-        l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
-    } else {
-        const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)t, false, false);
-        const auto hi =
-            __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(t >> 32), false, false);
-        l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
-    }
-    a = __builtin_bit_cast(double, ((unsigned long long)h0 << 32) | l0);
-    b = __builtin_bit_cast(double, ((unsigned long long)h1 << 32) | l1);
-}
-// v_min_f64 as it is (fmin also quiets both operands: two more instructions
-// each time; a NaN loses either way).
-__device__ __forceinline__ double vmin(double a, double b) {
-    double r;
-    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
-// Minimum over the wave (all lanes active; every lane gets it).
-__device__ __forceinline__ double wave_min(double x) {
-    double a, b;
-    x = vmin(x, dpp<DPP_XOR1>(x, x));
-    x = vmin(x, dpp<DPP_XOR2>(x, x));
-    x = vmin(x, dpp<DPP_QUADS>(x, x));   // (the quads are uniform by now,
-    x = vmin(x, dpp<DPP_EIGHTS>(x, x));  // and the eights)
-    swap_rows<1>(x, x, a, b);
-    x = vmin(a, b);
-    swap_rows<2>(x, x, a, b);
-    return vmin(a, b);
 }
 
 // The corrector of one particle on 8 consecutive lanes of a wave (all lanes
@@ -1335,10 +1429,7 @@ __device__ __forceinline__ void chunk_sums(const Soa &s, const ClPlan &pl, const
                     if (s0 + u * L < pl.S) acc[q] += v[q][u];
         }
     }
-    for (int q = 0; q < 6; ++q) {
-        for (uint32_t o = 1; o < L; o <<= 1) acc[q] += __shfl_xor(acc[q], o);
-        f[q] = acc[q];
-    }
+    for (int q = 0; q < 6; ++q) f[q] = lanes_sum(acc[q], L);
 }
 
 // Finish pass of an update: adds the j-chunk partials of each active
@@ -1379,7 +1470,7 @@ __global__ __launch_bounds__(BS) void k_finish(Soa s, Ens e, const uint32_t *mov
 // ---------------------------------------------------------------------------
 
 __device__ __forceinline__ double block_min(double v, double *red) {
-    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+    v = wave_min(v);
     uint32_t w = threadIdx.x >> 6;
     if (__lane_id() == 0) red[w] = v;
     __syncthreads();
@@ -1440,11 +1531,18 @@ __global__ __launch_bounds__(BS) void k_blockmin_dirty(Soa s, Ens e, uint32_t pa
 // next block time makes.  (An ensemble keeps the two
 // launches: its many blocks with one or two active particles each would
 // put one corrector per workgroup instead of up to BS/L.)
+//
+// A small step's pass is one chain: list, partials, sums, corrector, minimum.
+// With at most 32 active particles in the block the corrector runs on 8 lanes
+// each (corr8); with that and DPP sums the average launch of an N = 10007 run
+// takes 6.9 us instead of 8.5, of an N = 65536 run 6.2 instead of 8.2.
 __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32_t *move,
                                                      const double *partial, float eta,
                                                      double dt_min, double dt_max, uint32_t par) {
     __shared__ double red[BS / 64];
     __shared__ double tnew[JT];  // t + dt of the block's corrected particles (NaN: not active)
+    constexpr uint32_t C8 = BS / 8;  // particles of one corr8 pass
+    __shared__ double fs[6 * C8];    // their forces
     ClState *cs = &e.cs[0];
     const uint32_t *dl = e.dirty + (size_t)par * 3 * e.nblk;
     // What the first block needs is requested at once: the loop's stop
@@ -1479,25 +1577,72 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
         // t + dt of the block as it stands, loaded ahead of the corrector
         const uint32_t j = b * JT + threadIdx.x;
         const double tdt = s.t[j] + s.dt[j];
-        __syncthreads();  // red and tnew of the previous block have been read
-        tnew[threadIdx.x] = NAN;
-        __syncthreads();
-        for (uint32_t base = 0; base < cnt; base += per) {
-            const uint32_t kk = base + threadIdx.x / L;
-            const bool valid = kk < cnt;
-            const uint32_t k = k0 + (valid ? kk : 0u);
-            const uint32_t i = move[k];
-            // the corrector's inputs from the selection's records: their
-            // loads go out with those of the partials
-            double o[6], pr[6], dt1 = 0.0;
-            if (valid) load_arec(e, k, o, pr, dt1);
-            double f[6];
-            chunk_sums(s, pl, partial, k, i, valid, f);
-            if (valid && threadIdx.x % L == 0) {
-                const double dtn = correct_store(s, i, o, pr, dt1, f, T, eta, dt_min, dt_max);
-                if (pl.S > 1)
-                    for (int q = 0; q < 6; ++q) s.f[q][i] = f[q];
-                tnew[i - b * JT] = T + dtn;
+        if (cnt <= C8) {
+            // The corrector of the kk-th active particle on lanes 8 kk ... + 7
+            // (beyond one pass of that, one lane each: 3 times fewer
+            // instructions).  Its inputs from the selection's records: their
+            // loads go out ahead of the partials'.
+            const uint32_t kk = threadIdx.x / 8, lane = threadIdx.x & 7u;
+            const bool mine = kk < cnt, vel = lane >= 4;
+            const uint32_t c = min(lane & 3u, 2u), q = c + (vel ? 3u : 0u);
+            const uint32_t ka = k0 + (mine ? kk : 0u);
+            const double *ar = reinterpret_cast<const double *>(e.arec);
+            const size_t np = (size_t)e.nblk * JT;
+            const double pr = ar[4 * ((vel ? np : 0) + ka) + c];
+            const double o0 = ar[4 * (2 * np + ka) + c], o1 = ar[4 * (3 * np + ka) + c];
+            const double dt1 = ar[4 * (2 * np + ka) + 3];
+            const uint32_t i = move[ka];
+            __syncthreads();  // red, tnew and fs of the previous block have been read
+            tnew[threadIdx.x] = NAN;
+            for (uint32_t base = 0; base < cnt; base += per) {
+                const uint32_t ks = base + threadIdx.x / L;
+                const bool valid = ks < cnt;
+                const uint32_t k = k0 + (valid ? ks : 0u);
+                double f[6];
+                chunk_sums(s, pl, partial, k, pl.S == 1 ? move[k] : 0u, valid, f);
+                if (valid && threadIdx.x % L == 0)
+                    for (int y = 0; y < 6; ++y) fs[6 * ks + y] = f[y];
+            }
+            __syncthreads();
+            if (threadIdx.x / 64 * 8 < cnt) {  // (whole waves)
+                const Corr8 ck = corr8_coef(dt1, T, vel);
+                const double f0 = fs[6 * (mine ? kk : 0u) + c], f1 = fs[6 * (mine ? kk : 0u) + 3 + c];
+                double x, ad;
+                const double dtn =
+                    corr8(ck, vel, o0, o1, f0, f1, pr, eta, dt_min, dt_max, x, ad);
+                if (mine && (lane & 3u) < 3u) {
+                    double *col = s.r[0] + i;
+                    col[(q + (vel ? COL_R + 1 : COL_R)) * np] = x;  // (m between r and v)
+                    if (pl.S > 1) col[(q + COL_F) * np] = vel ? f1 : f0;
+                    col[(q + COL_A2) * np] = ad;
+                    if (lane == 0) {
+                        col[COL_T * np] = T;
+                        col[COL_DT * np] = dtn;
+                        tnew[i - b * JT] = T + dtn;
+                    }
+                }
+            }
+        } else {
+            __syncthreads();  // red, tnew and fs of the previous block have been read
+            tnew[threadIdx.x] = NAN;
+            __syncthreads();
+            for (uint32_t base = 0; base < cnt; base += per) {
+                const uint32_t kk = base + threadIdx.x / L;
+                const bool valid = kk < cnt;
+                const uint32_t k = k0 + (valid ? kk : 0u);
+                const uint32_t i = move[k];
+                // the corrector's inputs from the selection's records: their
+                // loads go out with those of the partials
+                double o[6], pr[6], dt1 = 0.0;
+                if (valid) load_arec(e, k, o, pr, dt1);
+                double f[6];
+                chunk_sums(s, pl, partial, k, i, valid, f);
+                if (valid && threadIdx.x % L == 0) {
+                    const double dtn = correct_store(s, i, o, pr, dt1, f, T, eta, dt_min, dt_max);
+                    if (pl.S > 1)
+                        for (int q = 0; q < 6; ++q) s.f[q][i] = f[q];
+                    tnew[i - b * JT] = T + dtn;
+                }
             }
         }
         __syncthreads();
@@ -1634,8 +1779,6 @@ constexpr uint32_t SP = SN / SB;         // particles per thread
 constexpr uint32_t SW = SB / 64;         // waves
 constexpr uint32_t SC = SN / 64;         // chunks of 64 particles
 constexpr uint32_t SMALL_MAX_ACT = 256;  // largest active set k_small_run takes
-// Columns of a context's state from r[0] on (create_impl lays them out).
-constexpr uint32_t COL_R = 0, COL_F = 7, COL_OLD = 13, COL_A2 = 19, COL_T = 25, COL_DT = 26;
 static_assert(SB % JT == 0 && SC == 16, "a row of 16 lanes holds the chunks");
 
 // p (a global-memory pointer), as a value the compiler cannot hoist out of
@@ -1738,53 +1881,6 @@ __device__ __forceinline__ void small_pairs(const double pi[6], uint32_t i, uint
     }
 }
 
-// Sums fo over the wave's lanes with the same slot (lane mod P, P < 64 a
-// power of two) and stores each slot's six sums at its row.  Swapping halves
-// and rows of 16 between two components leaves each half its own three and
-// each row one or two, so the later levels move 2 values instead of 6 (41
-// instructions at P = 1; 156 with all six carried through six levels).
-__device__ __forceinline__ void small_reduce(const double fo[6], uint32_t P, double *row) {
-    const uint32_t lane = __lane_id();
-    double a, b, u[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {  // lower half: components 0..2, upper: 3..5
-        swap_rows<2>(fo[k], fo[3 + k], a, b);
-        u[k] = a + b;
-    }
-    const uint32_t q = lane >= 32 ? 3u : 0u;
-    if (P == 32) {
-        for (int k = 0; k < 3; ++k) row[q + k] = u[k];
-        return;
-    }
-    swap_rows<1>(u[0], u[1], a, b);  // even rows: component q, odd: q + 1
-    double x = a + b;
-    swap_rows<1>(u[2], u[2], a, b);  // both: q + 2
-    double y = a + b;
-    // rotations by 8, 4, 2, 1 inside the rows: lane ^ 8, and so on (uniform
-    // under the larger ones by then)
-    if (P <= 8) {
-        x += dpp<0x128>(x, x);
-        y += dpp<0x128>(y, y);
-    }
-    if (P <= 4) {
-        x += dpp<0x124>(x, x);
-        y += dpp<0x124>(y, y);
-    }
-    if (P <= 2) {
-        x += dpp<0x122>(x, x);
-        y += dpp<0x122>(y, y);
-    }
-    if (P == 1) {
-        x += dpp<0x121>(x, x);
-        y += dpp<0x121>(y, y);
-    }
-    if ((lane & 15u) < P) {
-        const bool odd = (lane & 16u) != 0;
-        row[q + (odd ? 1u : 0u)] = x;
-        if (!odd) row[q + 2] = y;
-    }
-}
-
 // Block steps of systems of n <= SN particles, workgroup c of SB threads for
 // cluster c (a larger cluster's workgroup returns at once), up to max_run
 // steps per launch; clusters are independent, so the workgroups never wait
@@ -1803,7 +1899,7 @@ __device__ __forceinline__ void small_reduce(const double fo[6], uint32_t P, dou
 //
 // Pair sums: P = nact rounded up to a power of two i slots and G groups of
 // lanes; a lane of group g takes one slot and j = g, g + G, ...  P < 64:
-// G = SB / P, a wave's groups summed by halving (small_reduce: neighbouring
+// G = SB / P, a wave's groups summed by halving (slot_sums: neighbouring
 // groups first, so a lane's group is its slot-free bits reversed), the waves'
 // sums in order through LDS.  P >= 64: G = 1024 / P in two passes, one j per
 // wave (an LDS broadcast), summed in group order.  A fixed order for a given
@@ -1975,7 +2071,7 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
             if (P < 64) {
                 const uint32_t g = w * (64 >> lp) + (__brev(lane >> lp) >> (26 + lp));
                 small_pairs<MIXED>(pi, i, g, SB >> lp, n, lpp, lpv, e2, self_zero, fo);
-                small_reduce(fo, P, red + (w * P + slot) * 6);
+                slot_sums(fo, P, red + (w * P + slot) * 6);
             } else {
                 const uint32_t G = SN >> lp;
                 for (uint32_t g = tid >> lp; g < G; g += SB >> lp) {
