@@ -111,6 +111,8 @@ struct RunCtl {
     uint32_t qdone;                // update workgroups done with the work queue
     unsigned long long items;      // update work items this step
     unsigned long long fin_units;  // finish workgroup units this step
+    unsigned long long team_retry; // k_team_run leaves the steps before this one alone
+    uint32_t team_err, pad_;       // 1: a wait inside k_team_run ran out
     unsigned long long qnext;      // update work queue: items claimed beyond the
                                    // first gridDim.x (zero between launches)
 };
@@ -142,6 +144,8 @@ struct Ens {
                              // place in the cluster's active list, count), by step
                              // parity (the step's slot in its captured chunk, mod 2)
     double *bmin;            // [nblk] min(t + dt) per block
+    uint32_t *bcnt;          // [nblk] particles that have it (single system, BCNT_MANY:
+                             // not known)
     double4 *arec;           // [4][nblk * JT] the step's active particles in the order
                              // of the active list (index off[c] + k): predictor
                              // (pp, pv), then old forces and step ((a, dt), (jerk, 0));
@@ -179,11 +183,15 @@ __host__ __device__ inline double dkey_inv(unsigned long long k) {
 // chunk of a narrow group (IW 4 or 16) holds at least 4 tiles, 4K or 16K
 // pairs: shorter items cost more in partial sums than they gain (IW 16),
 // longer ones leave small steps waiting on one item's tile copies (IW 4).
+// (Systems of 5 to TEAM_TILES tiles take one tile per chunk at any width:
+// their small steps are made by one workgroup per tile, k_team_run, with
+// these chunks' sums.)
 // Large active sets of large systems (nact >= 8192 over more than 256
 // tiles) keep chunks of CHUNK_TILES_LARGE tiles: 8 to 32 items per resident
 // workgroup even out the end of the launch, and their finish pass reads
 // whole lines of partials (finish_lanes: 4 lanes per particle); measured at
 // N = 262144, nact 8192 to 32768: 2-5 % less update time.
+constexpr uint32_t TEAM_TILES = 256;  // largest system of k_team_run, in j tiles
 constexpr uint32_t QUEUE_FACTOR = 16;
 constexpr uint32_t CHUNK_TILES = 16;
 constexpr uint32_t CHUNK_TILES_LARGE = 4;
@@ -201,7 +209,7 @@ __host__ __device__ inline Decomp decompose(uint32_t nact, uint32_t iw,
                                             uint32_t max_split) {
     Decomp d;
     d.n_it = (nact + iw - 1) / iw;
-    uint32_t min_tiles = iw >= 64 ? 1u : 4u;
+    uint32_t min_tiles = iw >= 64 || (n_jt > 4 && n_jt <= TEAM_TILES) ? 1u : 4u;
     uint32_t S = 1;
     const uint32_t target = grid * QUEUE_FACTOR;
     if (d.n_it > 0 && d.n_it < target) {

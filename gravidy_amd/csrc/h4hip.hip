@@ -789,7 +789,7 @@ __device__ __forceinline__ uint32_t subgroup(uint32_t t) {
 // Sums fo over the BS/IW j sub-groups of each i slot (thread t of BS): in
 // the wave (slot_sums), then over the waves in order through red.  The fixed
 // tree makes it deterministic.  IW < BS: leaves, after a barrier, sum q of
-// slot k for subgroup_sum; IW = BS: fo already is the slot's.
+// slot k of wave g at red[(g IW + k) 6 + q]; IW = BS: fo already is the slot's.
 template <int IW>
 __device__ __forceinline__ void reduce_subgroups(const double fo[6], double *red, uint32_t t) {
     if constexpr (IW < BS) {
@@ -803,14 +803,6 @@ __device__ __forceinline__ void reduce_subgroups(const double fo[6], double *red
         }
         __syncthreads();
     }
-}
-
-// Sum q of slot k over the waves, in order (IW < BS).
-template <int IW>
-__device__ __forceinline__ double subgroup_sum(const double *red, uint32_t k, uint32_t q) {
-    double acc = red[k * 6 + q];
-    for (uint32_t g = 1; g < BS / 64; ++g) acc += red[(g * IW + k) * 6 + q];
-    return acc;
 }
 
 // FP64_EXACT: the pair terms of Hermite4CPU::update_acc_jrk
@@ -1078,30 +1070,45 @@ __device__ __forceinline__ void update_item(const Soa &s, const ClPlan &pl, uint
         }
     }
     reduce_subgroups<IW>(fo, red, threadIdx.x);
-    constexpr double scale = MIXED ? 1.0 : PAIR_SCALE;  // pair_fp64's 3 sqrt(3)
-    // partial_at(pl, q, sc, k), with the layout's strides
+    if constexpr (IW == BS) {
+        constexpr double scale = MIXED ? 1.0 : PAIR_SCALE;  // pair_fp64's 3 sqrt(3)
+        if (act) {
+            if (pl.S == 1) {
+                const size_t fs = s.f[1] - s.f[0];  // (columns equally spaced)
+                double *fi = s.f[0] + i;
+                for (int q = 0; q < 6; ++q) fi[q * fs] = fo[q] * scale;
+            } else {
+                // partial_at(pl, q, sc, k), with the layout's strides
+                const size_t kst = pl.cmaj ? pl.S : 1u, cst = pl.cmaj ? 1u : pl.rows;
+                double *pq = partial + (size_t)sc * cst + (size_t)k * kst;
+                const size_t qs = (size_t)pl.S * pl.rows;
+                for (int q = 0; q < 6; ++q) pq[q * qs] = fo[q] * scale;
+            }
+        }
+    }
+}
+
+// The sums of an item of less than BS slots, one thread per slot and
+// component (consecutive slots on consecutive threads): the waves' sums in
+// order from red, to f[i] or the item's partials.
+template <bool MIXED>
+__device__ __forceinline__ void store_item(const Soa &s, const ClPlan &pl, uint32_t it, uint32_t sc,
+                                           const uint32_t *mv, uint32_t nact, double *partial,
+                                           const double *red) {
+    constexpr double scale = MIXED ? 1.0 : PAIR_SCALE;
+    const uint32_t iw = pl.iw, lw = 31u - (uint32_t)__clz(iw);
     const size_t kst = pl.cmaj ? pl.S : 1u, cst = pl.cmaj ? 1u : pl.rows;
     const size_t qs = (size_t)pl.S * pl.rows;
-    if constexpr (IW == BS) {
-        if (act) {
-            double *pq = partial + (size_t)sc * cst + (size_t)k * kst;
-            if (pl.S == 1)
-                for (int q = 0; q < 6; ++q) s.f[q][i] = fo[q] * scale;
-            else
-                for (int q = 0; q < 6; ++q) pq[q * qs] = fo[q] * scale;
-        }
-    } else {
-        // one thread per slot and component (consecutive slots on
-        // consecutive threads)
-        for (uint32_t x = threadIdx.x; x < 6 * IW; x += BS) {
-            const uint32_t q = x / IW, sl = x % IW, ks = it * IW + sl;
-            if (ks >= nact) continue;
-            const double f = subgroup_sum<IW>(red, sl, q) * scale;
-            if (pl.S == 1)
-                s.f[0][(size_t)q * (s.f[1] - s.f[0]) + mv[ks]] = f;  // (columns equally spaced)
-            else
-                partial[(size_t)sc * cst + (size_t)ks * kst + q * qs] = f;
-        }
+    for (uint32_t x = threadIdx.x; x < 6 * iw; x += BS) {
+        const uint32_t q = x >> lw, sl = x & (iw - 1), ks = it * iw + sl;
+        if (ks >= nact) continue;
+        double f = red[sl * 6 + q];
+        for (uint32_t g = 1; g < BS / 64; ++g) f += red[(g * iw + sl) * 6 + q];
+        f *= scale;
+        if (pl.S == 1)
+            s.f[0][(size_t)q * (s.f[1] - s.f[0]) + mv[ks]] = f;  // (columns equally spaced)
+        else
+            partial[(size_t)sc * cst + (size_t)ks * kst + q * qs] = f;
     }
 }
 
@@ -1158,6 +1165,7 @@ __device__ __forceinline__ void update_items(const Soa &s, const Ens &e, const u
                                         lA, lB, red);
                 break;
         }
+        if (pl.iw < BS) store_item<MIXED>(s, pl, it, sc, mv, nact, part, red);
         if (total <= gridDim.x) break;
         __syncthreads();  // every lane has read the previous claim
         if (threadIdx.x == 0) claimed = gridDim.x + atomicAdd(&e.ctl->qnext, 1ull);
@@ -1480,6 +1488,31 @@ __device__ __forceinline__ double block_min(double v, double *red) {
     return v;  // valid in thread 0
 }
 
+// Minimum of v over the block and the number of threads that have it (within
+// find_particles_to_move's tolerance; BCNT_MANY if a value within the
+// tolerance of the minimum is not equal to it, which the one-workgroup-per-
+// tile steps leave to the others).  Valid in thread 0.
+constexpr uint32_t BCNT_MANY = 0xffffffu;
+__device__ __forceinline__ double block_min_count(double v, double *red, uint32_t *cnt,
+                                                  uint32_t &n) {
+    const uint32_t w = threadIdx.x >> 6;
+    double m = wave_min(v);
+    const uint32_t at = (uint32_t)__popcll(__ballot(v == m));
+    const bool close = __ballot(v != m && fabs(m - v) < 2 * DBL_EPSILON) != 0;
+    if (__lane_id() == 0) {
+        red[w] = m;
+        cnt[w] = close ? BCNT_MANY : at;
+    }
+    __syncthreads();
+    n = 0;
+    if (threadIdx.x == 0) {
+        for (uint32_t k = 1; k < BS / 64; ++k) m = vmin(m, red[k]);
+        for (uint32_t k = 0; k < BS / 64; ++k)
+            n += red[k] == m ? cnt[k] : fabs(m - red[k]) < 2 * DBL_EPSILON ? BCNT_MANY : 0u;
+    }
+    return m;
+}
+
 // min(t + dt) of one JT block (padding has dt = +inf).
 __device__ __forceinline__ double block_tmin(const Soa &s, uint32_t b, double *red) {
     uint32_t i = b * JT + threadIdx.x;
@@ -1543,6 +1576,7 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
     __shared__ double tnew[JT];  // t + dt of the block's corrected particles (NaN: not active)
     constexpr uint32_t C8 = BS / 8;  // particles of one corr8 pass
     __shared__ double fs[6 * C8];    // their forces
+    __shared__ uint32_t cnts[BS / 64];
     ClState *cs = &e.cs[0];
     const uint32_t *dl = e.dirty + (size_t)par * 3 * e.nblk;
     // What the first block needs is requested at once: the loop's stop
@@ -1647,17 +1681,27 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
         }
         __syncthreads();
         const double tn = tnew[threadIdx.x];
-        const double m = block_min(isnan(tn) ? tdt : tn, red);
-        if (threadIdx.x == 0) e.bmin[b] = m;
+        uint32_t nm;
+        const double m = block_min_count(isnan(tn) ? tdt : tn, red, cnts, nm);
+        if (threadIdx.x == 0) {
+            e.bmin[b] = m;
+            e.bcnt[b] = nm;
+        }
     }
 }
 
 __global__ __launch_bounds__(BS) void k_blockmin_all(Soa s, Ens e) {
     __shared__ double red[BS / 64];
+    __shared__ uint32_t cnts[BS / 64];
     for (uint32_t b = blockIdx.x; b < e.nblk; b += gridDim.x) {
         __syncthreads();
-        double m = block_tmin(s, b, red);
-        if (threadIdx.x == 0) e.bmin[b] = m;
+        const uint32_t i = b * JT + threadIdx.x;
+        uint32_t nm;
+        const double m = block_min_count(s.t[i] + s.dt[i], red, cnts, nm);
+        if (threadIdx.x == 0) {
+            e.bmin[b] = m;
+            e.bcnt[b] = nm;
+        }
     }
 }
 
@@ -1747,17 +1791,19 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
         ctl.max_steps = max_steps;
         ctl.ndirty[0] = ctl.ndirty[1] = 0;
         ctl.ndone = t;
+        ctl.team_retry = 0;
+        ctl.team_err = 0;
         ctl.items = 0;
         ctl.fin_units = 0;
     }
 }
 
 // The loop tail a single system's last block step left (k_finish_blocks),
-// when no further step of the loop makes it: after one h4h_step.
-__global__ __launch_bounds__(BS) void k_tail(Ens e) {
+// when no further step of the loop makes it: after one h4h_step, whose
+// result goes to the pinned record `host`.
+__global__ __launch_bounds__(BS) void k_tail(Ens e, ClState *host) {
     __shared__ double red[BS / 64];
     ClState *cs = &e.cs[0];
-    if (cs->done || !cs->tail_pend) return;
     double mn = INFINITY;
     for (uint32_t b = threadIdx.x; b < e.nblk; b += BS) mn = fmin(mn, e.bmin[b]);
     mn = block_min(mn, red);
@@ -1766,6 +1812,7 @@ __global__ __launch_bounds__(BS) void k_tail(Ens e) {
         record_tail(e, 0, cs->tail_t, cs->tail_nact, steps, mn,
                     loop_stops(*e.ctl, cs->tail_t, steps, mn));
         cs->tail_pend = 0;
+        *host = *cs;
     }
 }
 
@@ -1800,6 +1847,21 @@ __device__ __forceinline__ uint32_t row_sum(uint32_t c) {
     add(__builtin_amdgcn_update_dpp(0, (int)c, DPP_QUADS, 0xf, 0xf, false));
     add(__builtin_amdgcn_update_dpp(0, (int)c, DPP_EIGHTS, 0xf, 0xf, false));
     return c;
+}
+
+// Exclusive prefix sum of c over the wave, and the total.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t c, uint32_t &total) {
+    uint32_t x = c;  // inclusive, in the row of 16 first (row_shr 1, 2, 4, 8)
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);
+    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)x, 15);
+    const uint32_t r1 = r0 + (uint32_t)__builtin_amdgcn_readlane((int)x, 31);
+    const uint32_t r2 = r1 + (uint32_t)__builtin_amdgcn_readlane((int)x, 47);
+    total = r2 + (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+    const uint32_t row = __lane_id() >> 4;
+    return x - c + (row == 0 ? 0u : row == 1 ? r0 : row == 2 ? r1 : r2);
 }
 
 // Number of particles of the workgroup with their flag set (particle
@@ -1881,6 +1943,24 @@ __device__ __forceinline__ void small_pairs(const double pi[6], uint32_t i, uint
     }
 }
 
+// One block step at `itime` without a device loop (h4h_step): the kernels
+// that make whole steps take the loop's state from here instead of the loop
+// control and the cluster record, and write the step's result to the pinned
+// record `host` (its `steps` stays 0 if they leave the step to others), so
+// that such a step is one launch and no copy.
+struct OneStep {
+    double itime;
+    ClState *host;  // null: a device loop
+};
+__device__ __forceinline__ void one_step_result(const OneStep &one, double atime, uint32_t nact,
+                                                uint32_t n, uint32_t small) {
+    one.host->atime = atime;
+    one.host->nsteps = nact;
+    one.host->interactions = (unsigned long long)nact * n;
+    one.host->small_steps = small;
+    one.host->steps = 1;
+}
+
 // Block steps of systems of n <= SN particles, workgroup c of SB threads for
 // cluster c (a larger cluster's workgroup returns at once), up to max_run
 // steps per launch; clusters are independent, so the workgroups never wait
@@ -1923,7 +2003,7 @@ template <bool MIXED>
 __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run,
                                                   uint32_t max_act, double e2, double eta,
                                                   double dt_min, double dt_max,
-                                                  uint32_t self_zero) {
+                                                  uint32_t self_zero, OneStep one) {
 #pragma clang fp contract(off)
     __shared__ double4 lpp[SN], lpv[SN];          // predictor records
     __shared__ __align__(16) double red[6 * SN];  // pair sums per (group, slot)
@@ -1945,13 +2025,15 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     if (n > SN) return;
     const uint32_t off = e.off[c];  // first particle of the cluster
     if (max_act > SMALL_MAX_ACT) max_act = SMALL_MAX_ACT;
-    if (cs->done) return;
-    const double t_end = e.ctl->t_end, t_stop = e.ctl->t_stop;
-    const unsigned long long max_steps = e.ctl->max_steps;
-    unsigned long long steps = cs->steps;
-    unsigned long long inter = cs->interactions, nst = cs->nsteps;
+    const bool loop = one.host == nullptr;
+    if (loop && cs->done) return;
+    const double t_end = loop ? e.ctl->t_end : (double)INFINITY;
+    const double t_stop = loop ? e.ctl->t_stop : -(double)INFINITY;
+    const unsigned long long max_steps = loop ? e.ctl->max_steps : 1ull;
+    unsigned long long steps = loop ? cs->steps : 0ull;
+    unsigned long long inter = loop ? cs->interactions : 0ull, nst = loop ? cs->nsteps : 0ull;
     uint32_t hk = (uint32_t)(steps % e.hist_cap);  // history slot of the next step
-    double T = cs->atime;
+    double T = loop ? cs->atime : one.itime;
     // self_zero (set by the host, self_pair_is_zero): a particle's pair with
     // itself (r = 0, v = 0) has a finite weight m / e2^1.5 for every mass of
     // the context, so it adds exact zeros and the j loop needs no test for it.
@@ -1987,7 +2069,7 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     // first; its next block time is the minimum of t + dt, which these
     // threads hold.  (The dirty lists are cleared for the steps that follow
     // this launch, whose parities need not continue the last step's.)
-    if (cs->tail_pend) {
+    if (loop && cs->tail_pend) {
         const double Tp = cs->tail_t;
         const uint32_t np = cs->tail_nact;
         steps = cs->tail_steps + 1;
@@ -2217,7 +2299,8 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     // Loop state and predictor records of the last step made; per-block
     // minima of t + dt.
     if (it > 0) {
-        if (tid == 0) {
+        if (tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 1);
+        if (tid == 0 && loop) {
             cs->itime = t_last;
             cs->atime = T;
             cs->steps = steps;
@@ -2247,6 +2330,610 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
         for (uint32_t k = 1; k < WPB; ++k) m = fmin(m, wmin[tid * WPB + k]);
         e.bmin[off / JT + tid] = m;
     }
+}
+
+// ---------------------------------------------------------------------------
+// Mid-size systems: whole block steps in one workgroup per j tile or two
+// ---------------------------------------------------------------------------
+
+constexpr uint32_t TB = 2 * BS;         // threads of k_team_run
+constexpr uint32_t TM_ACT = 128;        // largest active set it takes
+constexpr uint32_t TEAM_ONE = 128;      // tiles up to which a workgroup has one (else two)
+constexpr uint32_t TEAM_WGS = TEAM_TILES / 2;
+constexpr uint32_t TEAM_BACKOFF = 64;   // steps left alone after a team did not form
+static_assert(TEAM_ONE <= TEAM_WGS && TEAM_WGS == 128, "workgroups of a team");
+
+// What the workgroups of a team exchange, in device memory.  Every 64-bit
+// word is written and read with agent-scope relaxed atomics (they go past
+// the XCDs' L2s, so no fence is needed: an agent acquire fence per step
+// measured 10 to 35 us) and holds SENT until it is written, so that reading a
+// word is also waiting for it.
+struct Team {
+    uint32_t *sync;             // decision, number of workgroups that have left
+    const uint32_t *plan;       // [TM_ACT + 1]: log2 of the lane-group width | log2 of the
+                                // finish lanes << 16, of the plan for nact (0: not one chunk
+                                // per tile)
+    unsigned long long *hdr;    // [3][workgroups][8]: min(t + dt) of the workgroup's tiles;
+                                // number of particles that have it | first one's index << 32;
+                                // its predicted position and velocity there
+    unsigned long long *rec;    // [3][workgroups][TM_ACT][8]: the others' position, velocity,
+                                // index
+    unsigned long long *part;   // [TM_ACT][6][tiles]: the tiles' partial sums per active particle
+                                // and component (the reader's lanes take consecutive tiles)
+};
+constexpr unsigned long long SENT = 0x7FF4A5A55A5A7E57ull;  // a signalling NaN: no sum's value
+enum : uint32_t { TS_DECISION = 0, TS_LEFT = 32, TS_WORDS = 64 };
+enum : uint32_t { TEAM_GO = 1, TEAM_NO = 2, TEAM_FAILED = 3 };
+
+template <class T>
+__device__ __forceinline__ T agent_load(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void agent_store(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long bits(double x) {
+    return __builtin_bit_cast(unsigned long long, x);
+}
+__device__ __forceinline__ double from_bits(unsigned long long u) {
+    return __builtin_bit_cast(double, u);
+}
+// Stores and loads of this wave so far are done.
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// The word at p once it is written (SENT if it did not come).  Every writer
+// of a formed team is resident, so the wait is short; POLLS (about a second)
+// only bounds it.  Before (decision not null): some 200 us, and no longer
+// than until somebody has given up.
+constexpr uint32_t POLLS = 1u << 20, POLLS_FORM = 256;
+__device__ __forceinline__ unsigned long long wait_word(const unsigned long long *p,
+                                                        const uint32_t *decision) {
+    unsigned long long v = agent_load(p);
+    const uint32_t polls = decision ? POLLS_FORM : POLLS;
+    for (uint32_t k = 1; v == SENT && k < polls; ++k) {
+        v = agent_load(p);
+        if (decision && k % 32 == 0 && agent_load(decision) == TEAM_NO) break;
+    }
+    return v;
+}
+
+// i tile `it` (IW slots, thread t of a group of BS) against a tile in LDS:
+// the work item of the update kernel for one chunk of one tile, the same
+// sums in the same order.  Leaves each wave's sums of the slots in red.
+template <int IW, bool MIXED>
+__device__ __forceinline__ void team_item(uint32_t it, uint32_t t, uint32_t nact, uint32_t j0,
+                                          const double4 *tile, const double *irec,
+                                          const uint32_t *ii, double e2, double *red) {
+    const uint32_t k = it * IW + t % IW, kk = k < nact ? k : 0u;
+    double pi[6];
+    for (int q = 0; q < 6; ++q) pi[q] = irec[6 * kk + q];
+    const uint32_t i = ii[kk], js = subgroup<IW>(t);
+    double fo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (__ballot((i - j0) < (uint32_t)JT))
+        tile_pairs<IW, true, MIXED, 1>(pi, i, j0, js, tile, tile + JT, e2, fo);
+    else
+        tile_pairs<IW, false, MIXED, 1>(pi, i, j0, js, tile, tile + JT, e2, fo);
+    double *row = red + ((it * (BS / 64) + (t >> 6)) * IW + t % IW) * 6;
+    if constexpr (IW < 64)
+        slot_sums(fo, IW, row);
+    else
+        for (int q = 0; q < 6; ++q) row[q] = fo[q];
+}
+
+// Block steps of a single system of 5 to TEAM_TILES j tiles, one workgroup
+// per TPW tiles, up to max_run steps per launch: the device loop's steps with
+// at most TM_ACT active particles whose plan has one chunk per tile, with the
+// same operations in the same order as the selection, update and finish
+// launches, so a step has the same bits whichever makes it.  A step of those
+// is three launches of 5-7 us each at least; here it is two exchanges:
+//
+// (1) every workgroup publishes its tiles' min(t + dt) and the particles that
+//     have it, already predicted to that time; all read all of them, and know
+//     the next block time T and the active particles.
+// (2) every workgroup predicts its particles to T, sums the pairs of the
+//     active particles with them and publishes the sums; the workgroups that
+//     own active particles add the tiles' sums and apply the corrector.
+//
+// What bounds a step is the chain from one next time to the next on a
+// workgroup that owns an active particle, two exchanges of 2-3 us each in it;
+// about 7.5 us at 16 and 40 tiles, 10 us at 256.  Average block steps of runs
+// (start to several hundred steps, all active sets): N = 4096 21.5 -> 12.2 us,
+// 10007 26.0 -> 17.8, 20000 33.0 -> 24.8, 65536 46.0 -> 39.2.  Up to TEAM_ONE
+// tiles a workgroup has one, its two groups of BS threads take turns at the
+// i tiles (N = 20000: 24.8 us, 27.1 with two tiles each); beyond, two, as 256
+// workgroups exchange more slowly than 128.  Steps with more than TM_ACT
+// active particles want the whole chip for their pairs.
+//
+// Buffers: (1) goes round three slots; a workgroup clears its words of the
+// slot before the last exchange when that exchange is complete (then every
+// other one has read them) and before it publishes in the next (which the
+// others wait for before they look at the cleared slot again).  The sums of
+// (2) have one reader each, which clears them before it publishes.  The last
+// workgroup to leave clears the last slot.
+//
+// Nothing here may wait for a workgroup that is not running.  The team forms
+// if the first exchange is complete within a bounded wait: whoever sees it
+// complete sets the decision to GO, whoever does not to NO, and the first
+// setting holds; after GO all are resident until they end.  After NO
+// everybody leaves without having changed anything, and so they do when the
+// next step is not one of theirs: the launches after this one make it.
+template <bool MIXED, uint32_t TPW>
+__global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t max_run,
+                                                 double e2, double eta, double dt_min,
+                                                 double dt_max, OneStep one) {
+#pragma clang fp contract(off)
+    constexpr uint32_t RED = 25 * TM_ACT;  // a tile's sums: 24 doubles per slot of <= 133
+    __shared__ double4 tile[TPW][2 * JT];  // predictor records
+    __shared__ __align__(16) double red[TPW * RED];  // pair sums; then fs, outs
+    __shared__ double hw[8 * TEAM_WGS];    // headers, word by word
+    __shared__ double irec[6 * TM_ACT];    // active particles: position, velocity
+    __shared__ uint32_t ii[TM_ACT], lst[TM_ACT];  // index; workgroup | place in its list << 16
+    __shared__ double stg[7 * TM_ACT];     // own active particles: old forces, step
+    __shared__ uint32_t lact[TM_ACT];      // their threads
+    __shared__ uint32_t plans[TM_ACT + 1];
+    __shared__ double wmn[TB / 64];
+    __shared__ uint32_t wct[TB / 64], s_dec, s_bad;
+    double *fs = red, *outs = red + 6 * TM_ACT;  // (19 per own active particle)
+    constexpr uint32_t NQ = TEAM_WGS / 64;
+    constexpr uint32_t OW = TPW * (BS / 64);  // waves that own particles
+
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid >> 6;
+    const uint32_t b = blockIdx.x, M = gridDim.x, tiles = e.nblk;
+    const uint32_t n = e.cnt[0];
+    const uint32_t i = b * TPW * JT + tid;
+    const bool in = tid < TPW * JT && i < n;
+    // The state's loads go out with those of the check below.
+    double r[3] = {0.0, 0.0, 0.0}, v[3] = {0.0, 0.0, 0.0};
+    double f[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double ti = 0.0, dti = 0.0, tdt = INFINITY;
+    float mf = 0.0f;
+    if (in) {
+        for (int k = 0; k < 3; ++k) {
+            r[k] = s.r[k][i];
+            v[k] = s.v[k][i];
+        }
+        for (int k = 0; k < 6; ++k) f[k] = s.f[k][i];
+        ti = s.t[i];
+        dti = s.dt[i];
+        mf = (float)s.m[i];
+        tdt = ti + dti;
+    }
+    if (tid <= TM_ACT) plans[tid] = tm.plan[tid];
+    ClState *cs = e.cs;
+    RunCtl *ctl = e.ctl;
+    const bool loop = one.host == nullptr, pend = loop && cs->tail_pend != 0;
+    const double Tp = cs->tail_t, atime = loop ? cs->atime : one.itime;
+    const uint32_t np_tail = cs->tail_nact;
+    unsigned long long steps = !loop ? 0ull : pend ? cs->tail_steps + 1 : cs->steps;
+    unsigned long long inter = loop ? cs->interactions : 0ull, nst = loop ? cs->nsteps : 0ull;
+    const double t_end = loop ? ctl->t_end : (double)INFINITY;
+    const double t_stop = loop ? ctl->t_stop : -(double)INFINITY;
+    const unsigned long long max_steps = loop ? ctl->max_steps : 1ull;
+    if (loop && (cs->done || steps < ctl->team_retry)) return;
+    if (pend) {
+        inter += (unsigned long long)np_tail * n;
+        nst += np_tail;
+    }
+    double T;
+    {
+        // Whether the next step is one of a team's, from the block minima.
+        constexpr uint32_t BQ = TEAM_TILES / 64;
+        double x[BQ], m = INFINITY;
+        uint32_t xc[BQ], c = 0;
+        for (uint32_t q = 0; q < BQ; ++q) {
+            const uint32_t k = 64 * q + lane;
+            x[q] = k < tiles ? e.bmin[k] : (double)INFINITY;
+            xc[q] = k < tiles ? e.bcnt[k] : 0u;
+        }
+        for (uint32_t q = 0; q < BQ; ++q) m = vmin(m, x[q]);
+        T = wave_min(m);
+        bool close = false;
+        for (uint32_t q = 0; q < BQ; ++q) {
+            c += x[q] == T ? min(xc[q], BCNT_MANY) : 0u;
+            close |= __ballot(x[q] != T && fabs(T - x[q]) < 2 * DBL_EPSILON) != 0;
+        }
+        c = row_sum(c);
+        const uint32_t nact = (uint32_t)__builtin_amdgcn_readlane((int)c, 0) +
+                              (uint32_t)__builtin_amdgcn_readlane((int)c, 16) +
+                              (uint32_t)__builtin_amdgcn_readlane((int)c, 32) +
+                              (uint32_t)__builtin_amdgcn_readlane((int)c, 48);
+        __syncthreads();  // plans
+        if (close || nact < 1 || nact > TM_ACT || !plans[nact]) return;
+        if (pend ? loop_stops(*ctl, Tp, steps, T) : T != atime) return;
+    }
+
+    bool go = false, stop = false, act = false;
+    uint32_t it = 0, slot = 0, hk = (uint32_t)(steps % e.hist_cap);
+    uint32_t nact = 0, cnt = 0, cnt_before = 0;  // published in this and the last exchange
+    double t_last = 0.0;
+    if (tid == 0) s_bad = 0;
+    // corrector lanes
+    const bool vel = (lane & 4u) != 0;
+    const uint32_t cc = min(lane & 3u, 2u), cq = cc + (vel ? 3u : 0u);
+    double st_o[6], st_a[6];  // of the step before, stored while waiting
+    for (;;) {
+        // (1) The next time of this workgroup's particles, and those that
+        // have it.  (A wave whose minimum is within the selection's tolerance
+        // of the time but not equal to it makes the count BCNT_MANY.)
+        unsigned long long mask = 0;
+        if (w < OW) {
+            const double m = wave_min(tdt);
+            mask = __ballot(in && fabs(m - tdt) < 2 * DBL_EPSILON);
+            if (lane == 0) {
+                wmn[w] = m;
+                wct[w] = (uint32_t)__popcll(mask);
+            }
+        }
+        __syncthreads();
+        double t_own = wmn[0];
+        for (uint32_t k = 1; k < OW; ++k) t_own = vmin(t_own, wmn[k]);
+        cnt_before = cnt;
+        cnt = 0;
+        uint32_t rank = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+        for (uint32_t k = 0; k < OW; ++k) {
+            const uint32_t c = wmn[k] == t_own ? wct[k]
+                               : fabs(t_own - wmn[k]) < 2 * DBL_EPSILON ? BCNT_MANY : 0u;
+            rank += k < w && wmn[k] == t_own ? c : 0u;  // (there always is a rank 0)
+            cnt += c;
+        }
+        const bool cand = w < OW && wmn[w] == t_own && ((mask >> lane) & 1ull);
+        unsigned long long *hd = tm.hdr + ((size_t)slot * M + b) * 8;
+        if (cand && rank < TM_ACT) {
+            double4 pa, pb;
+            predict_vals(r, v, f, t_own - ti, mf, pa, pb);
+            unsigned long long *o =
+                rank ? tm.rec + (((size_t)slot * M + b) * TM_ACT + rank) * 8 : hd + 2;
+            agent_store(o + 0, bits(pa.x));
+            agent_store(o + 1, bits(pa.y));
+            agent_store(o + 2, bits(pa.z));
+            agent_store(o + 3, bits(pb.x));
+            agent_store(o + 4, bits(pb.y));
+            agent_store(o + 5, bits(pb.z));
+            if (rank) {
+                agent_store(o + 6, (unsigned long long)i);
+            } else {
+                agent_store(hd + 1, (unsigned long long)cnt | (unsigned long long)i << 32);
+                agent_store(hd, bits(t_own));
+            }
+        }
+        if (!cnt && tid == 0) {  // (no finite time)
+            for (int k = 1; k < 8; ++k) agent_store(hd + k, 0ull);
+            agent_store(hd, bits((double)INFINITY));
+        }
+        // The step before's state, to HBM while the others publish.
+        if (act) {
+            const size_t np = (size_t)tiles * JT;  // the state's columns are np apart
+            auto *col = in_loop(s.r[0]) + i;
+            for (int k = 0; k < 3; ++k) col[(COL_R + k) * np] = r[k];
+            for (int k = 0; k < 3; ++k) col[(COL_R + 4 + k) * np] = v[k];
+            for (int k = 0; k < 6; ++k) col[(COL_F + k) * np] = f[k];
+            for (int k = 0; k < 6; ++k) col[(COL_OLD + k) * np] = st_o[k];
+            for (int k = 0; k < 6; ++k) col[(COL_A2 + k) * np] = st_a[k];
+            col[COL_T * np] = ti;
+            col[COL_DT * np] = dti;
+        }
+        // All workgroups'.
+        for (uint32_t k = tid; k < 8 * M; k += TB) {
+            const unsigned long long u =
+                wait_word(
+                tm.hdr + (size_t)slot * M * 8 + k, go ? nullptr : tm.sync + TS_DECISION);
+            if (u == SENT) s_bad = 1;
+            hw[k % 8 * TEAM_WGS + k / 8] = from_bits(u);
+        }
+        __syncthreads();
+        if (!go) {
+            if (tid == 0) {
+                const uint32_t want = s_bad ? TEAM_NO : TEAM_GO;
+                const uint32_t d = atomicCAS(&tm.sync[TS_DECISION], 0u, want);
+                s_dec = d ? d : want;
+                // (all were there, though this one's wait ran out: it goes on)
+                if (s_dec == TEAM_GO) s_bad = 0;
+            }
+            __syncthreads();
+            go = s_dec == TEAM_GO;
+            if (!go) break;
+            for (uint32_t k = tid; k < 8 * M; k += TB)
+                if (bits(hw[k % 8 * TEAM_WGS + k / 8]) == SENT) {  // (this wait had missed it)
+                    const unsigned long long u = wait_word(tm.hdr + k, nullptr);
+                    if (u == SENT) s_bad = 1;
+                    hw[k % 8 * TEAM_WGS + k / 8] = from_bits(u);
+                }
+            __syncthreads();
+            if (pend && b == 0 && tid == 0) {
+                record_tail(e, 0, Tp, np_tail, steps, T, false);
+                cs->tail_pend = 0;
+                ctl->ndirty[0] = ctl->ndirty[1] = 0;
+            }
+        }
+        if (s_bad) break;
+        // The next block time, the workgroups that have it, and the places of
+        // their particles in the active list (workgroup by workgroup); every
+        // wave for itself.
+        double x[NQ], m = INFINITY;
+        for (uint32_t q = 0; q < NQ; ++q) {
+            x[q] = 64 * q + lane < M ? hw[64 * q + lane] : (double)INFINITY;
+            m = vmin(m, x[q]);
+        }
+        const double mn = wave_min(m);
+        bool close = false;
+        const uint32_t last_nact = nact;
+        uint32_t place[NQ], c[NQ], heads = 0;
+        nact = 0;
+        for (uint32_t q = 0; q < NQ; ++q) {
+            close |= __ballot(x[q] != mn && fabs(mn - x[q]) < 2 * DBL_EPSILON) != 0;
+            const bool at = x[q] == mn && 64 * q + lane < M;
+            c[q] = at ? (uint32_t)bits(hw[TEAM_WGS + 64 * q + lane]) : 0u;
+            heads += (uint32_t)__popcll(__ballot(c[q] != 0));
+            uint32_t sum;
+            place[q] = nact + wave_scan(c[q], sum);
+            nact += sum;
+        }
+        const uint32_t mine = b < 64 ? (uint32_t)__builtin_amdgcn_readlane((int)c[0], (int)(b & 63))
+                                     : (uint32_t)__builtin_amdgcn_readlane((int)c[NQ - 1], (int)(b & 63));
+        const uint32_t k0 = b < 64
+                                ? (uint32_t)__builtin_amdgcn_readlane((int)place[0], (int)(b & 63))
+                                : (uint32_t)__builtin_amdgcn_readlane((int)place[NQ - 1], (int)(b & 63));
+        static_assert(NQ == 2, "two masks of workgroups");
+        if (it > 0) {
+            // The slot of the exchange before is read by all.
+            const uint32_t prev = slot == 0 ? 2u : slot - 1u;
+            if (tid < 8) agent_store(tm.hdr + ((size_t)prev * M + b) * 8 + tid, SENT);
+            unsigned long long *pr = tm.rec + ((size_t)prev * M + b) * TM_ACT * 8;
+            for (uint32_t k = 8 + tid; k < 8 * min(cnt_before, TM_ACT); k += TB)
+                agent_store(pr + k, SENT);
+            // Loop tail of the step made before this exchange.
+            steps += 1;
+            inter += (unsigned long long)last_nact * n;
+            nst += last_nact;
+            stop = t_last >= t_stop || steps >= max_steps || !(t_last < t_end) || !(mn > t_last);
+            if (b == 0 && tid == 0) {
+                e.hist_t[hk] = t_last;
+                e.hist_n[hk] = last_nact;
+            }
+            if (++hk == e.hist_cap) hk = 0;
+        }
+        T = mn;
+        if (stop || it >= max_run || close || nact < 1 || nact > TM_ACT) break;
+        const uint32_t plan = __builtin_amdgcn_readfirstlane(plans[nact]);
+        if (!plan) break;
+        const uint32_t lw = plan & 0xffffu, iw = 1u << lw, ll = plan >> 16, L = 1u << ll;
+        // (2) The active particles (the last wave: the headers' and the list of
+        // the others), and this workgroup's at T.
+        if (w == TB / 64 - 1)
+            for (uint32_t q = 0; q < NQ; ++q)
+                if (c[q]) {
+                    const double *h = hw + 64 * q + lane;
+                    for (int y = 0; y < 6; ++y) irec[6 * place[q] + y] = h[(2 + y) * TEAM_WGS];
+                    ii[place[q]] = (uint32_t)(bits(h[TEAM_WGS]) >> 32);
+                    for (uint32_t l = 0; l < c[q]; ++l) lst[place[q] + l] = (64 * q + lane) | l << 16;
+                }
+        act = mine && cand;
+        if (tid < TPW * JT) {
+            double4 pa = make_double4(PAD_POS, PAD_POS, PAD_POS, 0.0);
+            double4 pb = make_double4(0.0, 0.0, 0.0, mass_bits(0.0f));
+            if (in) predict_vals(r, v, f, T - ti, mf, pa, pb);
+            tile[tid / JT][tid % JT] = pa;
+            tile[tid / JT][JT + tid % JT] = pb;
+            if (act) {
+                lact[rank] = tid;
+                for (int q = 0; q < 6; ++q) stg[7 * rank + q] = f[q];
+                stg[7 * rank + 6] = dti;
+            }
+        }
+        __syncthreads();
+        if (nact > heads) {
+            const uint32_t l = tid < nact ? lst[tid] >> 16 : 0u;
+            if (l) {
+                const unsigned long long *o =
+                    tm.rec + (((size_t)slot * M + (lst[tid] & 0xffffu)) * TM_ACT + l) * 8;
+                unsigned long long u[7];
+                bool wait = true;
+                for (uint32_t polls = 0; wait && polls < POLLS; ++polls) {
+                    wait = false;
+#pragma unroll
+                    for (int q = 0; q < 7; ++q) u[q] = agent_load(o + q);
+#pragma unroll
+                    for (int q = 0; q < 7; ++q) wait |= u[q] == SENT;
+                }
+                if (wait) s_bad = 1;
+#pragma unroll
+                for (int q = 0; q < 6; ++q) irec[6 * tid + q] = from_bits(u[q]);
+                ii[tid] = (uint32_t)u[6];
+            }
+            __syncthreads();
+        }
+        {
+            const uint32_t grp = tid / BS, t = tid % BS, nit = (nact + iw - 1) >> lw;
+            const uint32_t tl = TPW == 2 ? grp : 0u;
+            const uint32_t j0 = (b * TPW + tl) * JT;
+            for (uint32_t a = TPW == 2 ? 0u : grp; a < nit; a += TPW == 2 ? 1u : 2u) {
+                if (iw == 4)
+                    team_item<4, MIXED>(a, t, nact, j0, tile[tl], irec, ii, e2, red + tl * RED);
+                else if (iw == 16)
+                    team_item<16, MIXED>(a, t, nact, j0, tile[tl], irec, ii, e2, red + tl * RED);
+                else
+                    team_item<64, MIXED>(a, t, nact, j0, tile[tl], irec, ii, e2, red + tl * RED);
+            }
+        }
+        wait_memory();  // the cleared words are clear (before anything is published again)
+        __syncthreads();
+        // The waves' sums in order, as the update's work item adds them.
+        for (uint32_t y = tid; y < TPW * 6 * nact; y += TB) {
+            constexpr double scale = MIXED ? 1.0 : PAIR_SCALE;
+            const uint32_t tl = TPW == 2 && y >= 6 * nact ? 1u : 0u;
+            const uint32_t yy = y - tl * 6 * nact, k = yy / 6, q = yy % 6;
+            if (b * TPW + tl >= tiles) continue;  // (an odd last tile's partner)
+            const uint32_t st = 6 << lw;
+            const double *row =
+                red + tl * RED + (((k >> lw) * (BS / 64) << lw) + (k & (iw - 1))) * 6 + q;
+            double acc = row[0];
+            for (uint32_t g = 1; g < BS / 64; ++g) acc += row[g * st];
+            agent_store(tm.part + (size_t)yy * tiles + b * TPW + tl, bits(acc * scale));
+        }
+        if (mine) {
+            __syncthreads();  // red is read: fs and outs go there
+            // The tiles' sums of this workgroup's active particles, as the
+            // finish pass adds them (chunk_sums): lane sl of L takes tiles sl,
+            // sl + L, ...
+            const uint32_t sl = tid & (L - 1);
+            for (uint32_t base = 0; base < mine; base += TB >> ll) {
+                const uint32_t kk = base + (tid >> ll);
+                const bool valid = kk < mine;
+                double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                if (valid) {
+                    unsigned long long *pk = tm.part + 6 * (size_t)(k0 + kk) * tiles;
+                    constexpr uint32_t U = 4;  // tiles of one wait
+                    for (uint32_t s0 = sl; s0 < tiles; s0 += U * L) {
+                        unsigned long long u[U][6];
+                        bool wait = true;
+                        for (uint32_t polls = 0; wait && polls < POLLS; ++polls) {
+                            wait = false;
+#pragma unroll
+                            for (uint32_t y = 0; y < U; ++y) {
+                                // (past the end: the lane's first tile again)
+                                const uint32_t sc = s0 + y * L < tiles ? s0 + y * L : s0;
+#pragma unroll
+                                for (int q = 0; q < 6; ++q)
+                                    u[y][q] = agent_load(pk + q * tiles + sc);
+                            }
+#pragma unroll
+                            for (uint32_t y = 0; y < U; ++y)
+#pragma unroll
+                                for (int q = 0; q < 6; ++q) wait |= u[y][q] == SENT;
+                        }
+                        if (wait) s_bad = 1;
+#pragma unroll
+                        for (uint32_t y = 0; y < U; ++y)
+                            if (s0 + y * L < tiles) {
+#pragma unroll
+                                for (int q = 0; q < 6; ++q) {
+                                    agent_store(pk + q * tiles + s0 + y * L, SENT);
+                                    acc[q] += from_bits(u[y][q]);
+                                }
+                            }
+                    }
+                }
+                for (int q = 0; q < 6; ++q) acc[q] = lanes_sum(acc[q], L);
+                if (valid && sl == 0)
+                    for (int q = 0; q < 6; ++q) fs[6 * kk + q] = acc[q];
+            }
+            __syncthreads();
+            for (uint32_t p0 = 0; p0 < mine; p0 += TB / 8) {
+                if (p0 + 8 * w >= mine) continue;  // (whole waves)
+                const uint32_t kk = min(p0 + tid / 8, mine - 1);
+                const double *st = stg + 7 * kk, *fk = fs + 6 * kk;
+                const uint32_t la = lact[kk];
+                const double pr = reinterpret_cast<const double *>(
+                    tile[la / JT] + la % JT + (vel ? (uint32_t)JT : 0u))[cc];
+                const Corr8 ck = corr8_coef(st[6], T, vel);
+                const double f0 = fk[cc], f1 = fk[3 + cc];
+                double xn, ad;
+                const double dtn = corr8(ck, vel, st[cc], st[3 + cc], f0, f1, pr, eta, dt_min,
+                                         dt_max, xn, ad);
+                if (p0 + tid / 8 < mine && (lane & 3u) < 3u) {
+                    double *o = outs + 19 * kk;
+                    o[cq] = vel ? f1 : f0;
+                    o[6 + cq] = xn;
+                    o[13 + cq] = ad;
+                    if ((lane & 7u) == 0) o[12] = dtn;
+                }
+            }
+            wait_memory();  // the cleared sums are clear
+            __syncthreads();
+            if (act) {
+                const double *o = outs + 19 * rank;
+                for (int q = 0; q < 6; ++q) {
+                    st_o[q] = f[q];
+                    f[q] = o[q];
+                    st_a[q] = o[13 + q];
+                }
+                for (int q = 0; q < 3; ++q) {
+                    r[q] = o[6 + q];
+                    v[q] = o[9 + q];
+                }
+                ti = T;
+                dti = o[12];
+                tdt = ti + dti;
+            }
+        }
+        t_last = T;
+        ++it;
+        slot = slot == 2 ? 0u : slot + 1u;
+    }
+    // Loop state, predictor records of the last step, block minima.
+    if (it > 0) {
+        if (b == 0 && tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 0);
+        if (b == 0 && tid == 0 && loop) {
+            cs->itime = t_last;
+            cs->atime = T;
+            cs->steps = steps;
+            cs->interactions = inter;
+            cs->nsteps = nst;
+            if (stop) {
+                cs->done = 1;
+                atomicAdd(&ctl->ndone, 1u);
+            }
+        }
+        if (in) {
+            s.pp[i] = tile[tid / JT][tid % JT];
+            s.pv[i] = tile[tid / JT][JT + tid % JT];
+        }
+        // (block_min_count's, tile by tile)
+        double m = INFINITY;
+        if (w < OW) {
+            m = wave_min(tdt);
+            const bool near = __ballot(tdt != m && fabs(m - tdt) < 2 * DBL_EPSILON) != 0;
+            const uint32_t at = (uint32_t)__popcll(__ballot(tdt == m));
+            if (lane == 0) {
+                wmn[w] = m;
+                wct[w] = near ? BCNT_MANY : at;
+            }
+        }
+        __syncthreads();
+        if (tid < TPW && b * TPW + tid < tiles) {
+            const uint32_t w0 = tid * (BS / 64);
+            uint32_t at = 0;
+            m = wmn[w0];
+            for (uint32_t k = 1; k < BS / 64; ++k) m = vmin(m, wmn[w0 + k]);
+            for (uint32_t k = 0; k < BS / 64; ++k)
+                at += wmn[w0 + k] == m ? wct[w0 + k]
+                      : fabs(m - wmn[w0 + k]) < 2 * DBL_EPSILON ? BCNT_MANY : 0u;
+            e.bmin[b * TPW + tid] = m;
+            e.bcnt[b * TPW + tid] = at;
+        }
+    }
+    // This workgroup's further records of the last exchange (nobody reads
+    // them), and its header if no team formed.
+    unsigned long long *rc = tm.rec + ((size_t)slot * M + b) * TM_ACT * 8;
+    for (uint32_t k = 8 + tid; k < 8 * min(cnt, TM_ACT); k += TB) agent_store(rc + k, SENT);
+    if (!go && tid < 8) agent_store(tm.hdr + (size_t)b * 8 + tid, SENT);
+    if (go && s_bad && tid == 0) {
+        ctl->team_err = 1;
+        if (!loop) one.host->done = TEAM_FAILED;
+    }
+    wait_memory();
+    __syncthreads();
+    if (tid == 0) s_dec = atomicAdd(&tm.sync[TS_LEFT], 1u) == M - 1;
+    __syncthreads();
+    if (!s_dec) return;
+    // The last one out.
+    if (go)
+        for (uint32_t k = tid; k < 8 * M; k += TB)
+            agent_store(tm.hdr + (size_t)slot * M * 8 + k, SENT);
+    else if (tid == 0)
+        ctl->team_retry = steps + TEAM_BACKOFF;
+    if (tid == 0) {
+        agent_store(&tm.sync[TS_DECISION], 0u);
+        agent_store(&tm.sync[TS_LEFT], 0u);
+    }
+}
+
+// Every word of a team's buffers waiting (context creation).
+__global__ __launch_bounds__(BS) void k_team_clear(Team tm, size_t words) {
+    for (size_t k = blockIdx.x * (size_t)BS + threadIdx.x; k < words; k += (size_t)gridDim.x * BS)
+        tm.hdr[k] = SENT;
+    if (blockIdx.x == 0 && threadIdx.x < TS_WORDS) tm.sync[threadIdx.x] = 0;
 }
 
 // Single-cluster ABI helpers.
@@ -2473,6 +3160,7 @@ struct h4h_ctx {
     double mass_max = 0.0;   // largest |float mass| of the uploaded state (+inf: not finite)
 
     hipStream_t stream = nullptr;
+    char *arena = nullptr;       // device memory of all the pointers below but partial
     double *state = nullptr;     // all SoA arrays
     double *staging = nullptr;   // n * 8 doubles
     double *partial = nullptr;   // j-split partials
@@ -2480,12 +3168,14 @@ struct h4h_ctx {
     uint32_t *move = nullptr;
     // cluster tables
     uint32_t *d_off = nullptr, *d_cnt = nullptr, *d_hoff = nullptr, *d_bcl = nullptr;
-    ClState *d_cs = nullptr;
+    ClState *d_cs = nullptr;  // behind d_ctl
     ClPlan *d_plan = nullptr;
     unsigned long long *d_pre = nullptr;  // items_pre | fin_pre | part_pre
     RunCtl *d_ctl = nullptr;
     uint32_t *d_dirty = nullptr;
-    double *d_bmin = nullptr;
+    double *d_bmin = nullptr;    // [nblk], then u32 x nblk counts
+    Team team{};                 // exchange buffers of k_team_run (behind d_arec)
+    bool team_ok = false;        // the system has a team's number of tiles
     double4 *d_arec = nullptr;   // the step's active particles' records (Ens::arec)
     uint32_t *d_tune = nullptr;  // [64] tuning table
     double *hist_t = nullptr;
@@ -2497,6 +3187,7 @@ struct h4h_ctx {
     ClState *cs_host = nullptr;
     double *hist_t_host = nullptr;
     uint32_t *hist_n_host = nullptr;
+    uint32_t *team_plan_host = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool graphs = true;          // device loops replay captured chunks
@@ -2548,6 +3239,30 @@ void drop_graph(h4h_ctx *ctx) {
     ctx->graph = nullptr;
 }
 
+// A single system of 5 to TEAM_TILES j tiles makes its small steps in
+// k_team_run.  Fewer tiles: k_small_run, whose one workgroup needs no
+// exchange.  More: a tile per workgroup would not leave every workgroup a CU.
+bool team_size(const h4h_ctx *ctx) { return ctx->K == 1 && ctx->nblk > 4 && ctx->nblk <= TEAM_TILES; }
+
+// The plans of the active counts a team takes (0: not one chunk per tile,
+// or a tuning table is set).
+int configure_team(h4h_ctx *ctx) {
+    if (!ctx->team_ok) return H4H_OK;
+    for (uint32_t k = 0; k <= TM_ACT; ++k) {
+        uint32_t plan = 0;
+        if (k >= 1 && k <= ctx->n && !ctx->e.tuned) {
+            const uint32_t iw = pick_iw(k, ctx->iw_fill);
+            const Decomp d = decompose(k, iw, ctx->nblk, ctx->e.grid, ctx->max_split);
+            if (iw <= 64 && d.S == ctx->nblk)
+                plan = (uint32_t)__builtin_ctz(iw) | (uint32_t)__builtin_ctz(finish_lanes(d.S, k)) << 16;
+        }
+        ctx->team_plan_host[k] = plan;
+    }
+    H4H_HIP(hipMemcpyAsync(const_cast<uint32_t *>(ctx->team.plan), ctx->team_plan_host,
+                           (TM_ACT + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+    return H4H_OK;
+}
+
 // (Re)sizes the j-split partials for the current grid and updates the
 // launch fields of the cluster table.
 int configure_launch(h4h_ctx *ctx) {
@@ -2560,6 +3275,8 @@ int configure_launch(h4h_ctx *ctx) {
     ctx->e.max_split = ctx->max_split;
     ctx->e.iw_fill = ctx->iw_fill;
     drop_graph(ctx);
+    int rc = configure_team(ctx);
+    if (rc) return rc;
     // j-split partials for any plan of any step (partial_bound).
     size_t need;
     if (ctx->K == 1) {
@@ -2660,13 +3377,37 @@ bool self_pair_is_zero(int precision, double e2, double mmax) {
 }
 
 // One workgroup per cluster.
-int launch_small(h4h_ctx *ctx, uint32_t max_run) {
+int launch_small(h4h_ctx *ctx, uint32_t max_run, OneStep one = {}) {
     auto *kern = ctx->precision == H4H_MIXED ? k_small_run<true> : k_small_run<false>;
     hipLaunchKernelGGL(kern, dim3(ctx->K), dim3(SB), 0, ctx->stream, ctx->s, ctx->e, max_run,
                        ctx->small_act, ctx->e2, (double)ctx->eta, ctx->dt_min, ctx->dt_max,
-                       self_pair_is_zero(ctx->precision, ctx->e2, ctx->mass_max) ? 1u : 0u);
+                       self_pair_is_zero(ctx->precision, ctx->e2, ctx->mass_max) ? 1u : 0u, one);
     H4H_LAUNCHED();
     return H4H_OK;
+}
+
+bool team_path(const h4h_ctx *ctx) {
+    return ctx->team_ok && !ctx->e.tuned && ctx->precision != H4H_FP64_EXACT;
+}
+
+int launch_team(h4h_ctx *ctx, uint32_t max_run, OneStep one = {}) {
+    const bool two = ctx->nblk > TEAM_ONE, mixed = ctx->precision == H4H_MIXED;
+    auto *kern = two ? (mixed ? k_team_run<true, 2> : k_team_run<false, 2>)
+                     : (mixed ? k_team_run<true, 1> : k_team_run<false, 1>);
+    hipLaunchKernelGGL(kern, dim3(two ? (ctx->nblk + 1) / 2 : ctx->nblk), dim3(TB), 0, ctx->stream,
+                       ctx->s, ctx->e, ctx->team, max_run, ctx->e2, (double)ctx->eta, ctx->dt_min,
+                       ctx->dt_max, one);
+    H4H_LAUNCHED();
+    return H4H_OK;
+}
+
+// After a loop's (or one step's) state is read back: whether a wait inside a
+// team ran out (the state is then between two steps).
+int check_team(h4h_ctx *ctx, bool failed) {
+    if (!failed) return H4H_OK;
+    ctx->team_ok = false;
+    drop_graph(ctx);
+    return fail(H4H_EHIP, "a wait between workgroups ran out; upload the state again");
 }
 
 int ensure_blockmin(h4h_ctx *ctx) {
@@ -2714,15 +3455,17 @@ int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par) {
     return H4H_OK;
 }
 
-// One chunk of the device loop: RUN_CHUNK block steps, or for a small
-// system SMALL_SLOTS slots of k_small_run (up to SMALL_RUN steps with small
-// active sets) followed by one block step of the multi-workgroup kernels
-// (the step k_small_run left, if any).  At most HIST_CAP steps.
+// One chunk of the device loop: RUN_CHUNK block steps, or for a small or
+// mid-size system SMALL_SLOTS slots of k_small_run or k_team_run (up to
+// SMALL_RUN steps with small active sets) followed by one block step of the
+// multi-workgroup kernels (the step it left, if any).  At most HIST_CAP steps.
 int enqueue_chunk(h4h_ctx *ctx) {
     int rc = H4H_OK;
-    if (small_path(ctx)) {
-        for (uint32_t k = 0; k < SMALL_SLOTS && rc == H4H_OK; ++k)
-            if ((rc = launch_small(ctx, SMALL_RUN)) == H4H_OK) rc = enqueue_step(ctx, false, k & 1);
+    if (small_path(ctx) || team_path(ctx)) {
+        for (uint32_t k = 0; k < SMALL_SLOTS && rc == H4H_OK; ++k) {
+            rc = small_path(ctx) ? launch_small(ctx, SMALL_RUN) : launch_team(ctx, SMALL_RUN);
+            if (rc == H4H_OK) rc = enqueue_step(ctx, false, k & 1);
+        }
     } else {
         for (uint32_t k = 0; k < RUN_CHUNK && rc == H4H_OK; ++k) rc = enqueue_step(ctx, false, k & 1);
     }
@@ -2748,10 +3491,10 @@ int ensure_graph(h4h_ctx *ctx) {
     return H4H_OK;
 }
 
+// (The loop control and the cluster states are neighbours, on the device and
+// in the pinned mirror: one copy.)
 int read_state(h4h_ctx *ctx) {
-    H4H_HIP(hipMemcpyAsync(ctx->ctl_host, ctx->d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost,
-                           ctx->stream));
-    H4H_HIP(hipMemcpyAsync(ctx->cs_host, ctx->d_cs, ctx->K * sizeof(ClState),
+    H4H_HIP(hipMemcpyAsync(ctx->ctl_host, ctx->d_ctl, sizeof(RunCtl) + ctx->K * sizeof(ClState),
                            hipMemcpyDeviceToHost, ctx->stream));
     H4H_HIP(hipStreamSynchronize(ctx->stream));
     return H4H_OK;
@@ -2816,7 +3559,9 @@ bool valid_precision(int p) { return p == H4H_FP64 || p == H4H_FP64_EXACT || p =
 
 // Workgroup sums the energy buffer of a context holds: one system's, or
 // ENERGY_OUT for an ensemble.
-size_t eout_len(const h4h_ctx *ctx) { return ctx->K > 1 ? ENERGY_OUT : ENERGY_GRID; }
+size_t eout_len(const h4h_ctx *ctx) {
+    return ctx->K > 1 ? ENERGY_OUT : energy_items(ctx->cnt[0]).wgs;
+}
 
 // Energies of clusters c0 .. c0 + count - 1, in launches of as many
 // clusters as fit the sums of eout (64 clusters of 1024 to 32768 particles:
@@ -2926,28 +3671,57 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
         return cleanup(fail(H4H_EHIP, "hipStreamCreate failed"));
     size_t np = ctx->n_dev;
-    bool ok = hipMalloc(&ctx->state, np * N_SOA * sizeof(double)) == hipSuccess &&
-              hipMalloc(&ctx->staging, (size_t)ctx->n * 8 * sizeof(double)) == hipSuccess &&
-              hipMalloc(&ctx->move, np * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->d_off, K * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->d_cnt, K * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->d_hoff, K * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->d_bcl, ctx->nblk * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->d_cs, K * sizeof(ClState)) == hipSuccess &&
-              hipMalloc(&ctx->d_plan, K * sizeof(ClPlan)) == hipSuccess &&
-              hipMalloc(&ctx->d_pre, 3 * (size_t)(K + 1) * sizeof(unsigned long long)) == hipSuccess &&
-              hipMalloc(&ctx->d_ctl, sizeof(RunCtl)) == hipSuccess &&
-              hipMalloc(&ctx->d_dirty, 6 * (size_t)ctx->nblk * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->d_bmin, ctx->nblk * sizeof(double)) == hipSuccess &&
-              hipMalloc(&ctx->d_arec, 4 * np * sizeof(double4)) == hipSuccess &&
-              hipMalloc(&ctx->d_tune, 64 * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&ctx->hist_t, HIST_CAP * sizeof(double)) == hipSuccess &&
-              hipMalloc(&ctx->hist_n, HIST_CAP * sizeof(uint32_t)) == hipSuccess;
-    if (!ok) return cleanup(fail(H4H_ENOMEM, "device allocation failed"));
+    ctx->team_ok = team_size(ctx);
+    const size_t tm_hdr = 3 * (size_t)ctx->nblk * 8,
+                 tm_rec = 3 * (size_t)ctx->nblk * 8 * TM_ACT,
+                 tm_part = (size_t)ctx->nblk * TM_ACT * 6, tm_words = tm_hdr + tm_rec + tm_part,
+                 tm_plan = TS_WORDS + TM_ACT + 2;  // u32
+    const size_t team_bytes =
+        ctx->team_ok ? tm_words * sizeof(double) + tm_plan * sizeof(uint32_t) : 0;
+    // One device allocation for everything but the partials (17 of them took
+    // half of the time of a small context's creation); what starts at zero is
+    // at its front, the four cluster tables are neighbours.
+    struct Piece {
+        void **p;
+        size_t bytes;
+    };
+    const size_t tables = 3 * (size_t)K + ctx->nblk;
+    const Piece pieces[] = {
+        {(void **)&ctx->d_ctl, sizeof(RunCtl) + K * sizeof(ClState)},
+        {(void **)&ctx->d_tune, 64 * sizeof(uint32_t)},
+        {(void **)&ctx->d_pre, 3 * (size_t)(K + 1) * sizeof(unsigned long long)},
+        {(void **)&ctx->state, np * N_SOA * sizeof(double)},
+        {(void **)&ctx->staging, (size_t)ctx->n * 8 * sizeof(double)},
+        {(void **)&ctx->move, np * sizeof(uint32_t)},
+        {(void **)&ctx->d_off, tables * sizeof(uint32_t)},
+        {(void **)&ctx->d_plan, K * sizeof(ClPlan)},
+        {(void **)&ctx->d_dirty, 6 * (size_t)ctx->nblk * sizeof(uint32_t)},
+        {(void **)&ctx->d_bmin, ctx->nblk * (sizeof(double) + sizeof(uint32_t))},
+        {(void **)&ctx->d_arec, 4 * np * sizeof(double4) + team_bytes},
+        {(void **)&ctx->hist_t, HIST_CAP * sizeof(double)},
+        {(void **)&ctx->hist_n, HIST_CAP * sizeof(uint32_t)},
+    };
+    size_t bytes = 0, zeroed = 0;
+    for (const Piece &x : pieces) {
+        bytes += (x.bytes + 255) / 256 * 256;
+        if (x.p == (void **)&ctx->state) zeroed = bytes;
+    }
+    if (hipMalloc(&ctx->arena, bytes) != hipSuccess)
+        return cleanup(fail(H4H_ENOMEM, "device allocation failed"));
+    bytes = 0;
+    for (const Piece &x : pieces) {
+        *x.p = ctx->arena + bytes;
+        bytes += (x.bytes + 255) / 256 * 256;
+    }
+    ctx->d_cnt = ctx->d_off + K;
+    ctx->d_hoff = ctx->d_cnt + K;
+    ctx->d_bcl = ctx->d_hoff + K;
+    ctx->d_cs = reinterpret_cast<ClState *>(ctx->d_ctl + 1);
     // One pinned allocation for all host mirrors (each costs ~0.2 ms).
     static_assert(sizeof(RunCtl) % 8 == 0 && sizeof(ClState) % 8 == 0, "carved in doubles");
     const size_t eo = eout_len(ctx) * 4, ct = sizeof(RunCtl) / 8, cst = K * sizeof(ClState) / 8;
-    if (hipHostMalloc(&ctx->pinned, (eo + ct + cst + HIST_CAP + HIST_CAP / 2) * sizeof(double),
+    const size_t pl = TM_ACT / 2 + 1;
+    if (hipHostMalloc(&ctx->pinned, (eo + ct + cst + HIST_CAP + HIST_CAP / 2 + pl) * sizeof(double),
                       hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(H4H_ENOMEM, "pinned allocation failed"));
     ctx->eout = ctx->pinned;
@@ -2955,9 +3729,18 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     ctx->cs_host = reinterpret_cast<ClState *>(ctx->eout + eo + ct);
     ctx->hist_t_host = ctx->eout + eo + ct + cst;
     ctx->hist_n_host = reinterpret_cast<uint32_t *>(ctx->hist_t_host + HIST_CAP);
+    ctx->team_plan_host = ctx->hist_n_host + HIST_CAP;
     for (int k = 0; k < 4; ++k)
         if (hipEventCreate(&ctx->ev[k]) != hipSuccess)
             return cleanup(fail(H4H_EHIP, "hipEventCreate failed"));
+    std::vector<uint32_t> tab(ctx->off);
+    tab.insert(tab.end(), ctx->cnt.begin(), ctx->cnt.end());
+    tab.insert(tab.end(), ctx->hoff.begin(), ctx->hoff.end());
+    tab.insert(tab.end(), bcl.begin(), bcl.end());
+    bool ok = hipMemcpyAsync(ctx->d_off, tab.data(), tables * sizeof(uint32_t),
+                             hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
+              hipMemsetAsync(ctx->arena, 0, zeroed, ctx->stream) == hipSuccess;
+    if (!ok) return cleanup(fail(H4H_EHIP, "initialisation failed"));
 
     Ens &e = ctx->e;
     e.K = K;
@@ -2974,12 +3757,24 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     e.ctl = ctx->d_ctl;
     e.dirty = ctx->d_dirty;
     e.bmin = ctx->d_bmin;
+    e.bcnt = reinterpret_cast<uint32_t *>(ctx->d_bmin + ctx->nblk);
     e.arec = ctx->d_arec;
     e.hist_t = ctx->hist_t;
     e.hist_n = ctx->hist_n;
     e.hist_cap = HIST_CAP;
     e.tuned = 0;
     e.tune = ctx->d_tune;
+    if (ctx->team_ok) {
+        unsigned long long *tb = reinterpret_cast<unsigned long long *>(ctx->d_arec + 4 * np);
+        Team &tm = ctx->team;
+        tm.hdr = tb;
+        tm.rec = tb + tm_hdr;
+        tm.part = tb + tm_hdr + tm_rec;
+        tm.sync = reinterpret_cast<uint32_t *>(tb + tm_words);
+        tm.plan = tm.sync + TS_WORDS;
+        hipLaunchKernelGGL(k_team_clear, dim3(256), dim3(BS), 0, ctx->stream, tm, tm_words);
+        if (hipGetLastError() != hipSuccess) return cleanup(fail(H4H_EHIP, "kernel launch"));
+    }
     int rc = configure_launch(ctx);
     if (rc) return cleanup(rc);
     ctx->small_ok = small_fits(ctx->device);
@@ -3012,16 +3807,7 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
         s.a2[0] != s.r[0] + COL_A2 * np || s.a3[0] != s.a2[0] + 3 * np ||
         s.t != s.r[0] + COL_T * np || s.dt != s.r[0] + COL_DT * np)
         return cleanup(fail(H4H_EINVAL, "state layout"));
-    ok = hipMemcpyAsync(ctx->d_off, ctx->off.data(), K * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
-         hipMemcpyAsync(ctx->d_cnt, ctx->cnt.data(), K * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
-         hipMemcpyAsync(ctx->d_hoff, ctx->hoff.data(), K * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
-         hipMemcpyAsync(ctx->d_bcl, bcl.data(), ctx->nblk * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
-         hipMemsetAsync(ctx->state, 0, np * N_SOA * sizeof(double), ctx->stream) == hipSuccess &&
-         hipMemsetAsync(ctx->d_cs, 0, K * sizeof(ClState), ctx->stream) == hipSuccess &&
-         hipMemsetAsync(ctx->d_ctl, 0, sizeof(RunCtl), ctx->stream) == hipSuccess &&
-         hipMemsetAsync(ctx->d_tune, 0, 64 * sizeof(uint32_t), ctx->stream) == hipSuccess &&
-         hipMemsetAsync(ctx->d_pre, 0, 3 * (size_t)(K + 1) * sizeof(unsigned long long), ctx->stream) == hipSuccess &&
-         hipStreamSynchronize(ctx->stream) == hipSuccess;
+    ok = hipStreamSynchronize(ctx->stream) == hipSuccess;
     if (!ok) return cleanup(fail(H4H_EHIP, "initialisation failed"));
     *out = ctx;
     return H4H_OK;
@@ -3184,11 +3970,7 @@ int h4h_destroy(h4h_ctx *ctx) {
     drop_graph(ctx);
     for (int k = 0; k < 4; ++k)
         if (ctx->ev[k]) (void)hipEventDestroy(ctx->ev[k]);
-    void *dev[] = {ctx->state, ctx->staging, ctx->partial, ctx->move, ctx->d_off,
-                   ctx->d_cnt, ctx->d_hoff, ctx->d_bcl, ctx->d_cs, ctx->d_plan, ctx->d_pre,
-                   ctx->d_ctl, ctx->d_dirty, ctx->d_bmin, ctx->d_arec, ctx->d_tune, ctx->hist_t,
-                   ctx->hist_n};
-    for (void *p : dev)
+    for (void *p : {(void *)ctx->arena, (void *)ctx->partial})
         if (p) (void)hipFree(p);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -3497,17 +4279,29 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     if (rc) return rc;
     if ((rc = ensure_blockmin(ctx))) return rc;
     if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
-    // One-step loop: ATIME = itime, stop after the step.
-    hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, (double)INFINITY,
-                       -INFINITY, 1ull, 1u, -INFINITY, itime);
-    H4H_LAUNCHED();
-    // The step the device loop would make: k_small_run when it takes it.
-    if (small_path(ctx) && (rc = launch_small(ctx, 1))) return rc;
-    if ((rc = enqueue_step(ctx, ctx->timing, 0))) return rc;
-    hipLaunchKernelGGL(k_tail, dim3(1), dim3(BS), 0, ctx->stream, ctx->e);
-    H4H_LAUNCHED();
-    if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
-    if ((rc = read_state(ctx))) return rc;
+    // The step the device loop would make: k_small_run or k_team_run when they
+    // take it, which the host looks at before it launches the others (most
+    // steps are theirs, and the launches cost more than a look).
+    ctx->cs_host[0] = ClState{};
+    if (small_path(ctx) || team_path(ctx)) {
+        const OneStep one{itime, ctx->cs_host};
+        if ((rc = small_path(ctx) ? launch_small(ctx, 1, one) : launch_team(ctx, 1, one))) return rc;
+        if (ctx->timing)
+            for (int k : {0, 1, 3}) H4H_HIP(hipEventRecord(ctx->ev[k], ctx->stream));
+        H4H_HIP(hipStreamSynchronize(ctx->stream));
+        if ((rc = check_team(ctx, ctx->cs_host[0].done == TEAM_FAILED))) return rc;
+    }
+    if (!ctx->cs_host[0].steps) {
+        // One-step loop: ATIME = itime, stop after the step.
+        hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, (double)INFINITY,
+                           -INFINITY, 1ull, 1u, -INFINITY, itime);
+        H4H_LAUNCHED();
+        if ((rc = enqueue_step(ctx, ctx->timing, 0))) return rc;
+        hipLaunchKernelGGL(k_tail, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, ctx->cs_host);
+        H4H_LAUNCHED();
+        if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
+        H4H_HIP(hipStreamSynchronize(ctx->stream));
+    }
     if (ctx->timing) {
         float ms = 0.f;
         H4H_HIP(hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[3]));
@@ -3542,10 +4336,8 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
         } else if ((rc = enqueue_chunk(ctx))) {
             return rc;
         }
-        H4H_HIP(hipMemcpyAsync(ctx->ctl_host, ctx->d_ctl, sizeof(RunCtl), hipMemcpyDeviceToHost,
-                               ctx->stream));
-        H4H_HIP(hipMemcpyAsync(ctx->cs_host, ctx->d_cs, sizeof(ClState), hipMemcpyDeviceToHost,
-                               ctx->stream));
+        H4H_HIP(hipMemcpyAsync(ctx->ctl_host, ctx->d_ctl, sizeof(RunCtl) + sizeof(ClState),
+                               hipMemcpyDeviceToHost, ctx->stream));
         if (hist) {
             H4H_HIP(hipMemcpyAsync(ctx->hist_t_host, ctx->hist_t, HIST_CAP * sizeof(double),
                                    hipMemcpyDeviceToHost, ctx->stream));
@@ -3553,6 +4345,7 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
                                    hipMemcpyDeviceToHost, ctx->stream));
         }
         H4H_HIP(hipStreamSynchronize(ctx->stream));
+        if ((rc = check_team(ctx, ctx->ctl_host->team_err != 0))) return rc;
         if (hist) {
             uint64_t steps = ctx->cs_host[0].steps;
             for (uint64_t k = seen; k < steps && k < cap; ++k) {
@@ -3689,7 +4482,7 @@ int h4h_set_tuning(h4h_ctx *ctx, const uint32_t *grid32, const uint32_t *iw32) {
     H4H_HIP(hipStreamSynchronize(ctx->stream));
     ctx->e.tuned = (grid32 || iw32) ? 1u : 0u;
     drop_graph(ctx);
-    return H4H_OK;
+    return configure_team(ctx);
 }
 
 // Measures the update kernel for nact = 2^b (b = 0 .. log2 n, plus n) with
