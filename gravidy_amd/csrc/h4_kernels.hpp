@@ -83,6 +83,7 @@ struct ClPlan {
     uint32_t lanes;     // finish lanes per particle (finish_lanes(S, nact))
     uint32_t grid;      // workgroup share given to decompose()
     uint32_t cmaj;      // 1: partials chunk-major (partial_at)
+    uint32_t jrun;      // 1: a j sub-group takes consecutive j (lane_group)
 };
 
 // Place of the j-chunk partial sum of component q, chunk sc, active
@@ -185,13 +186,15 @@ __host__ __device__ inline double dkey_inv(unsigned long long k) {
 // longer ones leave small steps waiting on one item's tile copies (IW 4).
 // (Systems of 5 to TEAM_TILES tiles take one tile per chunk at any width:
 // their small steps are made by one workgroup per tile, k_team_run, with
-// these chunks' sums.)
+// these chunks' sums; so do the larger steps, nact > NARROW_ACT, of all
+// systems of up to TEAM_TILES tiles.)
 // Large active sets of large systems (nact >= 8192 over more than 256
 // tiles) keep chunks of CHUNK_TILES_LARGE tiles: 8 to 32 items per resident
 // workgroup even out the end of the launch, and their finish pass reads
 // whole lines of partials (finish_lanes: 4 lanes per particle); measured at
 // N = 262144, nact 8192 to 32768: 2-5 % less update time.
 constexpr uint32_t TEAM_TILES = 256;  // largest system of k_team_run, in j tiles
+constexpr uint32_t NARROW_ACT = 128;  // largest nact that lane_group does not narrow
 constexpr uint32_t QUEUE_FACTOR = 16;
 constexpr uint32_t CHUNK_TILES = 16;
 constexpr uint32_t CHUNK_TILES_LARGE = 4;
@@ -209,7 +212,7 @@ __host__ __device__ inline Decomp decompose(uint32_t nact, uint32_t iw,
                                             uint32_t max_split) {
     Decomp d;
     d.n_it = (nact + iw - 1) / iw;
-    uint32_t min_tiles = iw >= 64 || (n_jt > 4 && n_jt <= TEAM_TILES) ? 1u : 4u;
+    uint32_t min_tiles = iw >= 64 || (n_jt <= TEAM_TILES && (n_jt > 4 || nact > NARROW_ACT)) ? 1u : 4u;
     uint32_t S = 1;
     const uint32_t target = grid * QUEUE_FACTOR;
     if (d.n_it > 0 && d.n_it < target) {
@@ -284,6 +287,42 @@ __host__ __device__ inline uint32_t pick_iw(uint32_t nact, uint32_t fill16 = DEF
         }
     }
     return best;
+}
+
+// Lane-group width of an FP64 or mixed plan: pick_iw's, but narrower where a
+// j range of n_jt chunks at most gives too few work items that wide.  An
+// item of 256 slots keeps its workgroup for 256 pairs per lane and tile (some
+// 30 us with one wave per SIMD) while, say, 500 of 10007 particles make 80 of
+// them.  64 slots make 320 items of a quarter of the work, 16 slots 1280 of a
+// sixteenth.  Update times, FP64, 256 | 64 | 16 slots, us:
+//   n =  1024, nact  400: 33 | 15 | 10     n = 10007, nact  500: 34 | 21 | 19
+//   n =  4096, nact 1000: 33 | 17 | 16     n = 10007, nact 1000: 34 | 25 | 24
+//   n =  4096, nact 2000: 35 | 21 | 21     n = 10007, nact 2000: 49 | 35 | 36
+//   n =  4096, nact 4096: 37 | 30 | 31     n = 10007, nact 4300: 69 | 66 | 94
+//   n = 65536, nact  500: 56 | 53 | 54     n = 10007, nact 6000: 85 | 83 | 117
+//   n = 65536, nact 1500: 127 | 164 | 147  n = 20000, nact 4000: 105 | 108 | 111
+// The lines: 1024 items of 256 slots (4 per CU), 512 of 64 slots.
+// nact <= NARROW_ACT keeps pick_iw's width: those steps are k_small_run's and
+// k_team_run's, whose workgroups keep their j and gain nothing.
+// Mixed precision narrows to 64 only (n = 4096, nact 1000: 33 -> 13 us), with
+// jrun = 1: each j sub-group then takes 64 consecutive j, so that the FP32
+// runs are the 32 consecutive pairs that 256 slots sum; with 16 slots they
+// would be others.
+// share: of the chip, in an ensemble.
+constexpr uint32_t ITEMS_256 = 1024, ITEMS_64 = 512;
+struct LaneGroup {
+    uint32_t iw, jrun;
+};
+__host__ __device__ inline LaneGroup lane_group(uint32_t nact, uint32_t fill16, uint32_t n_jt,
+                                                bool mixed, double share = 1.0) {
+    LaneGroup g{pick_iw(nact ? nact : 1, fill16), 0u};
+    if (nact <= NARROW_ACT) return g;
+    if (g.iw == 256 && (double)((nact + 255) / 256) * n_jt < share * ITEMS_256) {
+        g.iw = 64;
+        g.jrun = mixed ? 1u : 0u;
+    }
+    if (!mixed && g.iw == 64 && (double)((nact + 63) / 64) * n_jt < share * ITEMS_64) g.iw = 16;
+    return g;
 }
 
 // Active particles per work item of the exact kernel for nact active ones.

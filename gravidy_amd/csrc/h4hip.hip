@@ -182,14 +182,14 @@ __global__ __launch_bounds__(BS) void k_identity_active(uint32_t *move, Ens e) {
 // Per cluster: lane-group width, j split and work items from its active
 // count; the update workgroups are shared in proportion to nact * n.
 // Exclusive prefix sums over clusters go to items_pre / fin_pre /
-// part_pre, totals to ctl.  `exact`: one lane per i, no j split.
+// part_pre, totals to ctl.  prec: H4H_FP64_EXACT has no j split.
 // Work plan of cluster c for nact active particles; W = sum over the
 // clusters of nact * n (the update workgroups are shared in proportion).
 __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_t nact, double W,
-                                               uint32_t exact) {
+                                               int prec) {
     ClPlan pl;
-    pl.cmaj = 0;
-    if (exact) {
+    pl.cmaj = pl.jrun = 0;
+    if (prec == H4H_FP64_EXACT) {
         pl.iw = exact_iw(nact);
         pl.S = 1;
         pl.tpc = ntiles(e, c);
@@ -201,11 +201,17 @@ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_
         double share = W > 0.0 ? (double)nact * (double)e.cnt[c] / W : 0.0;
         uint32_t g = (uint32_t)(share * e.grid);
         pl.grid = g < 1 ? 1 : g;
-        pl.iw = pick_iw(nact ? nact : 1, e.iw_fill);
+        const LaneGroup lg = lane_group(nact, e.iw_fill, min(ntiles(e, c), e.max_split),
+                                        prec == H4H_MIXED, e.K == 1 ? 1.0 : share);
+        pl.iw = lg.iw;
+        pl.jrun = lg.jrun;
         if (e.tuned && e.K == 1 && nact) {
             uint32_t bucket = 31u - (uint32_t)__clz(nact);
             if (e.tune[bucket]) pl.grid = min(e.tune[bucket], e.grid);
-            if (e.tune[32 + bucket]) pl.iw = e.tune[32 + bucket];
+            if (e.tune[32 + bucket]) {
+                pl.iw = e.tune[32 + bucket];
+                pl.jrun = 0;
+            }
         }
         Decomp d = decompose(nact, pl.iw, ntiles(e, c), pl.grid, e.max_split);
         pl.S = d.S;
@@ -221,10 +227,10 @@ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_
 // Plan of a single-cluster context, made by every workgroup of the update
 // kernel from the active count (so the device step needs no k_plan
 // launch); workgroup 0 publishes it for the finish pass.
-__device__ __forceinline__ ClPlan plan_single(const Ens &e, uint32_t exact,
+__device__ __forceinline__ ClPlan plan_single(const Ens &e, int prec,
                                               unsigned long long &items) {
     const uint32_t nact = e.cs[0].nact;
-    const ClPlan pl = plan_cluster(e, 0, nact, (double)nact * (double)e.cnt[0], exact);
+    const ClPlan pl = plan_cluster(e, 0, nact, (double)nact * (double)e.cnt[0], prec);
     items = nact ? (unsigned long long)pl.n_it * pl.S : 0ull;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const uint32_t per = BS / pl.lanes;
@@ -240,7 +246,7 @@ __device__ __forceinline__ ClPlan plan_single(const Ens &e, uint32_t exact,
     return pl;
 }
 
-__device__ void plan_all(const Ens &e, uint32_t exact) {
+__device__ void plan_all(const Ens &e, int prec) {
     __shared__ double wsum[BS / 64];
     double w = 0.0;
     for (uint32_t c = threadIdx.x; c < e.K; c += BS)
@@ -250,7 +256,7 @@ __device__ void plan_all(const Ens &e, uint32_t exact) {
     __syncthreads();
     double W = 0.0;
     for (uint32_t k = 0; k < BS / 64; ++k) W += wsum[k];
-    for (uint32_t c = threadIdx.x; c < e.K; c += BS) e.plan[c] = plan_cluster(e, c, e.cs[c].nact, W, exact);
+    for (uint32_t c = threadIdx.x; c < e.K; c += BS) e.plan[c] = plan_cluster(e, c, e.cs[c].nact, W, prec);
     __syncthreads();
     // Exclusive prefix sums of work items, finish units and partial doubles
     // over the clusters, BS clusters at a time.
@@ -304,7 +310,7 @@ __device__ void plan_all(const Ens &e, uint32_t exact) {
     }
 }
 
-__global__ __launch_bounds__(BS) void k_plan(Ens e, uint32_t exact) { plan_all(e, exact); }
+__global__ __launch_bounds__(BS) void k_plan(Ens e, int prec) { plan_all(e, prec); }
 
 // ---------------------------------------------------------------------------
 // Exchanges inside a wave
@@ -670,11 +676,12 @@ __global__ __launch_bounds__(BS) void k_save_old(Soa s, Ens e, const uint32_t *m
 // Loads JT consecutive predictor records starting at j0 into an LDS tile;
 // each of the BS (= JT) threads moves one record (two coalesced double4
 // loads).  ES = 1: pp records at [0, JT), pv records at [JT, 2 JT);
-// ES = 2: record t at [2t] (pp) and [2t + 1] (pv).
+// ES = 2: record t at [2t] (pp) and [2t + 1] (pv).  Thread t's record goes to place at.
 template <uint32_t ES = 1>
-__device__ __forceinline__ void load_jtile(const Soa &s, uint32_t j0, double4 *tile) {
-    tile[ES * threadIdx.x] = s.pp[j0 + threadIdx.x];
-    tile[ES == 2 ? 2 * threadIdx.x + 1 : JT + threadIdx.x] = s.pv[j0 + threadIdx.x];
+__device__ __forceinline__ void load_jtile(const Soa &s, uint32_t j0, double4 *tile,
+                                           uint32_t at) {
+    tile[ES * at] = s.pp[j0 + threadIdx.x];
+    tile[ES == 2 ? 2 * at + 1 : JT + at] = s.pv[j0 + threadIdx.x];
 }
 
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -929,7 +936,7 @@ __device__ __forceinline__ void exact_item_wide(const Soa &s, const uint32_t *mv
     double fo[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     for (uint32_t j0 = j_begin; j0 < j_end; j0 += JT) {
         __syncthreads();
-        load_jtile(s, j0, tile);
+        load_jtile(s, j0, tile, threadIdx.x);
         __syncthreads();
         const uint32_t jn = min((uint32_t)JT, j_end - j0);
         for (uint32_t jj = 0; jj < jn; ++jj) {
@@ -957,7 +964,7 @@ __global__ __launch_bounds__(BS) void k_update_exact(Soa s, Ens e, const uint32_
     unsigned long long total = 0;
     ClPlan pl0{};
     if (single)
-        pl0 = plan_single(e, 1u, total);
+        pl0 = plan_single(e, H4H_FP64_EXACT, total);
     else
         total = e.ctl->items;
     for (unsigned long long item = blockIdx.x; item < total; item += gridDim.x) {
@@ -997,6 +1004,12 @@ __device__ __forceinline__ void update_item(const Soa &s, const ClPlan &pl, uint
     // instructions' offset field, with no extra address arithmetic (0.5 %
     // on the full step; the mixed kernel runs as fast with two arrays).
     constexpr uint32_t ES = (IW >= 64 && !MIXED) ? 2u : 1u;
+    // jrun: record j of a tile is stored where sub-group j / 64 reads its
+    // (j % 64)th (a second pair loop for it made the mixed kernel 12
+    // registers larger and 0.5 % slower).
+    constexpr bool RUNS = IW == 64 && MIXED;
+    auto place = [&](uint32_t j) { return RUNS && pl.jrun ? (j % 64) * (JT / 64) + j / 64 : j; };
+    const uint32_t at = place(threadIdx.x);
     // The first j tile is requested before the i particles, whose loads wait
     // for their indices, so the two memory latencies overlap: narrow groups
     // start its copy into lA (once the previous item is done with lA: tiles
@@ -1032,7 +1045,8 @@ __device__ __forceinline__ void update_item(const Soa &s, const ClPlan &pl, uint
         const bool self = (i - j0) < (uint32_t)JT;
         const double4 *sv = ES == 2 ? buf + 1 : buf + JT;
         if (__ballot(self))
-            tile_pairs<IW, true, MIXED, ES>(pi, i, j0, js, buf, sv, e2, fo);
+            tile_pairs<IW, true, MIXED, ES>(pi, RUNS && self ? j0 + place(i - j0) : i, j0, js, buf,
+                                            sv, e2, fo);
         else
             tile_pairs<IW, false, MIXED, ES>(pi, i, j0, js, buf, sv, e2, fo);
     };
@@ -1058,13 +1072,13 @@ __device__ __forceinline__ void update_item(const Soa &s, const ClPlan &pl, uint
         // Wide lane groups do 64-256 pairs per lane and tile: the copy is
         // a small share of the time and one buffer keeps registers free.
         __syncthreads();  // the previous item is done with lA (tiles or red)
-        lA[ES * threadIdx.x] = ja;
-        lA[ES == 2 ? 2 * threadIdx.x + 1 : JT + threadIdx.x] = jb;
+        lA[ES * at] = ja;
+        lA[ES == 2 ? 2 * at + 1 : JT + at] = jb;
         __syncthreads();
         tile(lA, t0);
         for (uint32_t tt = t0 + 1; tt < t1; ++tt) {
             __syncthreads();
-            load_jtile<ES>(s, tt * JT, lA);
+            load_jtile<ES>(s, tt * JT, lA, at);
             __syncthreads();
             tile(lA, tt);
         }
@@ -1124,7 +1138,7 @@ __device__ __forceinline__ void update_items(const Soa &s, const Ens &e, const u
     double *red = reinterpret_cast<double *>(lA);
     const bool single = e.K == 1;
     unsigned long long total = 0;
-    const ClPlan pl0 = single ? plan_single(e, 0u, total) : ClPlan{};
+    const ClPlan pl0 = single ? plan_single(e, MIXED ? H4H_MIXED : H4H_FP64, total) : ClPlan{};
     if (!single) total = e.ctl->items;
     // The first gridDim.x items go one to each workgroup; a workgroup that
     // has finished one takes the next unclaimed item from the queue counter,
@@ -3225,8 +3239,9 @@ uint32_t max_items(uint32_t n, uint32_t grid, uint32_t max_split, uint32_t fill1
     uint32_t best = 1;
     for (uint32_t nact = 1;; nact = (nact < 64 ? nact + 1 : nact * 2)) {
         uint32_t k = nact > n ? n : nact;
-        Decomp d = decompose(k, pick_iw(k, fill16), n_jt, grid, max_split);
-        best = std::max(best, d.n_items);
+        // (narrower groups make at least as many items)
+        const LaneGroup lg = lane_group(k, fill16, std::min(n_jt, max_split), false);
+        best = std::max(best, decompose(k, lg.iw, n_jt, grid, max_split).n_items);
         if (nact >= n) break;
     }
     return best;
@@ -3334,7 +3349,7 @@ int launch_select(h4h_ctx *ctx, uint32_t flags, double itime, uint32_t par = 0) 
 
 int launch_plan(h4h_ctx *ctx) {
     hipLaunchKernelGGL(k_plan, dim3(1), dim3(BS), 0, ctx->stream, ctx->e,
-                       ctx->precision == H4H_FP64_EXACT ? 1u : 0u);
+                       ctx->precision);
     H4H_LAUNCHED();
     return H4H_OK;
 }
@@ -4703,8 +4718,11 @@ int h4h_update_acc_jrk_static(const double *d_p6, const float *d_pm, uint32_t n,
     const uint32_t grid = std::min(DEFAULT_GRID, max_items(n, DEFAULT_GRID, DEFAULT_MAX_SPLIT,
                                                            DEFAULT_IW_FILL));
     if (precision != H4H_FP64_EXACT) {
-        const Decomp d = decompose(nact, pick_iw(nact, DEFAULT_IW_FILL), n_pad / JT, grid,
-                                   DEFAULT_MAX_SPLIT);
+        const Decomp d = decompose(
+            nact,
+            lane_group(nact, DEFAULT_IW_FILL, std::min(n_pad / JT, DEFAULT_MAX_SPLIT),
+                       precision == H4H_MIXED).iw,
+            n_pad / JT, grid, DEFAULT_MAX_SPLIT);
         if (d.S > 1 && 6ull * d.S * d.rows > ST_PART)
             return fail(H4H_EINVAL, "work plan exceeds the static buffer");
     }
