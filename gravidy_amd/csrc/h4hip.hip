@@ -295,18 +295,17 @@ __device__ void plan_all(const Ens &e, int prec) {
     __syncthreads();
     double W = 0.0;
     for (uint32_t k = 0; k < BS / 64; ++k) W += wsum[k];
-    for (uint32_t c = threadIdx.x; c < e.K; c += BS) e.plan[c] = plan_cluster(e, c, e.cs[c].nact, W, prec);
-    __syncthreads();
-    // Exclusive prefix sums of work items, finish units and partial doubles
-    // over the clusters, BS clusters at a time.
+    // The plans, and exclusive prefix sums of work items, finish units and
+    // partial doubles over the clusters, BS clusters at a time.
     __shared__ unsigned long long wtot[3][BS / 64];
     unsigned long long carry[3] = {0ull, 0ull, 0ull};
     for (uint32_t base = 0; base < e.K; base += BS) {
         const uint32_t c = base + threadIdx.x;
         unsigned long long v[3] = {0ull, 0ull, 0ull};
-        if (c < e.K && e.cs[c].nact) {
-            const ClPlan pl = e.plan[c];
-            const uint32_t nact = e.cs[c].nact;
+        const uint32_t nact = c < e.K ? e.cs[c].nact : 0u;
+        if (nact) {
+            const ClPlan pl = plan_cluster(e, c, nact, W, prec);
+            e.plan[c] = pl;
             const uint32_t per = BS / pl.lanes;
             v[0] = (unsigned long long)pl.n_it * pl.S;
             v[1] = (nact + per - 1) / per;
@@ -1448,7 +1447,6 @@ __global__ __launch_bounds__(BS) void k_correct(Soa s, Ens e, const uint32_t *mo
     }
 }
 
-enum : uint32_t { FIN_WRITE_F = 0, FIN_CORRECT = 1 };
 
 // Sum of active particle k's S j-chunk partials (plan pl, partials of its
 // cluster at part) on the group of L = pl.lanes consecutive lanes of one
@@ -1494,35 +1492,25 @@ __device__ __forceinline__ void chunk_sums(const Soa &s, const ClPlan &pl, const
 }
 
 // Finish pass of an update: adds the j-chunk partials of each active
-// particle (chunk_sums) and either stores the forces (FIN_WRITE_F) or
-// applies the corrector at the cluster's block time ATIME (FIN_CORRECT,
-// after a selection that wrote the active particles' records, whose loads
-// go out with those of the partials).  A particle's chunk sums are spread
-// over L = pl.lanes lanes, so a workgroup finishes BS/L particles with no
-// barrier.
+// particle (chunk_sums) and stores the forces.  A particle's chunk sums are
+// spread over L = pl.lanes lanes, so a workgroup finishes BS/L particles with
+// no barrier.
 __global__ __launch_bounds__(BS) void k_finish(Soa s, Ens e, const uint32_t *move,
-                                              const double *partial, uint32_t mode, float eta,
-                                              double dt_min, double dt_max) {
+                                              const double *partial) {
     const unsigned long long total = e.ctl->fin_units;
     for (unsigned long long u = blockIdx.x; u < total; u += gridDim.x) {
         const uint32_t c = find_cluster(e.fin_pre, e.K, u);
         const ClPlan pl = e.plan[c];
+        if (pl.S == 1) continue;  // the update stored them
         const uint32_t L = pl.lanes;
         const uint32_t lu = (uint32_t)(u - e.fin_pre[c]);
-        const uint32_t nact = e.cs[c].nact;
-        const double T = e.cs[c].atime;
         const uint32_t k = lu * (BS / L) + threadIdx.x / L;
-        const bool valid = k < nact;
+        const bool valid = k < e.cs[c].nact;
         const uint32_t i = valid ? move[e.off[c] + k] : 0u;
-        double o[6], pr[6], dt1 = 0.0;
-        if (mode == FIN_CORRECT && valid) load_arec(e, (size_t)e.off[c] + k, o, pr, dt1);
         double f[6];
         chunk_sums(s, pl, partial + e.part_pre[c], k, i, valid, f);
-        if (valid && threadIdx.x % L == 0) {
-            if (mode == FIN_CORRECT) correct_store(s, i, o, pr, dt1, f, T, eta, dt_min, dt_max);
-            if (pl.S > 1)
-                for (int q = 0; q < 6; ++q) s.f[q][i] = f[q];
-        }
+        if (valid && threadIdx.x % L == 0)
+            for (int q = 0; q < 6; ++q) s.f[q][i] = f[q];
     }
 }
 
@@ -1574,54 +1562,26 @@ __device__ __forceinline__ double block_tmin(const Soa &s, uint32_t b, double *r
     return m;  // valid in thread 0
 }
 
-// Recomputes the per-block minima of the blocks that had active particles
-// this step (dirty list `par`; the others did not change), and records each
-// live cluster's step for its loop tail, which the next launch that needs
-// the cluster's next block time makes (k_select PS_TAIL, k_small_run); the
-// cluster's active count of the next step starts from zero.
-__global__ __launch_bounds__(BS) void k_blockmin_dirty(Soa s, Ens e, uint32_t par) {
-    __shared__ double red[BS / 64];
-    for (uint32_t c = blockIdx.x * BS + threadIdx.x; c < e.K; c += gridDim.x * BS) {
-        ClState *cs = &e.cs[c];
-        if (cs->done) continue;
-        cs->tail_t = cs->atime;
-        cs->tail_nact = cs->nact;
-        cs->tail_steps = cs->steps;
-        cs->tail_pend = 1;
-        cs->nact = 0;
-    }
-    // this workgroup's first list entry is read with the count (the list
-    // has nblk entries and the grid is at most nblk)
-    const uint32_t *dl = e.dirty + (size_t)par * 3 * e.nblk;
-    uint32_t b = dl[3 * blockIdx.x];
-    const uint32_t nd = e.ctl->ndirty[par];
-    for (uint32_t w = blockIdx.x; w < nd; w += gridDim.x) {
-        if (w != blockIdx.x) b = dl[3 * w];
-        __syncthreads();
-        double m = block_tmin(s, b, red);
-        if (threadIdx.x == 0) e.bmin[b] = m;
-    }
-}
-
-// Finish pass of a block step of a single system, one block with active
-// particles per workgroup (the dirty list k_select made for the step's
-// parity: block, first place in the active list, count): the chunk sums
-// and the corrector with
+// Finish pass of a block step, one block with active particles per workgroup
+// (the dirty list k_select made for the step's parity: block, first place in
+// the cluster's active list, count): the chunk sums and the corrector with
 // NbodyUtils::get_timestep_normal and normalize_dt (Hermite4CPU.cpp:370-411,
 // NbodyUtils.cpp:337-424) of the block's active particles, then the block's
 // min(t + dt), from which the loop tail takes the next block time
-// (Hermite4::next_integration_time, Hermite4.cpp:90-102): one launch for
-// what k_finish and k_blockmin_dirty do in two.  The sums are chunk_sums',
-// so the forces are k_finish's bit for bit.  Workgroup 0 records the step
-// for its loop tail (ClState tail_*), which the next launch that needs the
-// next block time makes.  (An ensemble keeps the two
-// launches: its many blocks with one or two active particles each would
-// put one corrector per workgroup instead of up to BS/L.)
+// (Hermite4::next_integration_time, Hermite4.cpp:90-102).  The sums are
+// chunk_sums', so the forces are k_finish's bit for bit.  The step of every
+// live cluster is recorded for its loop tail (ClState tail_*), which the next
+// launch that needs the next block time makes, and the active count of the
+// next step starts from zero.
 //
 // A small step's pass is one chain: list, partials, sums, corrector, minimum.
 // With at most 32 active particles in the block the corrector runs on 8 lanes
 // each (corr8); with that and DPP sums the average launch of an N = 10007 run
-// takes 6.9 us instead of 8.5, of an N = 65536 run 6.2 instead of 8.2.
+// takes 6.9 us instead of 8.5, of an N = 65536 run 6.2 instead of 8.2.  For an
+// ensemble it replaces a pass over the active particles with one-lane
+// correctors and one over the blocks (9.7 + 4.0 us on average for 64 clusters
+// of 1024 to 32768).
+template <bool SINGLE>
 __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32_t *move,
                                                      const double *partial, float eta,
                                                      double dt_min, double dt_max, uint32_t par) {
@@ -1630,26 +1590,29 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
     constexpr uint32_t C8 = BS / 8;  // particles of one corr8 pass
     __shared__ double fs[6 * C8];    // their forces
     __shared__ uint32_t cnts[BS / 64];
-    ClState *cs = &e.cs[0];
     const uint32_t *dl = e.dirty + (size_t)par * 3 * e.nblk;
-    // What the first block needs is requested at once: the loop's stop
-    // flag, the list's count, this workgroup's list entry (read before the
-    // count is known: the list has nblk entries and the grid is at most
-    // nblk; an entry beyond the count is not used), the plan and the block
-    // time.
-    const uint32_t done = cs->done;
+    // What the first block needs is requested at once: the list's count and
+    // this workgroup's list entry (read before the count is known: the list
+    // has nblk entries and the grid is at most nblk; an entry beyond the count
+    // is not used), and for a single system the loop's stop flag, the plan and
+    // the block time.
     const uint32_t nd = e.ctl->ndirty[par];
     uint32_t w = blockIdx.x;
     uint32_t b = dl[3 * w], k0 = dl[3 * w + 1], cnt = dl[3 * w + 2];
-    const ClPlan pl = e.plan[0];
-    const double T = cs->atime;
-    if (done) return;  // the loop stopped at this step's selection
-    const uint32_t L = pl.lanes, per = BS / L;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        // this step's loop tail, for the next step's selection (k_select
-        // PS_TAIL), k_small_run or k_tail to make; the active count of the
-        // next step starts from zero
-        cs->tail_t = T;
+    ClPlan pl{};
+    double T = 0.0;
+    if constexpr (SINGLE) {
+        const uint32_t done = e.cs[0].done;
+        pl = e.plan[0];
+        T = e.cs[0].atime;
+        if (done) return;  // the loop stopped at this step's selection
+    }
+    // the step's loop tail, for the next step's selection (k_select PS_TAIL),
+    // k_small_run or k_tail to make
+    for (uint32_t c = blockIdx.x * BS + threadIdx.x; c < e.K; c += gridDim.x * BS) {
+        ClState *cs = &e.cs[c];
+        if (!SINGLE && cs->done) continue;
+        cs->tail_t = SINGLE ? T : cs->atime;
         cs->tail_nact = cs->nact;
         cs->tail_steps = cs->steps;
         cs->tail_pend = 1;
@@ -1661,6 +1624,16 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
             k0 = dl[3 * w + 1];
             cnt = dl[3 * w + 2];
         }
+        const double *part = partial;
+        uint32_t off = 0;  // of the cluster's active list
+        if constexpr (!SINGLE) {
+            const uint32_t c = cluster_of_block(e, b);
+            pl = e.plan[c];
+            T = e.cs[c].atime;
+            part = partial + e.part_pre[c];
+            off = e.off[c];
+        }
+        const uint32_t L = pl.lanes, per = BS / L;
         // t + dt of the block as it stands, loaded ahead of the corrector
         const uint32_t j = b * JT + threadIdx.x;
         const double tdt = s.t[j] + s.dt[j];
@@ -1672,7 +1645,7 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
             const uint32_t kk = threadIdx.x / 8, lane = threadIdx.x & 7u;
             const bool mine = kk < cnt, vel = lane >= 4;
             const uint32_t c = min(lane & 3u, 2u), q = c + (vel ? 3u : 0u);
-            const uint32_t ka = k0 + (mine ? kk : 0u);
+            const uint32_t ka = off + k0 + (mine ? kk : 0u);
             const double *ar = reinterpret_cast<const double *>(e.arec);
             const size_t np = (size_t)e.nblk * JT;
             const double pr = ar[4 * ((vel ? np : 0) + ka) + c];
@@ -1686,7 +1659,7 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
                 const bool valid = ks < cnt;
                 const uint32_t k = k0 + (valid ? ks : 0u);
                 double f[6];
-                chunk_sums(s, pl, partial, k, pl.S == 1 ? move[k] : 0u, valid, f);
+                chunk_sums(s, pl, part, k, pl.S == 1 ? move[off + k] : 0u, valid, f);
                 if (valid && threadIdx.x % L == 0)
                     for (int y = 0; y < 6; ++y) fs[6 * ks + y] = f[y];
             }
@@ -1717,13 +1690,13 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
                 const uint32_t kk = base + threadIdx.x / L;
                 const bool valid = kk < cnt;
                 const uint32_t k = k0 + (valid ? kk : 0u);
-                const uint32_t i = move[k];
+                const uint32_t i = move[off + k];
                 // the corrector's inputs from the selection's records: their
                 // loads go out with those of the partials
                 double o[6], pr[6], dt1 = 0.0;
-                if (valid) load_arec(e, k, o, pr, dt1);
+                if (valid) load_arec(e, off + k, o, pr, dt1);
                 double f[6];
-                chunk_sums(s, pl, partial, k, i, valid, f);
+                chunk_sums(s, pl, part, k, i, valid, f);
                 if (valid && threadIdx.x % L == 0) {
                     const double dtn = correct_store(s, i, o, pr, dt1, f, T, eta, dt_min, dt_max);
                     if (pl.S > 1)
@@ -3386,9 +3359,9 @@ int launch_update(h4h_ctx *ctx, bool compact = false) {
     return H4H_OK;
 }
 
-int launch_finish(h4h_ctx *ctx, uint32_t mode) {
+int launch_finish(h4h_ctx *ctx) {
     hipLaunchKernelGGL(k_finish, dim3(finish_grid(ctx)), dim3(BS), 0, ctx->stream, ctx->s, ctx->e,
-                       ctx->move, ctx->partial, mode, ctx->eta, ctx->dt_min, ctx->dt_max);
+                       ctx->move, ctx->partial);
     H4H_LAUNCHED();
     return H4H_OK;
 }
@@ -3494,7 +3467,7 @@ int ensure_blockmin(h4h_ctx *ctx) {
 // by the next launch that needs its next block time (the next step's
 // selection, k_small_run, or k_tail after h4h_step), so in a device loop
 // that ends, the step after the last one finds the loop stopped.  One
-// system: three launches (the minima in the finish pass); an ensemble: five.
+// system: three launches (its update makes its own plan); an ensemble: four.
 // par: the step's slot in its captured chunk, mod 2 (its dirty list).
 // Optional HIP events bracket the update kernel.
 int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par) {
@@ -3509,17 +3482,10 @@ int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par) {
     if (events) H4H_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
     if ((rc = launch_update(ctx, true))) return rc;
     if (events) H4H_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-    if (ctx->K == 1) {
-        hipLaunchKernelGGL(k_finish_blocks, dim3(std::min<uint32_t>(ctx->nblk, 1024)), dim3(BS), 0,
-                           ctx->stream, ctx->s, ctx->e, ctx->move, ctx->partial, ctx->eta,
-                           ctx->dt_min, ctx->dt_max, par);
-        H4H_LAUNCHED();
-    } else {
-        if ((rc = launch_finish(ctx, FIN_CORRECT))) return rc;
-        hipLaunchKernelGGL(k_blockmin_dirty, dim3(std::min<uint32_t>(ctx->nblk, 1024)), dim3(BS), 0,
-                           ctx->stream, ctx->s, ctx->e, par);
-        H4H_LAUNCHED();
-    }
+    hipLaunchKernelGGL(ctx->K == 1 ? k_finish_blocks<true> : k_finish_blocks<false>,
+                       dim3(std::min<uint32_t>(ctx->nblk, 1024)), dim3(BS), 0, ctx->stream, ctx->s,
+                       ctx->e, ctx->move, ctx->partial, ctx->eta, ctx->dt_min, ctx->dt_max, par);
+    H4H_LAUNCHED();
     return H4H_OK;
 }
 
@@ -3569,12 +3535,12 @@ int read_state(h4h_ctx *ctx) {
 }
 
 // Update pass of the single-method calls (plan already on the device).
-int update_pass(h4h_ctx *ctx, uint32_t fin_mode) {
+int update_pass(h4h_ctx *ctx) {
     if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
     int rc = launch_update(ctx);
     if (rc) return rc;
     if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-    if ((rc = launch_finish(ctx, fin_mode))) return rc;
+    if ((rc = launch_finish(ctx))) return rc;
     H4H_HIP(hipStreamSynchronize(ctx->stream));
     if (ctx->timing) {
         float ms = 0.f;
@@ -4347,7 +4313,7 @@ int h4h_init_acc_jrk(h4h_ctx *ctx) {
                        ctx->move, ctx->e);
     H4H_LAUNCHED();
     if ((rc = launch_plan(ctx))) return rc;
-    if ((rc = update_pass(ctx, FIN_WRITE_F))) return rc;
+    if ((rc = update_pass(ctx))) return rc;
     ctx->nact_host = ctx->K == 1 ? ctx->cnt[0] : 0;
     return H4H_OK;
 }
@@ -4412,7 +4378,7 @@ int h4h_update_acc_jrk(h4h_ctx *ctx, uint32_t nact) {
     if (rc) return rc;
     if (nact != ctx->nact_host)
         return fail(H4H_EINVAL, "nact differs from the current active list size");
-    if (nact && (rc = update_pass(ctx, FIN_WRITE_F))) return rc;
+    if (nact && (rc = update_pass(ctx))) return rc;
     ctx->stats.block_steps += 1;
     ctx->stats.interactions += (uint64_t)nact * ctx->n;
     ctx->stats.nsteps += nact;
@@ -4922,7 +4888,7 @@ int h4h_update_acc_jrk_static(const double *d_p6, const float *d_pm, uint32_t n,
     }
     H4H_LAUNCHED();
     hipLaunchKernelGGL(k_finish, dim3(std::min<uint32_t>(1024, std::max<uint32_t>(64, e.nblk))),
-                       dim3(BS), 0, st, s, e, move, partial, FIN_WRITE_F, 0.0f, 0.0, 0.0);
+                       dim3(BS), 0, st, s, e, move, partial);
     H4H_LAUNCHED();
     hipLaunchKernelGGL(k_static_out, dim3((nact + BS - 1) / BS), dim3(BS), 0, st, s, d_move, n,
                        nact, tab, d_f6);
