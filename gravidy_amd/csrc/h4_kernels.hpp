@@ -186,8 +186,8 @@ __host__ __device__ inline double dkey_inv(unsigned long long k) {
 // longer ones leave small steps waiting on one item's tile copies (IW 4).
 // (Systems of 5 to TEAM_TILES tiles take one tile per chunk at any width:
 // their small steps are made by one workgroup per tile, k_team_run, with
-// these chunks' sums; so do the larger steps, nact > NARROW_ACT, of all
-// systems of up to TEAM_TILES tiles.)
+// these chunks' sums; so do the larger steps, nact > NARROW_ACT, of single
+// systems of up to 4.)
 // Large active sets of large systems (nact >= 8192 over more than 256
 // tiles) keep chunks of CHUNK_TILES_LARGE tiles: 8 to 32 items per resident
 // workgroup even out the end of the launch, and their finish pass reads
@@ -209,10 +209,12 @@ struct Decomp {
 
 __host__ __device__ inline Decomp decompose(uint32_t nact, uint32_t iw,
                                             uint32_t n_jt, uint32_t grid,
-                                            uint32_t max_split) {
+                                            uint32_t max_split, bool ensemble = false) {
     Decomp d;
     d.n_it = (nact + iw - 1) / iw;
-    uint32_t min_tiles = iw >= 64 || (n_jt <= TEAM_TILES && (n_jt > 4 || nact > NARROW_ACT)) ? 1u : 4u;
+    const bool one_tile =
+        n_jt <= TEAM_TILES && (n_jt > 4 || (!ensemble && nact > NARROW_ACT));
+    uint32_t min_tiles = iw >= 64 || one_tile ? 1u : 4u;
     uint32_t S = 1;
     const uint32_t target = grid * QUEUE_FACTOR;
     if (d.n_it > 0 && d.n_it < target) {
@@ -308,7 +310,9 @@ __host__ __device__ inline uint32_t pick_iw(uint32_t nact, uint32_t fill16 = DEF
 // jrun = 1: each j sub-group then takes 64 consecutive j, so that the FP32
 // runs are the 32 consecutive pairs that 256 slots sum; with 16 slots they
 // would be others.
-// share: of the chip, in an ensemble.
+// share: of the part, in an ensemble.  (Its clusters of up to 4 tiles keep
+// pick_iw's width: a few steps beside the thousands of k_small_run, 17.0 ms
+// with and without for 256 clusters of 128 to 1024.)
 constexpr uint32_t ITEMS_256 = 1024, ITEMS_64 = 512;
 struct LaneGroup {
     uint32_t iw, jrun;

@@ -240,10 +240,13 @@ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_
         double share = W > 0.0 ? (double)nact * (double)e.cnt[c] / W : 0.0;
         uint32_t g = (uint32_t)(share * e.grid);
         pl.grid = g < 1 ? 1 : g;
-        const LaneGroup lg = lane_group(nact, e.iw_fill, min(ntiles(e, c), e.max_split),
-                                        prec == H4H_MIXED, e.K == 1 ? 1.0 : share);
-        pl.iw = lg.iw;
-        pl.jrun = lg.jrun;
+        pl.iw = pick_iw(nact ? nact : 1, e.iw_fill);
+        if (e.K == 1 || ntiles(e, c) > 4) {
+            const LaneGroup lg = lane_group(nact, e.iw_fill, min(ntiles(e, c), e.max_split),
+                                            prec == H4H_MIXED, e.K == 1 ? 1.0 : share);
+            pl.iw = lg.iw;
+            pl.jrun = lg.jrun;
+        }
         if (e.tuned && e.K == 1 && nact) {
             uint32_t bucket = 31u - (uint32_t)__clz(nact);
             if (e.tune[bucket]) pl.grid = min(e.tune[bucket], e.grid);
@@ -252,7 +255,7 @@ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_
                 pl.jrun = 0;
             }
         }
-        Decomp d = decompose(nact, pl.iw, ntiles(e, c), pl.grid, e.max_split);
+        Decomp d = decompose(nact, pl.iw, ntiles(e, c), pl.grid, e.max_split, e.K > 1);
         pl.S = d.S;
         pl.tpc = d.tiles_per_chunk;
         pl.n_it = d.n_it;
