@@ -564,8 +564,7 @@ __device__ __forceinline__ void predict_vals(const double r[3], const double v[3
 // launch reads the tail records and the block minima and writes only fields
 // no workgroup of it reads (the stop flag aside: a workgroup that sees it
 // set would have stopped anyway).  Blocks with active particles go to the
-// dirty list `par` (the step's slot in its captured chunk, mod 2), and
-// workgroup 0 clears the other list's count for the next step.
+// dirty list `par` (the step's slot in its captured chunk, mod 2).
 __global__ __launch_bounds__(BS) void k_select(Soa s, Ens e, uint32_t flags, double itime_arg,
                                               uint32_t par, uint32_t *move) {
 #pragma clang fp contract(off)
@@ -634,7 +633,6 @@ __global__ __launch_bounds__(BS) void k_select(Soa s, Ens e, uint32_t flags, dou
                 go = 1;
                 T = atime;
             }
-            if (b == 0) e.ctl->ndirty[par ^ 1] = 0;
             s_go = go;
             s_time = T;
         }
@@ -1610,6 +1608,8 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
         T = e.cs[0].atime;
         if (done) return;  // the loop stopped at this step's selection
     }
+    // the other list's count, for the next step's selection
+    if (blockIdx.x == 0 && threadIdx.x == 0) e.ctl->ndirty[par ^ 1] = 0;
     // the step's loop tail, for the next step's selection (k_select PS_TAIL),
     // k_small_run or k_tail to make
     for (uint32_t c = blockIdx.x * BS + threadIdx.x; c < e.K; c += gridDim.x * BS) {
@@ -2026,13 +2026,15 @@ __device__ __forceinline__ void one_step_result(const OneStep &one, double atime
 // barriers) and of this one: n = 256 14300 and 7600, n = 1024 21400 and
 // 13900.  512 threads of two particles each have 256 registers: 1024 threads
 // spilled 62 around the pair loop, 5000 cycles of a step at n = 1024.  On exit
-// the predictor records of the last step and the per-block minima of t + dt
-// are stored for the kernels that follow.
+// the per-block minima of t + dt are stored, and the step left to the
+// multi-workgroup kernels is predicted and selected from the registers, which
+// saves it k_select's launch (1.8 us here; 5.4 us and a launch gap there).
 template <bool MIXED>
 __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run,
                                                   uint32_t max_act, double e2, double eta,
                                                   double dt_min, double dt_max,
-                                                  uint32_t self_zero, OneStep one) {
+                                                  uint32_t self_zero, uint32_t par,
+                                                  uint32_t *move, OneStep one) {
 #pragma clang fp contract(off)
     __shared__ double4 lpp[SN], lpv[SN];          // predictor records
     __shared__ __align__(16) double red[6 * SN];  // pair sums per (group, slot)
@@ -2096,8 +2098,7 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     }
     // The loop tail the cluster's last multi-workgroup step left comes
     // first; its next block time is the minimum of t + dt, which these
-    // threads hold.  (The dirty lists are cleared for the steps that follow
-    // this launch, whose parities need not continue the last step's.)
+    // threads hold.
     if (loop && cs->tail_pend) {
         const double Tp = cs->tail_t;
         const uint32_t np = cs->tail_nact;
@@ -2107,7 +2108,6 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
         if (tid == 0) {
             record_tail(e, c, Tp, np, steps, mn, last);
             cs->tail_pend = 0;
-            e.ctl->ndirty[0] = e.ctl->ndirty[1] = 0;
         }
         if (last) return;  // (the block minima are the finish pass's)
         inter += (unsigned long long)np * n;
@@ -2341,11 +2341,64 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
                 atomicAdd(&e.ctl->ndone, 1u);
             }
         }
-        for (uint32_t k = 0; k < SP; ++k)
+        if (stop || !loop)
+            for (uint32_t k = 0; k < SP; ++k)
+                if (in[k]) {
+                    s.pp[off + tid + k * SB] = lpp[tid + k * SB];
+                    s.pv[off + tid + k * SB] = lpv[tid + k * SB];
+                }
+    }
+    // The step left is selected here, from the registers: what k_select does
+    // with PS_COMPACT, in particle order, so that each block's active
+    // particles are neighbours in the list.
+    if (loop && !stop) {
+        __syncthreads();  // wcnt may be being read
+        nact = small_count(act, wcnt, k_act);
+        for (uint32_t k = 0; k < SP; ++k) {
+            const uint32_t gi = off + tid + k * SB, slot = off + k_act[k];
+            double4 a, b;
             if (in[k]) {
-                s.pp[off + tid + k * SB] = lpp[tid + k * SB];
-                s.pv[off + tid + k * SB] = lpv[tid + k * SB];
+                predict_vals(r[k], v[k], f[k], T - ti[k], mf[k], a, b);
+                s.pp[gi] = a;
+                s.pv[gi] = b;
             }
+            if (act[k]) {
+                move[slot] = gi;
+                auto *col = in_loop(s.r[0]) + gi;
+                for (int q = 0; q < 6; ++q) col[(COL_OLD + q) * np] = f[k][q];
+                e.arec[slot] = a;
+                e.arec[np + slot] = b;
+                e.arec[2 * np + slot] = make_double4(f[k][0], f[k][1], f[k][2], dti[k]);
+                e.arec[3 * np + slot] = make_double4(f[k][3], f[k][4], f[k][5], 0.0);
+            }
+        }
+        if (w == 0) {  // block `lane` of the cluster: the list entry
+            constexpr uint32_t WPB = JT / 64;
+            uint32_t below = 0, cnt = 0;
+            for (uint32_t q = 0; q < SC; ++q) {
+                const uint32_t x = wcnt[q];
+                below += q / WPB < lane ? x : 0u;
+                cnt += q / WPB == lane ? x : 0u;
+            }
+            const unsigned long long has = __ballot(cnt != 0);
+            uint32_t d = 0;
+            if (lane == 0) {
+                const uint32_t total = (uint32_t)__popcll(has);
+                if (e.K == 1)
+                    e.ctl->ndirty[par] = total;
+                else
+                    d = atomicAdd(&e.ctl->ndirty[par], total);
+                cs->nact = nact;
+            }
+            d = (uint32_t)__builtin_amdgcn_readfirstlane((int)d) +
+                (uint32_t)__popcll(has & ((1ull << lane) - 1ull));
+            if (cnt) {
+                uint32_t *dl = e.dirty + ((size_t)par * e.nblk + d) * 3;
+                dl[0] = off / JT + lane;
+                dl[1] = below;
+                dl[2] = cnt;
+            }
+        }
     }
     __syncthreads();  // wmin is rewritten below
     for (uint32_t k = 0; k < SP; ++k) {
@@ -2672,7 +2725,6 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             if (pend && b == 0 && tid == 0) {
                 record_tail(e, 0, Tp, np_tail, steps, T, false);
                 cs->tail_pend = 0;
-                ctl->ndirty[0] = ctl->ndirty[1] = 0;
             }
         }
         if (s_bad) break;
@@ -3421,11 +3473,12 @@ bool self_pair_is_zero(int precision, double e2, double mmax) {
 }
 
 // One workgroup per cluster.
-int launch_small(h4h_ctx *ctx, uint32_t max_run, OneStep one = {}) {
+int launch_small(h4h_ctx *ctx, uint32_t max_run, uint32_t par, OneStep one = {}) {
     auto *kern = ctx->precision == H4H_MIXED ? k_small_run<true> : k_small_run<false>;
     hipLaunchKernelGGL(kern, dim3(ctx->K), dim3(SB), 0, ctx->stream, ctx->s, ctx->e, max_run,
                        ctx->small_act, ctx->e2, (double)ctx->eta, ctx->dt_min, ctx->dt_max,
-                       self_pair_is_zero(ctx->precision, ctx->e2, ctx->mass_max) ? 1u : 0u, one);
+                       self_pair_is_zero(ctx->precision, ctx->e2, ctx->mass_max) ? 1u : 0u, par,
+                       ctx->move, one);
     H4H_LAUNCHED();
     return H4H_OK;
 }
@@ -3471,11 +3524,12 @@ int ensure_blockmin(h4h_ctx *ctx) {
 // selection, k_small_run, or k_tail after h4h_step), so in a device loop
 // that ends, the step after the last one finds the loop stopped.  One
 // system: three launches (its update makes its own plan); an ensemble: four.
-// par: the step's slot in its captured chunk, mod 2 (its dirty list).
-// Optional HIP events bracket the update kernel.
-int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par) {
+// par: the step's slot in its captured chunk, mod 2 (its dirty list); select
+// false: k_small_run has made the selection.  Optional HIP events bracket the update kernel.
+int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par, bool select = true) {
     int rc;
-    if ((rc = launch_select(ctx,
+    if (select &&
+        (rc = launch_select(ctx,
                             PS_PREDICT | PS_SELECT | PS_SAVE_OLD | PS_DEVTIME | PS_DIRTY | PS_TAIL |
                                 PS_COMPACT,
                             0.0, par)))
@@ -3498,10 +3552,11 @@ int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par) {
 // multi-workgroup kernels (the step it left, if any).  At most HIST_CAP steps.
 int enqueue_chunk(h4h_ctx *ctx) {
     int rc = H4H_OK;
-    if (small_path(ctx) || team_path(ctx)) {
+    const bool small = small_path(ctx);
+    if (small || team_path(ctx)) {
         for (uint32_t k = 0; k < SMALL_SLOTS && rc == H4H_OK; ++k) {
-            rc = small_path(ctx) ? launch_small(ctx, SMALL_RUN) : launch_team(ctx, SMALL_RUN);
-            if (rc == H4H_OK) rc = enqueue_step(ctx, false, k & 1);
+            rc = small ? launch_small(ctx, SMALL_RUN, k & 1) : launch_team(ctx, SMALL_RUN);
+            if (rc == H4H_OK) rc = enqueue_step(ctx, false, k & 1, !small);
         }
     } else {
         for (uint32_t k = 0; k < RUN_CHUNK && rc == H4H_OK; ++k) rc = enqueue_step(ctx, false, k & 1);
@@ -4515,7 +4570,7 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     ctx->cs_host[0] = ClState{};
     if (small_path(ctx) || team_path(ctx)) {
         const OneStep one{itime, ctx->cs_host};
-        if ((rc = small_path(ctx) ? launch_small(ctx, 1, one) : launch_team(ctx, 1, one))) return rc;
+        if ((rc = small_path(ctx) ? launch_small(ctx, 1, 0, one) : launch_team(ctx, 1, one))) return rc;
         if (ctx->timing)
             for (int k : {0, 1, 3}) H4H_HIP(hipEventRecord(ctx->ev[k], ctx->stream));
         H4H_HIP(hipStreamSynchronize(ctx->stream));
