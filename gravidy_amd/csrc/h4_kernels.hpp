@@ -151,7 +151,7 @@ struct Ens {
                              // of the active list (index off[c] + k): predictor
                              // (pp, pv), then old forces and step ((a, dt), (jerk, 0));
                              // written by the selection of a device-loop step
-    double *hist_t;          // per-step history of cluster 0 (ring)
+    double *hist_t;          // per-step history of cluster 0 (ring, pinned host memory)
     uint32_t *hist_n;
     uint32_t hist_cap;
     uint32_t grid;           // persistent workgroups of the update kernel

@@ -3270,15 +3270,13 @@ struct h4h_ctx {
     bool team_ok = false;        // the system has a team's number of tiles
     double4 *d_arec = nullptr;   // the step's active particles' records (Ens::arec)
     uint32_t *d_tune = nullptr;  // [64] tuning table
-    double *hist_t = nullptr;
-    uint32_t *hist_n = nullptr;
     // pinned host memory: energy per-workgroup sums, mirrors
     double *pinned = nullptr;
     double *eout = nullptr;
     RunCtl *ctl_host = nullptr;
     ClState *cs_host = nullptr;
-    double *hist_t_host = nullptr;
-    uint32_t *hist_n_host = nullptr;
+    double *hist_t_host = nullptr;   // step history, written by the device (Ens::hist_t): a
+    uint32_t *hist_n_host = nullptr; // copy of it after each chunk took 5 us and a gap
     uint32_t *team_plan_host = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -3864,8 +3862,6 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
         {(void **)&ctx->d_dirty, 6 * (size_t)ctx->nblk * sizeof(uint32_t)},
         {(void **)&ctx->d_bmin, ctx->nblk * (sizeof(double) + sizeof(uint32_t))},
         {(void **)&ctx->d_arec, 4 * np * sizeof(double4) + team_bytes},
-        {(void **)&ctx->hist_t, HIST_CAP * sizeof(double)},
-        {(void **)&ctx->hist_n, HIST_CAP * sizeof(uint32_t)},
     };
     size_t bytes = 0, zeroed = 0;
     for (const Piece &x : pieces) {
@@ -3925,8 +3921,8 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     e.bmin = ctx->d_bmin;
     e.bcnt = reinterpret_cast<uint32_t *>(ctx->d_bmin + ctx->nblk);
     e.arec = ctx->d_arec;
-    e.hist_t = ctx->hist_t;
-    e.hist_n = ctx->hist_n;
+    e.hist_t = ctx->hist_t_host;
+    e.hist_n = ctx->hist_n_host;
     e.hist_cap = HIST_CAP;
     e.tuned = 0;
     e.tune = ctx->d_tune;
@@ -4623,12 +4619,6 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
         }
         H4H_HIP(hipMemcpyAsync(ctx->ctl_host, ctx->d_ctl, sizeof(RunCtl) + sizeof(ClState),
                                hipMemcpyDeviceToHost, ctx->stream));
-        if (hist) {
-            H4H_HIP(hipMemcpyAsync(ctx->hist_t_host, ctx->hist_t, HIST_CAP * sizeof(double),
-                                   hipMemcpyDeviceToHost, ctx->stream));
-            H4H_HIP(hipMemcpyAsync(ctx->hist_n_host, ctx->hist_n, HIST_CAP * sizeof(uint32_t),
-                                   hipMemcpyDeviceToHost, ctx->stream));
-        }
         H4H_HIP(hipStreamSynchronize(ctx->stream));
         if ((rc = check_team(ctx, ctx->ctl_host->team_err != 0))) return rc;
         if (hist) {
@@ -4668,14 +4658,7 @@ int h4h_run(h4h_ctx *ctx, double t_end, double t_stop, uint64_t max_steps, h4h_r
     io->steps = d.steps;
     io->interactions = d.interactions;
     io->nsteps = d.nsteps;
-    uint32_t last = 0;
-    if (d.steps) {
-        // nact of the last step: from the history ring
-        H4H_HIP(hipMemcpyAsync(ctx->hist_n_host, ctx->hist_n, HIST_CAP * sizeof(uint32_t),
-                               hipMemcpyDeviceToHost, ctx->stream));
-        H4H_HIP(hipStreamSynchronize(ctx->stream));
-        last = ctx->hist_n_host[(d.steps - 1) % HIST_CAP];
-    }
+    const uint32_t last = d.steps ? ctx->hist_n_host[(d.steps - 1) % HIST_CAP] : 0u;
     io->last_nact = last;
     if (d.steps && d.itime >= t_stop)
         io->stopped = H4H_STOP_OUTPUT;
