@@ -1829,19 +1829,30 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
 
 // The loop tail a single system's last block step left (k_finish_blocks),
 // when no further step of the loop makes it: after one h4h_step, whose
-// result goes to the pinned record `host`.
+// result goes to the pinned record `host` (with the next step's active count,
+// see one_step_result).
 __global__ __launch_bounds__(BS) void k_tail(Ens e, ClState *host) {
     __shared__ double red[BS / 64];
+    __shared__ uint32_t next;
     ClState *cs = &e.cs[0];
     double mn = INFINITY;
     for (uint32_t b = threadIdx.x; b < e.nblk; b += BS) mn = fmin(mn, e.bmin[b]);
     mn = block_min(mn, red);
+    if (threadIdx.x == 0) {
+        red[0] = mn;
+        next = 0;
+    }
+    __syncthreads();
+    for (uint32_t b = threadIdx.x; b < e.nblk; b += BS)
+        if (e.bmin[b] == red[0]) atomicAdd(&next, min(e.bcnt[b], BCNT_MANY));
+    __syncthreads();
     if (threadIdx.x == 0) {
         const unsigned long long steps = cs->tail_steps + 1;
         record_tail(e, 0, cs->tail_t, cs->tail_nact, steps, mn,
                     loop_stops(*e.ctl, cs->tail_t, steps, mn));
         cs->tail_pend = 0;
         *host = *cs;
+        host->tail_nact = next;
     }
 }
 
@@ -1981,9 +1992,12 @@ struct OneStep {
     double itime;
     ClState *host;  // null: a device loop
 };
+// next: the next block step's active count (ClState::tail_nact there;
+// BCNT_MANY or more: not known).
 __device__ __forceinline__ void one_step_result(const OneStep &one, double atime, uint32_t nact,
-                                                uint32_t n, uint32_t small) {
+                                                uint32_t n, uint32_t small, uint32_t next) {
     one.host->atime = atime;
+    one.host->tail_nact = next;
     one.host->nsteps = nact;
     one.host->interactions = (unsigned long long)nact * n;
     one.host->small_steps = small;
@@ -2328,7 +2342,7 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     // Loop state and predictor records of the last step made; per-block
     // minima of t + dt.
     if (it > 0) {
-        if (tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 1);
+        if (tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 1, nact);
         if (tid == 0 && loop) {
             cs->itime = t_last;
             cs->atime = T;
@@ -2401,16 +2415,28 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
         }
     }
     __syncthreads();  // wmin is rewritten below
+    // (block_min_count's, block by block)
     for (uint32_t k = 0; k < SP; ++k) {
         const double m = wave_min(tdt[k]);
-        if (lane == 0) wmin[k * SW + w] = m;
+        const bool near = __ballot(tdt[k] != m && fabs(m - tdt[k]) < 2 * DBL_EPSILON) != 0;
+        const uint32_t at = (uint32_t)__popcll(__ballot(tdt[k] == m));
+        if (lane == 0) {
+            wmin[k * SW + w] = m;
+            wcnt[k * SW + w] = near ? BCNT_MANY : at;
+        }
     }
     __syncthreads();
     constexpr uint32_t WPB = JT / 64;  // chunks per block
     if (tid < ntiles(e, c)) {
-        double m = wmin[tid * WPB];
-        for (uint32_t k = 1; k < WPB; ++k) m = fmin(m, wmin[tid * WPB + k]);
+        const uint32_t w0 = tid * WPB;
+        double m = wmin[w0];
+        uint32_t at = 0;
+        for (uint32_t k = 1; k < WPB; ++k) m = vmin(m, wmin[w0 + k]);
+        for (uint32_t k = 0; k < WPB; ++k)
+            at += wmin[w0 + k] == m ? wcnt[w0 + k]
+                  : fabs(m - wmin[w0 + k]) < 2 * DBL_EPSILON ? BCNT_MANY : 0u;
         e.bmin[off / JT + tid] = m;
+        e.bcnt[off / JT + tid] = at;
     }
 }
 
@@ -2775,7 +2801,8 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             if (++hk == e.hist_cap) hk = 0;
         }
         T = mn;
-        if (stop || it >= max_run || close || nact < 1 || nact > TM_ACT) break;
+        if (close) nact = BCNT_MANY;  // (not counted)
+        if (stop || it >= max_run || nact < 1 || nact > TM_ACT) break;
         const uint32_t plan = __builtin_amdgcn_readfirstlane(plans[nact]);
         if (!plan) break;
         const uint32_t lw = plan & 0xffffu, iw = 1u << lw, ll = plan >> 16, L = 1u << ll;
@@ -2944,7 +2971,7 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     }
     // Loop state, predictor records of the last step, block minima.
     if (it > 0) {
-        if (b == 0 && tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 0);
+        if (b == 0 && tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 0, nact);
         if (b == 0 && tid == 0 && loop) {
             cs->itime = t_last;
             cs->atime = T;
@@ -3249,6 +3276,8 @@ struct h4h_ctx {
     bool small_ok = false;   // the device can launch k_small_run
     uint32_t small_act = SMALL_ACT;  // k_small_run takes active sets up to this (0: off)
     uint32_t nact_host = 0;  // size of cluster 0's active list (single-system calls)
+    uint32_t next_nact = 0;  // active count of the step at next_time, told by the last h4h_step
+    double next_time = 0.0;  // (while the block minima stay valid; 0: not known)
     double mass_max = 0.0;   // largest |float mass| of the uploaded state (+inf: not finite)
 
     hipStream_t stream = nullptr;
@@ -4558,15 +4587,21 @@ int h4h_next_integration_time(h4h_ctx *ctx, double *atime) {
 int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     int rc = check_single(ctx);
     if (rc) return rc;
-    if ((rc = ensure_blockmin(ctx))) return rc;
-    if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
     // The step the device loop would make: k_small_run or k_team_run when they
     // take it, which the host looks at before it launches the others (most
-    // steps are theirs, and the launches cost more than a look).
+    // steps are theirs, and the launches cost more than a look).  A step that
+    // the last one has counted and found too large for them is spared the look
+    // (18 us of 50).
+    const bool small = small_path(ctx);
+    const bool large = ctx->bm_valid && itime == ctx->next_time && ctx->next_nact < BCNT_MANY &&
+                       ctx->next_nact > (small ? std::min(ctx->small_act, SMALL_MAX_ACT) : TM_ACT);
+    ctx->next_nact = 0;
+    if ((rc = ensure_blockmin(ctx))) return rc;
+    if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
     ctx->cs_host[0] = ClState{};
-    if (small_path(ctx) || team_path(ctx)) {
+    if (!large && (small || team_path(ctx))) {
         const OneStep one{itime, ctx->cs_host};
-        if ((rc = small_path(ctx) ? launch_small(ctx, 1, 0, one) : launch_team(ctx, 1, one))) return rc;
+        if ((rc = small ? launch_small(ctx, 1, 0, one) : launch_team(ctx, 1, one))) return rc;
         if (ctx->timing)
             for (int k : {0, 1, 3}) H4H_HIP(hipEventRecord(ctx->ev[k], ctx->stream));
         H4H_HIP(hipStreamSynchronize(ctx->stream));
@@ -4594,6 +4629,8 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     const ClState &cs = ctx->cs_host[0];
     uint32_t k = (uint32_t)cs.nsteps;  // the step's nact (counters were reset)
     ctx->nact_host = 0;
+    ctx->next_nact = cs.tail_nact;
+    ctx->next_time = cs.atime;
     ctx->stats.block_steps += 1;
     ctx->stats.interactions += cs.interactions;
     ctx->stats.nsteps += k;
@@ -4606,6 +4643,7 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
 // Replays captured chunks of RUN_CHUNK steps until every cluster's loop has
 // stopped; copies cluster 0's per-step history when asked.
 static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint64_t cap) {
+    ctx->next_nact = 0;
     int rc = ctx->graphs ? ensure_graph(ctx) : H4H_OK;
     if (rc) return rc;
     uint64_t seen = 0;
