@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -1827,10 +1828,32 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
     }
 }
 
+// Stores and loads of this wave so far are done.
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// The result of one h4h_step, to the pinned record the host waits at: its
+// fields, and when they are there `done`.  (Waiting for the launch itself
+// takes 5 us more, of a step of 18 to 28.)  next: the next block step's
+// active count (tail_nact there; BCNT_MANY or more: not known).
+enum : uint32_t { STEP_DONE = 1, STEP_LEFT = 2, STEP_FAILED = 3 };
+template <class T>
+__device__ __forceinline__ void host_store(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void step_result(ClState *host, double atime, uint32_t nact, uint32_t n,
+                                            unsigned long long small, uint32_t next) {
+    host_store(&host->atime, atime);
+    host_store(&host->nsteps, (unsigned long long)nact);
+    host_store(&host->interactions, (unsigned long long)nact * n);
+    host_store(&host->small_steps, small);
+    host_store(&host->tail_nact, next);
+    wait_memory();
+    host_store(&host->done, (uint32_t)STEP_DONE);
+}
+
 // The loop tail a single system's last block step left (k_finish_blocks),
 // when no further step of the loop makes it: after one h4h_step, whose
-// result goes to the pinned record `host` (with the next step's active count,
-// see one_step_result).
+// result goes to the pinned record `host`.
 __global__ __launch_bounds__(BS) void k_tail(Ens e, ClState *host) {
     __shared__ double red[BS / 64];
     __shared__ uint32_t next;
@@ -1851,8 +1874,7 @@ __global__ __launch_bounds__(BS) void k_tail(Ens e, ClState *host) {
         record_tail(e, 0, cs->tail_t, cs->tail_nact, steps, mn,
                     loop_stops(*e.ctl, cs->tail_t, steps, mn));
         cs->tail_pend = 0;
-        *host = *cs;
-        host->tail_nact = next;
+        step_result(host, mn, cs->tail_nact, e.cnt[0], 0, next);
     }
 }
 
@@ -1986,23 +2008,12 @@ __device__ __forceinline__ void small_pairs(const double pi[6], uint32_t i, uint
 // One block step at `itime` without a device loop (h4h_step): the kernels
 // that make whole steps take the loop's state from here instead of the loop
 // control and the cluster record, and write the step's result to the pinned
-// record `host` (its `steps` stays 0 if they leave the step to others), so
-// that such a step is one launch and no copy.
+// record `host` (STEP_LEFT if they leave the step to others), so that such a
+// step is one launch and no copy.
 struct OneStep {
     double itime;
     ClState *host;  // null: a device loop
 };
-// next: the next block step's active count (ClState::tail_nact there;
-// BCNT_MANY or more: not known).
-__device__ __forceinline__ void one_step_result(const OneStep &one, double atime, uint32_t nact,
-                                                uint32_t n, uint32_t small, uint32_t next) {
-    one.host->atime = atime;
-    one.host->tail_nact = next;
-    one.host->nsteps = nact;
-    one.host->interactions = (unsigned long long)nact * n;
-    one.host->small_steps = small;
-    one.host->steps = 1;
-}
 
 // Block steps of systems of n <= SN particles, workgroup c of SB threads for
 // cluster c (a larger cluster's workgroup returns at once), up to max_run
@@ -2342,7 +2353,6 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     // Loop state and predictor records of the last step made; per-block
     // minima of t + dt.
     if (it > 0) {
-        if (tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 1, nact);
         if (tid == 0 && loop) {
             cs->itime = t_last;
             cs->atime = T;
@@ -2438,6 +2448,14 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
         e.bmin[off / JT + tid] = m;
         e.bcnt[off / JT + tid] = at;
     }
+    if (loop) return;
+    wait_memory();
+    __syncthreads();  // the step's stores are done
+    if (tid) return;
+    if (it > 0)
+        step_result(one.host, T, (uint32_t)nst, n, 1, nact);
+    else
+        host_store(&one.host->done, (uint32_t)STEP_LEFT);
 }
 
 // ---------------------------------------------------------------------------
@@ -2471,7 +2489,7 @@ struct Team {
 };
 constexpr unsigned long long SENT = 0x7FF4A5A55A5A7E57ull;  // a signalling NaN: no sum's value
 enum : uint32_t { TS_DECISION = 0, TS_LEFT = 32, TS_WORDS = 64 };
-enum : uint32_t { TEAM_GO = 1, TEAM_NO = 2, TEAM_FAILED = 3 };
+enum : uint32_t { TEAM_GO = 1, TEAM_NO = 2 };
 
 template <class T>
 __device__ __forceinline__ T agent_load(const T *p) {
@@ -2487,9 +2505,6 @@ __device__ __forceinline__ unsigned long long bits(double x) {
 __device__ __forceinline__ double from_bits(unsigned long long u) {
     return __builtin_bit_cast(double, u);
 }
-// Stores and loads of this wave so far are done.
-__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // The word at p once it is written (SENT if it did not come).  Every writer
 // of a formed team is resident, so the wait is short; POLLS (about a second)
 // only bounds it.  Before (decision not null): some 200 us, and no longer
@@ -2647,8 +2662,11 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
                               (uint32_t)__builtin_amdgcn_readlane((int)c, 32) +
                               (uint32_t)__builtin_amdgcn_readlane((int)c, 48);
         __syncthreads();  // plans
-        if (close || nact < 1 || nact > TM_ACT || !plans[nact]) return;
-        if (pend ? loop_stops(*ctl, Tp, steps, T) : T != atime) return;
+        if (close || nact < 1 || nact > TM_ACT || !plans[nact] ||
+            (pend ? loop_stops(*ctl, Tp, steps, T) : T != atime)) {
+            if (!loop && b == 0 && tid == 0) host_store(&one.host->done, (uint32_t)STEP_LEFT);
+            return;
+        }
     }
 
     bool go = false, stop = false, act = false;
@@ -2971,7 +2989,6 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     }
     // Loop state, predictor records of the last step, block minima.
     if (it > 0) {
-        if (b == 0 && tid == 0 && !loop) one_step_result(one, T, (uint32_t)nst, n, 0, nact);
         if (b == 0 && tid == 0 && loop) {
             cs->itime = t_last;
             cs->atime = T;
@@ -3016,10 +3033,7 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     unsigned long long *rc = tm.rec + ((size_t)slot * M + b) * TM_ACT * 8;
     for (uint32_t k = 8 + tid; k < 8 * min(cnt, TM_ACT); k += TB) agent_store(rc + k, SENT);
     if (!go && tid < 8) agent_store(tm.hdr + (size_t)b * 8 + tid, SENT);
-    if (go && s_bad && tid == 0) {
-        ctl->team_err = 1;
-        if (!loop) one.host->done = TEAM_FAILED;
-    }
+    if (go && s_bad && tid == 0) agent_store(&ctl->team_err, 1u);
     wait_memory();
     __syncthreads();
     if (tid == 0) s_dec = atomicAdd(&tm.sync[TS_LEFT], 1u) == M - 1;
@@ -3035,6 +3049,13 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
         agent_store(&tm.sync[TS_DECISION], 0u);
         agent_store(&tm.sync[TS_LEFT], 0u);
     }
+    if (loop || tid) return;
+    if (agent_load(&ctl->team_err))
+        host_store(&one.host->done, (uint32_t)STEP_FAILED);
+    else if (it > 0)
+        step_result(one.host, T, (uint32_t)nst, n, 0, nact);
+    else
+        host_store(&one.host->done, (uint32_t)STEP_LEFT);
 }
 
 // Every word of a team's buffers waiting (context creation).
@@ -3532,6 +3553,23 @@ int check_team(h4h_ctx *ctx, bool failed) {
     ctx->team_ok = false;
     drop_graph(ctx);
     return fail(H4H_EHIP, "a wait between workgroups ran out; upload the state again");
+}
+
+// The result of h4h_step's launches: when it is in the pinned record, or
+// (with timing events, or if it does not come soon) after them.
+int await_step(h4h_ctx *ctx) {
+    if (!ctx->timing) {
+        const uint32_t *done = &ctx->cs_host[0].done;
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+        do {
+            for (int k = 0; k < 64; ++k) {
+                if (__atomic_load_n(done, __ATOMIC_ACQUIRE)) return H4H_OK;
+                __builtin_ia32_pause();
+            }
+        } while (std::chrono::steady_clock::now() < until);
+    }
+    H4H_HIP(hipStreamSynchronize(ctx->stream));
+    return H4H_OK;
 }
 
 int ensure_blockmin(h4h_ctx *ctx) {
@@ -4604,10 +4642,11 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
         if ((rc = small ? launch_small(ctx, 1, 0, one) : launch_team(ctx, 1, one))) return rc;
         if (ctx->timing)
             for (int k : {0, 1, 3}) H4H_HIP(hipEventRecord(ctx->ev[k], ctx->stream));
-        H4H_HIP(hipStreamSynchronize(ctx->stream));
-        if ((rc = check_team(ctx, ctx->cs_host[0].done == TEAM_FAILED))) return rc;
+        if ((rc = await_step(ctx))) return rc;
+        if ((rc = check_team(ctx, ctx->cs_host[0].done == STEP_FAILED))) return rc;
     }
-    if (!ctx->cs_host[0].steps) {
+    if (ctx->cs_host[0].done != STEP_DONE) {
+        ctx->cs_host[0].done = 0;
         // One-step loop: ATIME = itime, stop after the step.
         hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, (double)INFINITY,
                            -INFINITY, 1ull, 1u, -INFINITY, itime);
@@ -4616,7 +4655,7 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
         hipLaunchKernelGGL(k_tail, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, ctx->cs_host);
         H4H_LAUNCHED();
         if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
-        H4H_HIP(hipStreamSynchronize(ctx->stream));
+        if ((rc = await_step(ctx))) return rc;
     }
     if (ctx->timing) {
         float ms = 0.f;
