@@ -2463,7 +2463,11 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
 // ---------------------------------------------------------------------------
 
 constexpr uint32_t TB = 2 * BS;         // threads of k_team_run
-constexpr uint32_t TM_ACT = 128;        // largest active set it takes
+// Largest active set of a team with tpw tiles per workgroup.  Its pairs keep a
+// workgroup one tile each: at 256 and one tile 15 us, where the launches of a
+// larger step take 45; with two tiles what they take.
+constexpr uint32_t team_act(uint32_t tpw) { return tpw == 1 ? 256u : 128u; }
+constexpr uint32_t ONE_ACT = 128;       // of a single step (h4h_step)
 constexpr uint32_t TEAM_ONE = 128;      // tiles up to which a workgroup has one (else two)
 constexpr uint32_t TEAM_WGS = TEAM_TILES / 2;
 constexpr uint32_t TEAM_BACKOFF = 64;   // steps left alone after a team did not form
@@ -2476,15 +2480,15 @@ static_assert(TEAM_ONE <= TEAM_WGS && TEAM_WGS == 128, "workgroups of a team");
 // word is also waiting for it.
 struct Team {
     uint32_t *sync;             // decision, number of workgroups that have left
-    const uint32_t *plan;       // [TM_ACT + 1]: log2 of the lane-group width | log2 of the
+    const uint32_t *plan;       // [team_act + 1]: log2 of the lane-group width | log2 of the
                                 // finish lanes << 16, of the plan for nact (0: not one chunk
                                 // per tile)
     unsigned long long *hdr;    // [3][workgroups][8]: min(t + dt) of the workgroup's tiles;
                                 // number of particles that have it | first one's index << 32;
                                 // its predicted position and velocity there
-    unsigned long long *rec;    // [3][workgroups][TM_ACT][8]: the others' position, velocity,
+    unsigned long long *rec;    // [3][workgroups][team_act][8]: the others' position, velocity,
                                 // index
-    unsigned long long *part;   // [TM_ACT][6][tiles]: the tiles' partial sums per active particle
+    unsigned long long *part;   // [team_act][6][tiles]: the tiles' partial sums per active particle
                                 // and component (the reader's lanes take consecutive tiles)
 };
 constexpr unsigned long long SENT = 0x7FF4A5A55A5A7E57ull;  // a signalling NaN: no sum's value
@@ -2546,7 +2550,7 @@ __device__ __forceinline__ void team_item(uint32_t it, uint32_t t, uint32_t nact
 
 // Block steps of a single system of 5 to TEAM_TILES j tiles, one workgroup
 // per TPW tiles, up to max_run steps per launch: the device loop's steps with
-// at most TM_ACT active particles whose plan has one chunk per tile, with the
+// at most team_act active particles whose plan has one chunk per tile, with the
 // same operations in the same order as the selection, update and finish
 // launches, so a step has the same bits whichever makes it.  A step of those
 // is three launches of 5-7 us each at least; here it is two exchanges:
@@ -2565,8 +2569,8 @@ __device__ __forceinline__ void team_item(uint32_t it, uint32_t t, uint32_t nact
 // 10007 26.0 -> 17.8, 20000 33.0 -> 24.8, 65536 46.0 -> 39.2.  Up to TEAM_ONE
 // tiles a workgroup has one, its two groups of BS threads take turns at the
 // i tiles (N = 20000: 24.8 us, 27.1 with two tiles each); beyond, two, as 256
-// workgroups exchange more slowly than 128.  Steps with more than TM_ACT
-// active particles want the whole chip for their pairs.
+// workgroups exchange more slowly than 128.  Steps with more active particles
+// want the whole chip for their pairs.
 //
 // Buffers: (1) goes round three slots; a workgroup clears its words of the
 // slot before the last exchange when that exchange is complete (then every
@@ -2581,12 +2585,18 @@ __device__ __forceinline__ void team_item(uint32_t it, uint32_t t, uint32_t nact
 // setting holds; after GO all are resident until they end.  After NO
 // everybody leaves without having changed anything, and so they do when the
 // next step is not one of theirs: the launches after this one make it.
-template <bool MIXED, uint32_t TPW>
+//
+// ONE: a single step at `one.itime` (h4h_step), the first exchange and the
+// sums; the last workgroup to leave clears what was published, takes the next
+// time from the block minima and writes the result (a third exchange took 2 us
+// more of 23).
+template <bool MIXED, uint32_t TPW, bool ONE>
 __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t max_run,
                                                  double e2, double eta, double dt_min,
                                                  double dt_max, OneStep one) {
 #pragma clang fp contract(off)
-    constexpr uint32_t RED = 25 * TM_ACT;  // a tile's sums: 24 doubles per slot of <= 133
+    constexpr uint32_t TM_ACT = ONE ? ONE_ACT : team_act(TPW);
+    constexpr uint32_t RED = 25 * TM_ACT;  // a tile's sums: 24 doubles per slot (<= 133 or 256)
     __shared__ double4 tile[TPW][2 * JT];  // predictor records
     __shared__ __align__(16) double red[TPW * RED];  // pair sums; then fs, outs
     __shared__ double hw[8 * TEAM_WGS];    // headers, word by word
@@ -2625,7 +2635,8 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     if (tid <= TM_ACT) plans[tid] = tm.plan[tid];
     ClState *cs = e.cs;
     RunCtl *ctl = e.ctl;
-    const bool loop = one.host == nullptr, pend = loop && cs->tail_pend != 0;
+    constexpr bool loop = !ONE;
+    const bool pend = loop && cs->tail_pend != 0;
     const double Tp = cs->tail_t, atime = loop ? cs->atime : one.itime;
     const uint32_t np_tail = cs->tail_nact;
     unsigned long long steps = !loop ? 0ull : pend ? cs->tail_steps + 1 : cs->steps;
@@ -2678,6 +2689,18 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     const bool vel = (lane & 4u) != 0;
     const uint32_t cc = min(lane & 3u, 2u), cq = cc + (vel ? 3u : 0u);
     double st_o[6], st_a[6];  // of the step before, stored while waiting
+    auto store_state = [&] {
+        if (!act) return;
+        const size_t np = (size_t)tiles * JT;  // the state's columns are np apart
+        auto *col = in_loop(s.r[0]) + i;
+        for (int k = 0; k < 3; ++k) col[(COL_R + k) * np] = r[k];
+        for (int k = 0; k < 3; ++k) col[(COL_R + 4 + k) * np] = v[k];
+        for (int k = 0; k < 6; ++k) col[(COL_F + k) * np] = f[k];
+        for (int k = 0; k < 6; ++k) col[(COL_OLD + k) * np] = st_o[k];
+        for (int k = 0; k < 6; ++k) col[(COL_A2 + k) * np] = st_a[k];
+        col[COL_T * np] = ti;
+        col[COL_DT * np] = dti;
+    };
     for (;;) {
         // (1) The next time of this workgroup's particles, and those that
         // have it.  (A wave whose minimum is within the selection's tolerance
@@ -2705,7 +2728,7 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
         }
         const bool cand = w < OW && wmn[w] == t_own && ((mask >> lane) & 1ull);
         unsigned long long *hd = tm.hdr + ((size_t)slot * M + b) * 8;
-        if (cand && rank < TM_ACT) {
+        if (cand && rank < TM_ACT && (loop || rank == 0 || t_own == T)) {
             double4 pa, pb;
             predict_vals(r, v, f, t_own - ti, mf, pa, pb);
             unsigned long long *o =
@@ -2728,17 +2751,7 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             agent_store(hd, bits((double)INFINITY));
         }
         // The step before's state, to HBM while the others publish.
-        if (act) {
-            const size_t np = (size_t)tiles * JT;  // the state's columns are np apart
-            auto *col = in_loop(s.r[0]) + i;
-            for (int k = 0; k < 3; ++k) col[(COL_R + k) * np] = r[k];
-            for (int k = 0; k < 3; ++k) col[(COL_R + 4 + k) * np] = v[k];
-            for (int k = 0; k < 6; ++k) col[(COL_F + k) * np] = f[k];
-            for (int k = 0; k < 6; ++k) col[(COL_OLD + k) * np] = st_o[k];
-            for (int k = 0; k < 6; ++k) col[(COL_A2 + k) * np] = st_a[k];
-            col[COL_T * np] = ti;
-            col[COL_DT * np] = dti;
-        }
+        if (loop) store_state();
         // All workgroups'.
         for (uint32_t k = tid; k < 8 * M; k += TB) {
             const unsigned long long u =
@@ -2985,6 +2998,11 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
         }
         t_last = T;
         ++it;
+        if (!loop) {
+            nst = nact;
+            store_state();
+            break;
+        }
         slot = slot == 2 ? 0u : slot + 1u;
     }
     // Loop state, predictor records of the last step, block minima.
@@ -3024,14 +3042,20 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             for (uint32_t k = 0; k < BS / 64; ++k)
                 at += wmn[w0 + k] == m ? wct[w0 + k]
                       : fabs(m - wmn[w0 + k]) < 2 * DBL_EPSILON ? BCNT_MANY : 0u;
-            e.bmin[b * TPW + tid] = m;
-            e.bcnt[b * TPW + tid] = at;
+            if (loop) {
+                e.bmin[b * TPW + tid] = m;
+                e.bcnt[b * TPW + tid] = at;
+            } else {  // (read by the last one out)
+                agent_store(reinterpret_cast<unsigned long long *>(e.bmin) + b * TPW + tid, bits(m));
+                agent_store(e.bcnt + b * TPW + tid, at);
+            }
         }
     }
     // This workgroup's further records of the last exchange (nobody reads
     // them), and its header if no team formed.
     unsigned long long *rc = tm.rec + ((size_t)slot * M + b) * TM_ACT * 8;
-    for (uint32_t k = 8 + tid; k < 8 * min(cnt, TM_ACT); k += TB) agent_store(rc + k, SENT);
+    if (loop || !it)
+        for (uint32_t k = 8 + tid; k < 8 * min(cnt, TM_ACT); k += TB) agent_store(rc + k, SENT);
     if (!go && tid < 8) agent_store(tm.hdr + (size_t)b * 8 + tid, SENT);
     if (go && s_bad && tid == 0) agent_store(&ctl->team_err, 1u);
     wait_memory();
@@ -3049,11 +3073,32 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
         agent_store(&tm.sync[TS_DECISION], 0u);
         agent_store(&tm.sync[TS_LEFT], 0u);
     }
-    if (loop || tid) return;
+    if (loop) return;
+    double x = INFINITY, mn = INFINITY;
+    uint32_t xc = 0;
+    if (it > 0) {
+        for (uint32_t k = tid; k < 8 * nact; k += TB)  // the active particles' records
+            if (const uint32_t l = lst[k / 8] >> 16)
+                agent_store(tm.rec + ((size_t)(lst[k / 8] & 0xffffu) * TM_ACT + l) * 8 + k % 8, SENT);
+        if (tid < tiles) {
+            x = from_bits(agent_load(reinterpret_cast<unsigned long long *>(e.bmin) + tid));
+            xc = min(agent_load(e.bcnt + tid), BCNT_MANY);
+        }
+        const double m = wave_min(x);
+        if (lane == 0) wmn[w] = m;
+        if (tid == 0) lact[0] = 0;
+        __syncthreads();
+        for (uint32_t k = 0; k < TB / 64; ++k) mn = vmin(mn, wmn[k]);
+        if (x != mn) xc = fabs(mn - x) < 2 * DBL_EPSILON ? BCNT_MANY : 0u;
+        if (xc) atomicAdd(&lact[0], xc);
+    }
+    wait_memory();
+    __syncthreads();
+    if (tid) return;
     if (agent_load(&ctl->team_err))
         host_store(&one.host->done, (uint32_t)STEP_FAILED);
     else if (it > 0)
-        step_result(one.host, T, (uint32_t)nst, n, 0, nact);
+        step_result(one.host, mn, (uint32_t)nst, n, 0, lact[0]);
     else
         host_store(&one.host->done, (uint32_t)STEP_LEFT);
 }
@@ -3388,22 +3433,27 @@ void drop_graph(h4h_ctx *ctx) {
 // exchange.  More: a tile per workgroup would not leave every workgroup a CU.
 bool team_size(const h4h_ctx *ctx) { return ctx->K == 1 && ctx->nblk > 4 && ctx->nblk <= TEAM_TILES; }
 
+uint32_t team_act(const h4h_ctx *ctx) { return team_act(ctx->nblk > TEAM_ONE ? 2u : 1u); }
+
 // The plans of the active counts a team takes (0: not one chunk per tile,
 // or a tuning table is set).
 int configure_team(h4h_ctx *ctx) {
     if (!ctx->team_ok) return H4H_OK;
-    for (uint32_t k = 0; k <= TM_ACT; ++k) {
+    for (uint32_t k = 0; k <= team_act(ctx); ++k) {
         uint32_t plan = 0;
         if (k >= 1 && k <= ctx->n && !ctx->e.tuned) {
-            const uint32_t iw = pick_iw(k, ctx->iw_fill);
-            const Decomp d = decompose(k, iw, ctx->nblk, ctx->e.grid, ctx->max_split);
-            if (iw <= 64 && d.S == ctx->nblk)
-                plan = (uint32_t)__builtin_ctz(iw) | (uint32_t)__builtin_ctz(finish_lanes(d.S, k)) << 16;
+            const LaneGroup lg = lane_group(k, ctx->iw_fill, std::min(ctx->nblk, ctx->max_split),
+                                            ctx->precision == H4H_MIXED);
+            const Decomp d = decompose(k, lg.iw, ctx->nblk, ctx->e.grid, ctx->max_split);
+            if (lg.iw <= 64 && !lg.jrun && d.S == ctx->nblk)
+                plan = (uint32_t)__builtin_ctz(lg.iw) |
+                       (uint32_t)__builtin_ctz(finish_lanes(d.S, k)) << 16;
         }
         ctx->team_plan_host[k] = plan;
     }
     H4H_HIP(hipMemcpyAsync(const_cast<uint32_t *>(ctx->team.plan), ctx->team_plan_host,
-                           (TM_ACT + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+                           (team_act(ctx) + 1) * sizeof(uint32_t), hipMemcpyHostToDevice,
+                           ctx->stream));
     return H4H_OK;
 }
 
@@ -3537,8 +3587,11 @@ bool team_path(const h4h_ctx *ctx) {
 
 int launch_team(h4h_ctx *ctx, uint32_t max_run, OneStep one = {}) {
     const bool two = ctx->nblk > TEAM_ONE, mixed = ctx->precision == H4H_MIXED;
-    auto *kern = two ? (mixed ? k_team_run<true, 2> : k_team_run<false, 2>)
-                     : (mixed ? k_team_run<true, 1> : k_team_run<false, 1>);
+    auto *kern = one.host
+                     ? (two ? (mixed ? k_team_run<true, 2, true> : k_team_run<false, 2, true>)
+                            : (mixed ? k_team_run<true, 1, true> : k_team_run<false, 1, true>))
+                     : (two ? (mixed ? k_team_run<true, 2, false> : k_team_run<false, 2, false>)
+                            : (mixed ? k_team_run<true, 1, false> : k_team_run<false, 1, false>));
     hipLaunchKernelGGL(kern, dim3(two ? (ctx->nblk + 1) / 2 : ctx->nblk), dim3(TB), 0, ctx->stream,
                        ctx->s, ctx->e, ctx->team, max_run, ctx->e2, (double)ctx->eta, ctx->dt_min,
                        ctx->dt_max, one);
@@ -3904,9 +3957,9 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     size_t np = ctx->n_dev;
     ctx->team_ok = team_size(ctx);
     const size_t tm_hdr = 3 * (size_t)ctx->nblk * 8,
-                 tm_rec = 3 * (size_t)ctx->nblk * 8 * TM_ACT,
-                 tm_part = (size_t)ctx->nblk * TM_ACT * 6, tm_words = tm_hdr + tm_rec + tm_part,
-                 tm_plan = TS_WORDS + TM_ACT + 2;  // u32
+                 tm_rec = 3 * (size_t)ctx->nblk * 8 * team_act(ctx),
+                 tm_part = (size_t)ctx->nblk * team_act(ctx) * 6, tm_words = tm_hdr + tm_rec + tm_part,
+                 tm_plan = TS_WORDS + team_act(ctx) + 2;  // u32
     const size_t team_bytes =
         ctx->team_ok ? tm_words * sizeof(double) + tm_plan * sizeof(uint32_t) : 0;
     // One device allocation for everything but the partials (17 of them took
@@ -3949,7 +4002,7 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     // One pinned allocation for all host mirrors (each costs ~0.2 ms).
     static_assert(sizeof(RunCtl) % 8 == 0 && sizeof(ClState) % 8 == 0, "carved in doubles");
     const size_t eo = eout_len(ctx) * 4, ct = sizeof(RunCtl) / 8, cst = K * sizeof(ClState) / 8;
-    const size_t pl = TM_ACT / 2 + 1;
+    const size_t pl = team_act(ctx) / 2 + 1;
     if (hipHostMalloc(&ctx->pinned, (eo + ct + cst + HIST_CAP + HIST_CAP / 2 + pl) * sizeof(double),
                       hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(H4H_ENOMEM, "pinned allocation failed"));
@@ -4302,9 +4355,10 @@ int h4h_set_precision(h4h_ctx *ctx, int precision) {
     int rc = check_ctx(ctx, false);
     if (rc) return rc;
     if (!valid_precision(precision)) return fail(H4H_EINVAL, "unknown precision");
-    if (precision != ctx->precision) drop_graph(ctx);
+    if (precision == ctx->precision) return H4H_OK;
+    drop_graph(ctx);
     ctx->precision = precision;
-    return H4H_OK;
+    return configure_team(ctx);
 }
 
 int h4h_set_launch(h4h_ctx *ctx, uint32_t workgroups, uint32_t max_jsplit) {
@@ -4632,7 +4686,7 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     // (18 us of 50).
     const bool small = small_path(ctx);
     const bool large = ctx->bm_valid && itime == ctx->next_time && ctx->next_nact < BCNT_MANY &&
-                       ctx->next_nact > (small ? std::min(ctx->small_act, SMALL_MAX_ACT) : TM_ACT);
+                       ctx->next_nact > (small ? std::min(ctx->small_act, SMALL_MAX_ACT) : ONE_ACT);
     ctx->next_nact = 0;
     if ((rc = ensure_blockmin(ctx))) return rc;
     if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
