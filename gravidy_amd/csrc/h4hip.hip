@@ -2688,7 +2688,9 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     // corrector lanes
     const bool vel = (lane & 4u) != 0;
     const uint32_t cc = min(lane & 3u, 2u), cq = cc + (vel ? 3u : 0u);
-    double st_o[6], st_a[6];  // of the step before, stored while waiting
+    // The state after a step, while the others publish: the old forces and
+    // the derivatives are still in stg and outs (place `was` of the list).
+    uint32_t was = 0;
     auto store_state = [&] {
         if (!act) return;
         const size_t np = (size_t)tiles * JT;  // the state's columns are np apart
@@ -2696,8 +2698,8 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
         for (int k = 0; k < 3; ++k) col[(COL_R + k) * np] = r[k];
         for (int k = 0; k < 3; ++k) col[(COL_R + 4 + k) * np] = v[k];
         for (int k = 0; k < 6; ++k) col[(COL_F + k) * np] = f[k];
-        for (int k = 0; k < 6; ++k) col[(COL_OLD + k) * np] = st_o[k];
-        for (int k = 0; k < 6; ++k) col[(COL_A2 + k) * np] = st_a[k];
+        for (int k = 0; k < 6; ++k) col[(COL_OLD + k) * np] = stg[7 * was + k];
+        for (int k = 0; k < 6; ++k) col[(COL_A2 + k) * np] = outs[19 * was + 13 + k];
         col[COL_T * np] = ti;
         col[COL_DT * np] = dti;
     };
@@ -2982,11 +2984,8 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             __syncthreads();
             if (act) {
                 const double *o = outs + 19 * rank;
-                for (int q = 0; q < 6; ++q) {
-                    st_o[q] = f[q];
-                    f[q] = o[q];
-                    st_a[q] = o[13 + q];
-                }
+                was = rank;
+                for (int q = 0; q < 6; ++q) f[q] = o[q];
                 for (int q = 0; q < 3; ++q) {
                     r[q] = o[6 + q];
                     v[q] = o[9 + q];
