@@ -1853,11 +1853,13 @@ __device__ __forceinline__ void step_result(ClState *host, double atime, uint32_
 
 // The loop tail a single system's last block step left (k_finish_blocks),
 // when no further step of the loop makes it: after one h4h_step, whose
-// result goes to the pinned record `host`.
+// result goes to the pinned record `host`, or at the end of a loop's step
+// budget (null; the loop may have stopped before).
 __global__ __launch_bounds__(BS) void k_tail(Ens e, ClState *host) {
     __shared__ double red[BS / 64];
     __shared__ uint32_t next;
     ClState *cs = &e.cs[0];
+    if (!host && cs->done) return;
     double mn = INFINITY;
     for (uint32_t b = threadIdx.x; b < e.nblk; b += BS) mn = fmin(mn, e.bmin[b]);
     mn = block_min(mn, red);
@@ -1874,7 +1876,7 @@ __global__ __launch_bounds__(BS) void k_tail(Ens e, ClState *host) {
         record_tail(e, 0, cs->tail_t, cs->tail_nact, steps, mn,
                     loop_stops(*e.ctl, cs->tail_t, steps, mn));
         cs->tail_pend = 0;
-        step_result(host, mn, cs->tail_nact, e.cnt[0], 0, next);
+        if (host) step_result(host, mn, cs->tail_nact, e.cnt[0], 0, next);
     }
 }
 
@@ -4736,13 +4738,24 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
 // stopped; copies cluster 0's per-step history when asked.
 static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint64_t cap) {
     ctx->next_nact = 0;
-    int rc = ctx->graphs ? ensure_graph(ctx) : H4H_OK;
-    if (rc) return rc;
-    uint64_t seen = 0;
+    int rc = H4H_OK;
+    uint64_t seen = 0, made = 0;  // steps copied out, steps made
+    const bool plain = ctx->K == 1 && !small_path(ctx) && !team_path(ctx);
     bool hist = (step_time || step_nact) && ctx->K == 1;
     if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
     for (;;) {
-        if (ctx->graphs) {
+        if (plain && made < cap && cap - made <= RUN_CHUNK) {
+            // the last steps of the budget, and their loop tail: a chunk's
+            // steps beyond it are three empty launches each (a run that ends
+            // with a chunk needed another one of 32 for its last loop tail:
+            // 0.18 ms)
+            for (uint64_t k = 0; k < cap - made; ++k)
+                if ((rc = enqueue_step(ctx, false, k & 1))) return rc;
+            hipLaunchKernelGGL(k_tail, dim3(1), dim3(BS), 0, ctx->stream, ctx->e,
+                               (ClState *)nullptr);
+            H4H_LAUNCHED();
+        } else if (ctx->graphs) {
+            if ((rc = ensure_graph(ctx))) return rc;
             H4H_HIP(hipGraphLaunch(ctx->graph_exec, ctx->stream));
         } else if ((rc = enqueue_chunk(ctx))) {
             return rc;
@@ -4759,6 +4772,7 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
             }
             seen = steps;
         }
+        made = ctx->cs_host[0].steps + (ctx->cs_host[0].tail_pend ? 1 : 0);
         if (ctx->ctl_host->ndone >= ctx->K) break;
     }
     if (ctx->timing) {
