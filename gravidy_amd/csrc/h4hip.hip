@@ -2241,10 +2241,18 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
                 // groups in order: 8 (P < 64), else 1024 / P = 16, 8 or 4
                 double fq = 0.0;
                 const double *rk = red + k * 6 + cq;
-                const uint32_t ngrp = P < 64 ? SW : SN >> lp;
-                for (uint32_t q0 = 0; q0 < ngrp; q0 += 4) {
+                if (P < 64) {
+                    double x8[SW];  // (all loads under way before the first sum)
 #pragma unroll
-                    for (uint32_t q = 0; q < 4; ++q) fq += rk[(q0 + q) * P * 6];
+                    for (uint32_t q = 0; q < SW; ++q) x8[q] = rk[q * P * 6];
+#pragma unroll
+                    for (uint32_t q = 0; q < SW; ++q) fq += x8[q];
+                } else {
+                    const uint32_t ngrp = SN >> lp;
+                    for (uint32_t q0 = 0; q0 < ngrp; q0 += 4) {
+#pragma unroll
+                        for (uint32_t q = 0; q < 4; ++q) fq += rk[(q0 + q) * P * 6];
+                    }
                 }
                 if (!MIXED) fq *= PAIR_SCALE;
                 const double fx = xor4(fq);
@@ -2278,6 +2286,12 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
                 rest_min(k * SW + w, act[k] ? (double)INFINITY : tdt[k]);
         __syncthreads();
 
+        // (what the next time needs is read before the owners' state, so that
+        // the reads' latencies overlap)
+        const double wv = wmin[lane % SC];
+        const uint32_t wc = (uint32_t)__popcll(wmask[lane % SC]);
+        const double x = lane < nact && nact <= 64 ? T + outs[13 * min(lane, nact - 1) + 12]
+                                                   : (double)INFINITY;
         // The owners take their corrected state.
 #pragma unroll
         for (uint32_t k = 0; k < SP; ++k)
@@ -2302,10 +2316,6 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
         bool close;
         uint32_t cnt = 0;
         if (nact <= 64) {
-            const double wv = wmin[lane % SC];
-            const uint32_t wc = (uint32_t)__popcll(wmask[lane % SC]);
-            const double x = lane < nact ? T + outs[13 * min(lane, nact - 1) + 12]
-                                         : (double)INFINITY;
             mn = wave_min(vmin(x, wv));
             close = __ballot((wv != mn && fabs(mn - wv) < 2 * DBL_EPSILON) ||
                              (x != mn && fabs(mn - x) < 2 * DBL_EPSILON)) != 0;
