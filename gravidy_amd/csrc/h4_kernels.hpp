@@ -145,7 +145,7 @@ struct Ens {
                              // place in the cluster's active list, count), by step
                              // parity (the step's slot in its captured chunk, mod 2)
     double *bmin;            // [nblk] min(t + dt) per block
-    uint32_t *bcnt;          // [nblk] particles that have it (single system, BCNT_MANY:
+    uint32_t *bcnt;          // [nblk] particles that have it (BCNT_MANY or more:
                              // not known)
     double4 *arec;           // [4][nblk * JT] the step's active particles in the order
                              // of the active list (index off[c] + k): predictor
