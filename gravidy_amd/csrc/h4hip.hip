@@ -3321,15 +3321,18 @@ static_assert(HIST_CAP >= RUN_CHUNK && HIST_CAP >= SMALL_SLOTS * (SMALL_RUN + 1)
               "history ring shorter than the steps of one graph");
 constexpr int N_SOA = 35;           // doubles per particle in `state`
 
-// Downloads of DL_MIN doubles or more (4 MB) go through pinned slots, written
-// by k_rows_out over the bus and copied to the caller's arrays by DL_THREADS
-// threads with two slots each.  One thread's copies and its page faults on
-// arrays not touched before take longer than the bus: 28 doubles of 262144
-// particles 8.1 -> 2.2 ms into new arrays, 3.4 -> 1.5 ms into used ones;
-// 2 threads 3.2 and 1.7, 8 threads 1.8 and 1.7.  Slots of 256 KB: 2.7 ms.
-// Below 4 MB the gain is less than the slots' allocation (0.5 ms).
+// Downloads go through pinned slots, written by k_rows_out over the bus and
+// copied to the caller's arrays by the calling thread and, for more than a few
+// pieces, others, two slots each.  From DL_MIN doubles (4 MB): 4 threads and
+// 512 KB slots, as one thread's copies and its page faults on arrays not
+// touched before take longer than the bus: 28 doubles of 262144 particles 8.1
+// -> 3.9 ms into new arrays, 3.4 -> 1.8 ms into used ones (the pieces alone: 2
+// threads 3.2 and 1.7 ms, 4 2.4 and 1.6, 8 1.8 and 1.7; slots of 256 KB: 2.7).
+// Below: 2 threads at most and 256 KB slots, 1 MB in all, which is had in 15 to
+// 40 us (2 MB: 270); a gather, a copy and a wait per array took 0.30 ms at n =
+// 1024 and 0.67 at n = 4096.
 constexpr uint32_t DL_THREADS = 4, DL_SLOTS = 2 * DL_THREADS;
-constexpr uint32_t DL_SLOT = 1u << 16;   // doubles
+constexpr uint32_t DL_SLOT = 1u << 16, DL_SLOT_SMALL = 1u << 15;  // doubles
 constexpr size_t DL_MIN = 8 * (size_t)DL_SLOT;
 }  // namespace
 
@@ -3388,8 +3391,8 @@ struct h4h_ctx {
     hipGraphExec_t graph_exec = nullptr;
     bool graphs = true;          // device loops replay captured chunks
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    double *dl_pin = nullptr;    // pinned slots of large downloads (download_rows), made by the
-                                 // first one
+    double *dl_pin = nullptr;    // pinned slots of downloads (download_rows), made by the first
+    size_t dl_len = 0;           // one that needs them: doubles
     hipEvent_t dl_ev[DL_SLOTS] = {};
     Soa s{};
     Ens e{};
@@ -3757,17 +3760,22 @@ int download_cols(h4h_ctx *ctx, double *dst, uint32_t ncols, Cols src) {
     return H4H_OK;
 }
 
-// The slots of download_rows; false: not to be had, with the error cleared.
-bool make_slots(h4h_ctx *ctx) {
-    if (ctx->dl_pin) return true;
-    for (hipEvent_t &ev : ctx->dl_ev)
+// `slots` slots of `len` doubles; false: not to be had, with the error cleared.
+bool make_slots(h4h_ctx *ctx, uint32_t slots, size_t len) {
+    for (uint32_t k = 0; k < slots; ++k) {
+        hipEvent_t &ev = ctx->dl_ev[k];
         if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
             ev = nullptr;
             (void)hipGetLastError();
             return false;
         }
-    if (hipHostMalloc((void **)&ctx->dl_pin, (size_t)DL_SLOTS * DL_SLOT * sizeof(double)) != hipSuccess) {
+    }
+    if (ctx->dl_len >= slots * len) return true;
+    if (ctx->dl_pin) (void)hipHostFree(ctx->dl_pin);  // (no download is under way)
+    ctx->dl_len = slots * len;
+    if (hipHostMalloc((void **)&ctx->dl_pin, ctx->dl_len * sizeof(double)) != hipSuccess) {
         ctx->dl_pin = nullptr;
+        ctx->dl_len = 0;
         (void)hipGetLastError();
         return false;
     }
@@ -3778,15 +3786,16 @@ bool make_slots(h4h_ctx *ctx) {
 // thread takes the next piece that nobody has, has the device write it, and
 // copies it on while the device writes its other slot.  The caller is one of
 // the threads, so that the call ends without the others too.
-int download_rows(h4h_ctx *ctx, const RowArrays &t, double *const *dst) {
-    const unsigned long long total = t.at[t.n], pieces = (total + DL_SLOT - 1) / DL_SLOT;
+int download_rows(h4h_ctx *ctx, const RowArrays &t, double *const *dst, uint32_t threads,
+                  uint32_t size) {
+    const unsigned long long total = t.at[t.n], pieces = (total + size - 1) / size;
     std::atomic<unsigned long long> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](uint32_t w) {
         unsigned long long piece[2];
-        auto slot = [&](uint32_t k) { return ctx->dl_pin + (size_t)(2 * w + k) * DL_SLOT; };
+        auto slot = [&](uint32_t k) { return ctx->dl_pin + (size_t)(2 * w + k) * size; };
         auto length = [&](unsigned long long p) {
-            return (uint32_t)std::min<unsigned long long>(DL_SLOT, total - p * DL_SLOT);
+            return (uint32_t)std::min<unsigned long long>(size, total - p * size);
         };
         auto check = [&](hipError_t rc) {
             if (rc != hipSuccess) err = (int)rc;
@@ -3797,7 +3806,7 @@ int download_rows(h4h_ctx *ctx, const RowArrays &t, double *const *dst) {
             if (piece[k] >= pieces) return;
             const uint32_t len = length(piece[k]);
             hipLaunchKernelGGL(k_rows_out, dim3(blocks_for(len)), dim3(BS), 0, ctx->stream,
-                               ctx->s.r[0], t, ctx->e, piece[k] * DL_SLOT, len, slot(k));
+                               ctx->s.r[0], t, ctx->e, piece[k] * size, len, slot(k));
             check(hipGetLastError());
             check(hipEventRecord(ctx->dl_ev[2 * w + k], ctx->stream));
         };
@@ -3806,7 +3815,7 @@ int download_rows(h4h_ctx *ctx, const RowArrays &t, double *const *dst) {
         issue(1);
         for (uint32_t k = 0; piece[k] < pieces; k ^= 1) {
             if (!check(hipEventSynchronize(ctx->dl_ev[2 * w + k])) || err != (int)hipSuccess) return;
-            const unsigned long long b = piece[k] * DL_SLOT, end = b + length(piece[k]);
+            const unsigned long long b = piece[k] * size, end = b + length(piece[k]);
             for (uint32_t a = 0; a < t.n; ++a) {
                 const unsigned long long lo = std::max(b, t.at[a]), hi = std::min(end, t.at[a + 1]);
                 if (lo < hi)
@@ -3815,7 +3824,6 @@ int download_rows(h4h_ctx *ctx, const RowArrays &t, double *const *dst) {
             issue(k);
         }
     };
-    const uint32_t threads = std::min(DL_THREADS, std::max(1u, std::thread::hardware_concurrency()));
     std::thread th[DL_THREADS];
     try {
         for (uint32_t w = 1; w < threads; ++w) th[w] = std::thread(work, w);
@@ -4448,12 +4456,17 @@ int h4h_download(h4h_ctx *ctx, double *r4, double *v4, double *f6, double *time,
     rows(a3, 3, COL_A3, NO_COL);
     rows(time, 1, COL_T, NO_COL);
     rows(dt, 1, COL_DT, NO_COL);
-    if (t.at[t.n] >= DL_MIN) {
+    if (t.at[t.n]) {
         int current = 0;  // the slots' events are of the context's device
         H4H_HIP(hipGetDevice(&current));
         if (current != ctx->device) H4H_HIP(hipSetDevice(ctx->device));
-        const bool slots = make_slots(ctx);
-        rc = slots ? download_rows(ctx, t, to) : H4H_OK;
+        const bool large = t.at[t.n] >= DL_MIN;
+        const uint32_t size = large ? DL_SLOT : DL_SLOT_SMALL;
+        const uint32_t threads =
+            std::min({large ? DL_THREADS : 2u, (uint32_t)(t.at[t.n] / (2 * (size_t)size)) + 1u,
+                      std::max(1u, std::thread::hardware_concurrency())});
+        const bool slots = make_slots(ctx, 2 * threads, size);
+        rc = slots ? download_rows(ctx, t, to, threads, size) : H4H_OK;
         if (current != ctx->device) H4H_HIP(hipSetDevice(current));
         if (slots) return rc;
     }

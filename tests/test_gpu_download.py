@@ -1,8 +1,8 @@
-"""h4h_download of 4 MB or more (written by the device into pinned slots and
-copied on by several threads) against the arrays downloaded one at a time and
-against what was uploaded, bit for bit: one double below and above the
-threshold, pieces that end inside an array, a ragged last piece, clusters
-back to back."""
+"""h4h_download (written by the device into pinned slots and copied on by one
+or more threads) against the arrays downloaded one at a time and against what
+was uploaded, bit for bit: one double below and above the 4 MB of larger slots
+and more threads, pieces that end inside an array, a ragged last piece,
+clusters back to back."""
 import ctypes
 
 import numpy as np
@@ -49,6 +49,20 @@ def test_large_download(n):
         v4[:, 3] = 0.0
         check(h, n, {"r": r, "v": v4, "f": f, "t": t, "dt": dt})
         h.step(2.0 ** -7)  # old, a2, a3 of the active particles
+        check(h, n, {})
+
+
+# one piece, a piece more than one and two (32768 doubles), the second thread's
+@pytest.mark.parametrize("n", [1, 2, 300, 1170, 1171, 2340, 2341, 9000])
+def test_small_download(n):
+    r, v = ic.plummer(n, n)
+    f = np.random.default_rng(n).normal(size=(n, 6))
+    t = np.zeros(n)
+    dt = np.full(n, 2.0 ** -5)
+    with Hermite4HIP(r, v, E2) as h:
+        h.upload(r, v, f, t, dt)
+        check(h, n, {"r": r, "f": f, "t": t, "dt": dt})
+        h.step(2.0 ** -5)
         check(h, n, {})
 
 
