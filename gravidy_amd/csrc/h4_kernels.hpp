@@ -305,7 +305,8 @@ __host__ __device__ inline uint32_t pick_iw(uint32_t nact, uint32_t fill16 = DEF
 //   n = 65536, nact 1500: 127 | 164 | 147  n = 20000, nact 4000: 105 | 108 | 111
 // The lines: 1024 items of 256 slots (4 per CU), 512 of 64 slots.
 // nact <= NARROW_ACT keeps pick_iw's width: those steps are k_small_run's and
-// k_team_run's, whose workgroups keep their j and gain nothing.
+// k_team_run's (which takes larger ones too, at the width they have here), whose
+// workgroups keep their j and gain nothing.
 // Mixed precision narrows to 64 only (n = 4096, nact 1000: 33 -> 13 us), with
 // jrun = 1: each j sub-group then takes 64 consecutive j, so that the FP32
 // runs are the 32 consecutive pairs that 256 slots sum; with 16 slots they

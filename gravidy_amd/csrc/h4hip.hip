@@ -2577,8 +2577,8 @@ __device__ __forceinline__ void team_item(uint32_t it, uint32_t t, uint32_t nact
 // What bounds a step is the chain from one next time to the next on a
 // workgroup that owns an active particle, two exchanges of 2-3 us each in it;
 // about 7.5 us at 16 and 40 tiles, 10 us at 256.  Average block steps of runs
-// (start to several hundred steps, all active sets): N = 4096 21.5 -> 12.2 us,
-// 10007 26.0 -> 17.8, 20000 33.0 -> 24.8, 65536 46.0 -> 39.2.  Up to TEAM_ONE
+// (start to several hundred steps, all active sets): N = 4096 21.5 -> 10.9 us,
+// 10007 26.0 -> 15.3, 65536 46.0 -> 37.6.  Up to TEAM_ONE
 // tiles a workgroup has one, its two groups of BS threads take turns at the
 // i tiles (N = 20000: 24.8 us, 27.1 with two tiles each); beyond, two, as 256
 // workgroups exchange more slowly than 128.  Steps with more active particles
@@ -4241,8 +4241,8 @@ __global__ __launch_bounds__(BS) void k_static_finish(Soa s, Ens e, const uint32
 // them (a work item of the plan), reads the particles straight from p6 and pm,
 // all tiles at once, and writes its rows, so nothing passes between
 // workgroups.  Same tiles, sub-groups and sums as update_item: the same bits.
-// Bound by its launch and one trip to memory: n = 1024, nact = 24 takes 9.9 us a
-// call in a row (of which 6 the pairs) instead of 22.3 with five launches.
+// Bound by its launch and one trip to memory: n = 1024, nact = 24 takes 10.3 us a
+// call in a row (4 of them issuing the pairs) instead of 22.3 with five launches.
 constexpr uint32_t ONE_TILES = 4;
 template <int IW, bool MIXED>
 __device__ __forceinline__ void static_item(const double *p6, const float *pm, uint32_t n,
