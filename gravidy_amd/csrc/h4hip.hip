@@ -1831,6 +1831,24 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
 // Stores and loads of this wave so far are done.
 __device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// What a step made without a device loop leaves in the cluster's record, as the
+// loop of one step does: later calls start from it (h4h_ensemble_run, its
+// ITIME and ATIME; h4h_correction_pos_vel, the size of the active list).
+// Stored after the result, for which the host waits (before it: 0.4 us more a
+// step): the launches that read it come after this one.
+__device__ __forceinline__ void step_state(ClState *cs, double itime, double atime, uint32_t nact,
+                                           uint32_t n, unsigned long long small) {
+    cs->itime = itime;
+    cs->atime = atime;
+    cs->nact = 0;
+    cs->tail_pend = 0;
+    cs->steps = 1;
+    cs->interactions = (unsigned long long)nact * n;
+    cs->nsteps = nact;
+    cs->small_steps = small;
+    cs->done = 1;
+}
+
 // The result of one h4h_step, to the pinned record the host waits at: its
 // fields, and when they are there `done`.  (Waiting for the launch itself
 // takes 5 us more, of a step of 18 to 28.)  next: the next block step's
@@ -2464,10 +2482,12 @@ __global__ __launch_bounds__(SB) void k_small_run(Soa s, Ens e, uint32_t max_run
     wait_memory();
     __syncthreads();  // the step's stores are done
     if (tid) return;
-    if (it > 0)
+    if (it > 0) {
         step_result(one.host, T, (uint32_t)nst, n, 1, nact);
-    else
+        step_state(cs, one.itime, T, (uint32_t)nst, n, 1);
+    } else {
         host_store(&one.host->done, (uint32_t)STEP_LEFT);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -3108,10 +3128,12 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     if (tid) return;
     if (agent_load(&ctl->team_err))
         host_store(&one.host->done, (uint32_t)STEP_FAILED);
-    else if (it > 0)
+    else if (it > 0) {
         step_result(one.host, mn, (uint32_t)nst, n, 0, lact[0]);
-    else
+        step_state(cs, one.itime, mn, (uint32_t)nst, n, 0);
+    } else {
         host_store(&one.host->done, (uint32_t)STEP_LEFT);
+    }
 }
 
 // Every word of a team's buffers waiting (context creation).
