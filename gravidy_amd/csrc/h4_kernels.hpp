@@ -330,15 +330,43 @@ __host__ __device__ inline LaneGroup lane_group(uint32_t nact, uint32_t fill16, 
     return g;
 }
 
-// Active particles per work item of the exact kernel for nact active ones.
-// Few get a workgroup each: the ordered add chain bounds it (n = 16385:
-// nact 256 88 us, 117 us with 3 per workgroup; both 170 us at 1024).  More
-// share one, 3 chains on one wave and its term waves busier (nact 4096: 391
-// against 631 us).  From EXACT_WIDE on, one lane per particle fills the CUs
-// (n = 65536: 16.0 ms at any nact up to 65536, against 0.356 us times nact).
+// Whether the exact kernel gives every active particle of a launch a lane of
+// its own, or a few of them a workgroup (exact_iw).  Of one system: from
+// EXACT_WIDE active ones on, which fill the CUs (n = 65536: 16.0 ms at any nact
+// up to 65536, against 0.356 us times nact).
 constexpr uint32_t EXACT_WIDE = 45056;
-__host__ __device__ inline uint32_t exact_iw(uint32_t nact) {
-    return nact <= 768 ? 1u : nact < EXACT_WIDE ? 3u : (uint32_t)BS;
+// Of an ensemble's clusters, summed up; all of them the same way, as a lane's
+// chain takes twice as long beside the other kind's workgroups (24 clusters of
+// 500 to 20000: 6.4 ms mixed, 5.4 and 5.7 unmixed).
+struct ExactLoad {
+    double pairs;       // nact n
+    double act;         // nact
+    double lanes;       // nact rounded up to whole workgroups
+    double lane_pairs;  // of those with n
+    double nmax;        // largest n with an active particle
+};
+// Times in us.  A few per workgroup: 1.8e11 pairs/s, 250 more of them per
+// particle for filling and emptying its pipeline.  A lane each: 4.0e11 pairs/s
+// with full CUs, and no less than the chain of the largest cluster, 0.25 us per
+// j with one workgroup on a CU and 0.5 with more of them.  Initial forces, wide
+// and not, us: 64 clusters of 10000 16050 and 35100, of 1000 290 and 475, of
+// 700 205 and 250; 6 of 9000 2270 and 2970; 4 of 3000 760 and 250.
+__host__ __device__ inline bool exact_wide(const ExactLoad &l) {
+    const double few = 5.6e-6 * (l.pairs + 250.0 * l.act);
+    const double per_cu = l.lanes / (256.0 * BS);
+    const double chain = 0.25 * l.nmax * (per_cu < 1.0 ? 1.0 : per_cu > 2.0 ? 2.0 : per_cu);
+    return chain < few && 2.5e-6 * l.lane_pairs < few;
+}
+
+// Active particles per work item of the exact kernel for nact active ones of
+// a cluster; load: the nact of a single system of its size with the pairs of
+// all clusters (sum of nact n over n), so nact itself for one system.  Few get a
+// workgroup each: the ordered add chain bounds it (n = 16385: nact 256 88 us,
+// 117 us with 3 per workgroup; both 170 us at 1024).  More share one, 3 chains
+// on one wave and its term waves busier (nact 4096: 391 against 631 us; initial
+// forces of 64 clusters of 200: 49 against 76 us).
+__host__ __device__ inline uint32_t exact_iw(uint32_t nact, double load, bool wide) {
+    return wide ? (uint32_t)BS : load <= 768.0 || nact <= 1 ? 1u : 3u;
 }
 
 // Work items of the energy of n particles: i blocks of ENERGY_I particles
@@ -370,6 +398,58 @@ __host__ __device__ inline EnergyItems energy_items(uint32_t n) {
             : e.items >= 512            ? (uint32_t)(e.items / 2)
                                         : (uint32_t)(e.items < 256 ? e.items : 256);
     return e;
+}
+
+// j tiles of cluster c.
+__host__ __device__ __forceinline__ uint32_t ntiles(const Ens &e, uint32_t c) {
+    return (e.cnt[c] + JT - 1) / JT;
+}
+
+// Work plan of cluster c for nact active particles; W = sum over the
+// clusters of nact * n (the update workgroups are shared in proportion);
+// wide: of an exact plan, exact_wide.
+__host__ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_t nact,
+                                                        double W, bool exact, bool mixed,
+                                                        bool wide) {
+    ClPlan pl;
+    pl.cmaj = pl.jrun = 0;
+    if (exact) {
+        pl.iw = exact_iw(nact, e.K == 1 ? (double)nact : W / (double)e.cnt[c], wide);
+        pl.S = 1;
+        pl.tpc = ntiles(e, c);
+        pl.n_it = (nact + pl.iw - 1) / pl.iw;
+        pl.rows = pl.n_it * pl.iw;
+        pl.lanes = 1;
+        pl.grid = e.grid;
+    } else {
+        double share = W > 0.0 ? (double)nact * (double)e.cnt[c] / W : 0.0;
+        uint32_t g = (uint32_t)(share * e.grid);
+        pl.grid = g < 1 ? 1 : g;
+        pl.iw = pick_iw(nact ? nact : 1, e.iw_fill);
+        const uint32_t nt = ntiles(e, c);
+        if (e.K == 1 || nt > 4) {
+            const LaneGroup lg = lane_group(nact, e.iw_fill, nt < e.max_split ? nt : e.max_split,
+                                            mixed, e.K == 1 ? 1.0 : share);
+            pl.iw = lg.iw;
+            pl.jrun = lg.jrun;
+        }
+        if (e.tuned && e.K == 1 && nact) {
+            uint32_t bucket = 31u - (uint32_t)__builtin_clz(nact);
+            if (e.tune[bucket]) pl.grid = e.tune[bucket] < e.grid ? e.tune[bucket] : e.grid;
+            if (e.tune[32 + bucket]) {
+                pl.iw = e.tune[32 + bucket];
+                pl.jrun = 0;
+            }
+        }
+        Decomp d = decompose(nact, pl.iw, nt, pl.grid, e.max_split, e.K > 1);
+        pl.S = d.S;
+        pl.tpc = d.tiles_per_chunk;
+        pl.n_it = d.n_it;
+        pl.rows = d.rows;
+        pl.lanes = finish_lanes(d.S, nact);
+        pl.cmaj = (d.S > 1 && pl.lanes >= 16 && d.rows >= 64) ? 1u : 0u;
+    }
+    return pl;
 }
 
 // ---------------------------------------------------------------------------

@@ -76,9 +76,6 @@ constexpr uint32_t ENERGY_OUT = 8 * ENERGY_GRID;  // workgroup sums of one energ
 
 __device__ __forceinline__ uint32_t cluster_of_block(const Ens &e, uint32_t b) { return e.bcl[b]; }
 
-__device__ __forceinline__ uint32_t ntiles(const Ens &e, uint32_t c) {
-    return (e.cnt[c] + JT - 1) / JT;
-}
 
 // Index of the cluster whose [pre[c], pre[c+1]) range holds x (pre has
 // K+1 entries, non-decreasing, pre[0] = 0, x < pre[K]).
@@ -214,145 +211,6 @@ __global__ __launch_bounds__(BS) void k_identity_active(uint32_t *move, Ens e) {
     if (local < e.cnt[c]) move[i] = i;
     if (local == 0) e.cs[c].nact = e.cnt[c];
 }
-
-// ---------------------------------------------------------------------------
-// Work plan of a step (one workgroup)
-// ---------------------------------------------------------------------------
-
-// Per cluster: lane-group width, j split and work items from its active
-// count; the update workgroups are shared in proportion to nact * n.
-// Exclusive prefix sums over clusters go to items_pre / fin_pre /
-// part_pre, totals to ctl.  prec: H4H_FP64_EXACT has no j split.
-// Work plan of cluster c for nact active particles; W = sum over the
-// clusters of nact * n (the update workgroups are shared in proportion).
-__device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c, uint32_t nact, double W,
-                                               int prec) {
-    ClPlan pl;
-    pl.cmaj = pl.jrun = 0;
-    if (prec == H4H_FP64_EXACT) {
-        pl.iw = exact_iw(nact);
-        pl.S = 1;
-        pl.tpc = ntiles(e, c);
-        pl.n_it = (nact + pl.iw - 1) / pl.iw;
-        pl.rows = pl.n_it * pl.iw;
-        pl.lanes = 1;
-        pl.grid = e.grid;
-    } else {
-        double share = W > 0.0 ? (double)nact * (double)e.cnt[c] / W : 0.0;
-        uint32_t g = (uint32_t)(share * e.grid);
-        pl.grid = g < 1 ? 1 : g;
-        pl.iw = pick_iw(nact ? nact : 1, e.iw_fill);
-        if (e.K == 1 || ntiles(e, c) > 4) {
-            const LaneGroup lg = lane_group(nact, e.iw_fill, min(ntiles(e, c), e.max_split),
-                                            prec == H4H_MIXED, e.K == 1 ? 1.0 : share);
-            pl.iw = lg.iw;
-            pl.jrun = lg.jrun;
-        }
-        if (e.tuned && e.K == 1 && nact) {
-            uint32_t bucket = 31u - (uint32_t)__clz(nact);
-            if (e.tune[bucket]) pl.grid = min(e.tune[bucket], e.grid);
-            if (e.tune[32 + bucket]) {
-                pl.iw = e.tune[32 + bucket];
-                pl.jrun = 0;
-            }
-        }
-        Decomp d = decompose(nact, pl.iw, ntiles(e, c), pl.grid, e.max_split, e.K > 1);
-        pl.S = d.S;
-        pl.tpc = d.tiles_per_chunk;
-        pl.n_it = d.n_it;
-        pl.rows = d.rows;
-        pl.lanes = finish_lanes(d.S, nact);
-        pl.cmaj = (d.S > 1 && pl.lanes >= 16 && d.rows >= 64) ? 1u : 0u;
-    }
-    return pl;
-}
-
-// Plan of a single-cluster context, made by every workgroup of the update
-// kernel from the active count (so the device step needs no k_plan
-// launch); workgroup 0 publishes it for the finish pass.
-__device__ __forceinline__ ClPlan plan_single(const Ens &e, int prec,
-                                              unsigned long long &items) {
-    const uint32_t nact = e.cs[0].nact;
-    const ClPlan pl = plan_cluster(e, 0, nact, (double)nact * (double)e.cnt[0], prec);
-    items = nact ? (unsigned long long)pl.n_it * pl.S : 0ull;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const uint32_t per = BS / pl.lanes;
-        const unsigned long long units = (nact + per - 1) / per;
-        e.plan[0] = pl;
-        e.items_pre[0] = e.fin_pre[0] = e.part_pre[0] = 0ull;
-        e.items_pre[1] = items;
-        e.fin_pre[1] = units;
-        e.part_pre[1] = (nact && pl.S > 1) ? 6ull * pl.S * pl.rows : 0ull;
-        e.ctl->items = items;
-        e.ctl->fin_units = units;
-    }
-    return pl;
-}
-
-__device__ void plan_all(const Ens &e, int prec) {
-    __shared__ double wsum[BS / 64];
-    double w = 0.0;
-    for (uint32_t c = threadIdx.x; c < e.K; c += BS)
-        w += (double)e.cs[c].nact * (double)e.cnt[c];
-    for (int o = 32; o > 0; o >>= 1) w += __shfl_xor(w, o);
-    if (__lane_id() == 0) wsum[threadIdx.x >> 6] = w;
-    __syncthreads();
-    double W = 0.0;
-    for (uint32_t k = 0; k < BS / 64; ++k) W += wsum[k];
-    // The plans, and exclusive prefix sums of work items, finish units and
-    // partial doubles over the clusters, BS clusters at a time.
-    __shared__ unsigned long long wtot[3][BS / 64];
-    unsigned long long carry[3] = {0ull, 0ull, 0ull};
-    for (uint32_t base = 0; base < e.K; base += BS) {
-        const uint32_t c = base + threadIdx.x;
-        unsigned long long v[3] = {0ull, 0ull, 0ull};
-        const uint32_t nact = c < e.K ? e.cs[c].nact : 0u;
-        if (nact) {
-            const ClPlan pl = plan_cluster(e, c, nact, W, prec);
-            e.plan[c] = pl;
-            const uint32_t per = BS / pl.lanes;
-            v[0] = (unsigned long long)pl.n_it * pl.S;
-            v[1] = (nact + per - 1) / per;
-            v[2] = pl.S > 1 ? 6ull * pl.S * pl.rows : 0ull;
-        }
-        unsigned long long inc[3] = {v[0], v[1], v[2]};
-        for (uint32_t o = 1; o < 64; o <<= 1)
-            for (int q = 0; q < 3; ++q) {
-                unsigned long long y = __shfl_up(inc[q], o);
-                if (__lane_id() >= o) inc[q] += y;
-            }
-        const uint32_t w = threadIdx.x >> 6;
-        if (__lane_id() == 63)
-            for (int q = 0; q < 3; ++q) wtot[q][w] = inc[q];
-        __syncthreads();
-        unsigned long long tot[3];
-        for (int q = 0; q < 3; ++q) {
-            unsigned long long before = 0ull, all = 0ull;
-            for (uint32_t k = 0; k < BS / 64; ++k) {
-                if (k < w) before += wtot[q][k];
-                all += wtot[q][k];
-            }
-            inc[q] += before + carry[q];  // inclusive, with earlier chunks
-            tot[q] = all;
-        }
-        if (c < e.K) {
-            e.items_pre[c] = inc[0] - v[0];
-            e.fin_pre[c] = inc[1] - v[1];
-            e.part_pre[c] = inc[2] - v[2];
-        }
-        for (int q = 0; q < 3; ++q) carry[q] += tot[q];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        e.items_pre[e.K] = carry[0];
-        e.fin_pre[e.K] = carry[1];
-        e.part_pre[e.K] = carry[2];
-        e.ctl->items = carry[0];
-        e.ctl->fin_units = carry[1];
-    }
-}
-
-__global__ __launch_bounds__(BS) void k_plan(Ens e, int prec) { plan_all(e, prec); }
 
 // ---------------------------------------------------------------------------
 // Exchanges inside a wave
@@ -492,6 +350,131 @@ __device__ __forceinline__ void slot_sums(const double fo[6], uint32_t P, double
         if (!odd) row[q + 2] = y;
     }
 }
+
+// ---------------------------------------------------------------------------
+// Work plan of a step (one workgroup)
+// ---------------------------------------------------------------------------
+
+// Per cluster: lane-group width, j split and work items from its active
+// count; the update workgroups are shared in proportion to nact * n.
+// Exclusive prefix sums over clusters go to items_pre / fin_pre /
+// part_pre, totals to ctl.
+
+// Plan of a single-cluster context, made by every workgroup of the update
+// kernel from the active count (so the device step needs no k_plan
+// launch); workgroup 0 publishes it for the finish pass.
+__device__ __forceinline__ ClPlan plan_single(const Ens &e, int prec,
+                                              unsigned long long &items) {
+    const uint32_t nact = e.cs[0].nact;
+    const ClPlan pl = plan_cluster(e, 0, nact, (double)nact * (double)e.cnt[0],
+                                   prec == H4H_FP64_EXACT, prec == H4H_MIXED,
+                                   nact >= EXACT_WIDE);
+    items = nact ? (unsigned long long)pl.n_it * pl.S : 0ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const uint32_t per = BS / pl.lanes;
+        const unsigned long long units = (nact + per - 1) / per;
+        e.plan[0] = pl;
+        e.items_pre[0] = e.fin_pre[0] = e.part_pre[0] = 0ull;
+        e.items_pre[1] = items;
+        e.fin_pre[1] = units;
+        e.part_pre[1] = (nact && pl.S > 1) ? 6ull * pl.S * pl.rows : 0ull;
+        e.ctl->items = items;
+        e.ctl->fin_units = units;
+    }
+    return pl;
+}
+
+__device__ void plan_all(const Ens &e, int prec) {
+    __shared__ double wsum[5][BS / 64];
+    // nact n of all clusters; the others of ExactLoad for an exact plan
+    const bool exact = prec == H4H_FP64_EXACT;
+    double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (uint32_t c = threadIdx.x; c < e.K; c += BS) {
+        const uint32_t nact = e.cs[c].nact;
+        const double n = (double)e.cnt[c], lanes = (double)((nact + BS - 1) / BS * BS);
+        w[0] += (double)nact * n;
+        w[1] += (double)nact;
+        w[2] += lanes;
+        w[3] += lanes * n;
+        w[4] = nact ? fmax(w[4], n) : w[4];
+    }
+    const uint32_t wave = threadIdx.x >> 6, lane = __lane_id();
+    w[0] = lanes_sum(w[0], 64);
+    if (lane == 0) wsum[0][wave] = w[0];
+    if (exact && e.K > 1) {
+        for (int q = 1; q < 4; ++q) w[q] = lanes_sum(w[q], 64);
+        w[4] = -wave_min(-w[4]);
+        if (lane == 0)
+            for (int q = 1; q < 5; ++q) wsum[q][wave] = w[q];
+    }
+    __syncthreads();
+    double W = 0.0;
+    for (uint32_t k = 0; k < BS / 64; ++k) W += wsum[0][k];
+    bool wide = W >= (double)EXACT_WIDE * (double)e.cnt[0];  // (one system: nact)
+    if (exact && e.K > 1) {
+        ExactLoad l{W, 0.0, 0.0, 0.0, 0.0};
+        for (uint32_t k = 0; k < BS / 64; ++k) {
+            l.act += wsum[1][k];
+            l.lanes += wsum[2][k];
+            l.lane_pairs += wsum[3][k];
+            l.nmax = fmax(l.nmax, wsum[4][k]);
+        }
+        wide = exact_wide(l);
+    }
+    // The plans, and exclusive prefix sums of work items, finish units and
+    // partial doubles over the clusters, BS clusters at a time.
+    __shared__ unsigned long long wtot[3][BS / 64];
+    unsigned long long carry[3] = {0ull, 0ull, 0ull};
+    for (uint32_t base = 0; base < e.K; base += BS) {
+        const uint32_t c = base + threadIdx.x;
+        unsigned long long v[3] = {0ull, 0ull, 0ull};
+        const uint32_t nact = c < e.K ? e.cs[c].nact : 0u;
+        if (nact) {
+            const ClPlan pl = plan_cluster(e, c, nact, W, exact, prec == H4H_MIXED, wide);
+            e.plan[c] = pl;
+            const uint32_t per = BS / pl.lanes;
+            v[0] = (unsigned long long)pl.n_it * pl.S;
+            v[1] = (nact + per - 1) / per;
+            v[2] = pl.S > 1 ? 6ull * pl.S * pl.rows : 0ull;
+        }
+        unsigned long long inc[3] = {v[0], v[1], v[2]};
+        for (uint32_t o = 1; o < 64; o <<= 1)
+            for (int q = 0; q < 3; ++q) {
+                unsigned long long y = __shfl_up(inc[q], o);
+                if (__lane_id() >= o) inc[q] += y;
+            }
+        const uint32_t w = threadIdx.x >> 6;
+        if (__lane_id() == 63)
+            for (int q = 0; q < 3; ++q) wtot[q][w] = inc[q];
+        __syncthreads();
+        unsigned long long tot[3];
+        for (int q = 0; q < 3; ++q) {
+            unsigned long long before = 0ull, all = 0ull;
+            for (uint32_t k = 0; k < BS / 64; ++k) {
+                if (k < w) before += wtot[q][k];
+                all += wtot[q][k];
+            }
+            inc[q] += before + carry[q];  // inclusive, with earlier chunks
+            tot[q] = all;
+        }
+        if (c < e.K) {
+            e.items_pre[c] = inc[0] - v[0];
+            e.fin_pre[c] = inc[1] - v[1];
+            e.part_pre[c] = inc[2] - v[2];
+        }
+        for (int q = 0; q < 3; ++q) carry[q] += tot[q];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        e.items_pre[e.K] = carry[0];
+        e.fin_pre[e.K] = carry[1];
+        e.part_pre[e.K] = carry[2];
+        e.ctl->items = carry[0];
+        e.ctl->fin_units = carry[1];
+    }
+}
+
+__global__ __launch_bounds__(BS) void k_plan(Ens e, int prec) { plan_all(e, prec); }
 
 // ---------------------------------------------------------------------------
 // Predictor / active selection / save old (one workgroup per JT block)
