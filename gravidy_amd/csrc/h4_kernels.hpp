@@ -272,6 +272,21 @@ __host__ __device__ inline uint32_t finish_lanes(uint32_t S, uint32_t nact) {
     return S <= 128 ? 16u : 64u;
 }
 
+// Whether the finish of a block step is one pass over the blocks with active
+// particles (k_finish_blocks), or, for ensembles of many blocks, one over the
+// active particles and one over the blocks (k_finish_correct,
+// k_blockmin_dirty).  The former saves a launch, but has a workgroup's barriers
+// for each block, most of which have one or two active particles: beyond what
+// is resident at once, that is the longer.  Block steps, us, one pass | two, FP64:
+//   1024 blocks (64 clusters of 4096)     79.0 |  81.5
+//   2048 (256 of 2048; 32 of 16384)      120.6 | 119.4, 206.2 | 207.2
+//   2526 (64 of 1024 to 32768)           252.2 | 246.6
+//   4096 (512 of 2048; 64 of 16384)      218.7 | 212.1, 381.7 | 380.6
+constexpr uint32_t FINISH_BLOCKS = 2048;
+__host__ __device__ inline bool finish_by_blocks(uint32_t K, uint32_t nblk) {
+    return K == 1 || nblk <= FINISH_BLOCKS;
+}
+
 // Lane-group width for nact active particles: the widest of 256/64/16/4
 // that keeps at least fill16/16 of the i slots busy (default 12/16), else
 // the least padded.

@@ -1499,6 +1499,35 @@ __global__ __launch_bounds__(BS) void k_finish(Soa s, Ens e, const uint32_t *mov
     }
 }
 
+// The same, with the corrector at the cluster's block time: the finish of a
+// block step of an ensemble of many blocks (finish_by_blocks), after a selection
+// that wrote the active particles' records, whose loads go out with those of
+// the partials.
+__global__ __launch_bounds__(BS) void k_finish_correct(Soa s, Ens e, const uint32_t *move,
+                                                      const double *partial, float eta,
+                                                      double dt_min, double dt_max) {
+    const unsigned long long total = e.ctl->fin_units;
+    for (unsigned long long u = blockIdx.x; u < total; u += gridDim.x) {
+        const uint32_t c = find_cluster(e.fin_pre, e.K, u);
+        const ClPlan pl = e.plan[c];
+        const uint32_t L = pl.lanes;
+        const uint32_t lu = (uint32_t)(u - e.fin_pre[c]);
+        const double T = e.cs[c].atime;
+        const uint32_t k = lu * (BS / L) + threadIdx.x / L;
+        const bool valid = k < e.cs[c].nact;
+        const uint32_t i = valid ? move[e.off[c] + k] : 0u;
+        double o[6], pr[6], dt1 = 0.0;
+        if (valid) load_arec(e, (size_t)e.off[c] + k, o, pr, dt1);
+        double f[6];
+        chunk_sums(s, pl, partial + e.part_pre[c], k, i, valid, f);
+        if (valid && threadIdx.x % L == 0) {
+            correct_store(s, i, o, pr, dt1, f, T, eta, dt_min, dt_max);
+            if (pl.S > 1)
+                for (int q = 0; q < 6; ++q) s.f[q][i] = f[q];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Block times
 // ---------------------------------------------------------------------------
@@ -1564,8 +1593,9 @@ __device__ __forceinline__ double block_tmin(const Soa &s, uint32_t b, double *r
 // each (corr8); with that and DPP sums the average launch of an N = 10007 run
 // takes 6.9 us instead of 8.5, of an N = 65536 run 6.2 instead of 8.2.  For an
 // ensemble it replaces a pass over the active particles with one-lane
-// correctors and one over the blocks (9.7 + 4.0 us on average for 64 clusters
-// of 1024 to 32768).
+// correctors and one over the blocks (k_finish_correct, k_blockmin_dirty; 64
+// clusters of 4096: 12.1 us instead of 8.7 + 4.3), unless it has many blocks
+// (finish_by_blocks).
 template <bool SINGLE>
 __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32_t *move,
                                                      const double *partial, float eta,
@@ -1700,6 +1730,31 @@ __global__ __launch_bounds__(BS) void k_finish_blocks(Soa s, Ens e, const uint32
             e.bmin[b] = m;
             e.bcnt[b] = nm;
         }
+    }
+}
+
+// After k_finish_correct: the minima of the blocks of dirty list `par` (the
+// others did not change), and what k_finish_blocks leaves for the next step.
+__global__ __launch_bounds__(BS) void k_blockmin_dirty(Soa s, Ens e, uint32_t par) {
+    __shared__ double red[BS / 64];
+    if (blockIdx.x == 0 && threadIdx.x == 0) e.ctl->ndirty[par ^ 1] = 0;
+    for (uint32_t c = blockIdx.x * BS + threadIdx.x; c < e.K; c += gridDim.x * BS) {
+        ClState *cs = &e.cs[c];
+        if (cs->done) continue;
+        cs->tail_t = cs->atime;
+        cs->tail_nact = cs->nact;
+        cs->tail_steps = cs->steps;
+        cs->tail_pend = 1;
+        cs->nact = 0;
+    }
+    const uint32_t *dl = e.dirty + (size_t)par * 3 * e.nblk;
+    uint32_t b = dl[3 * blockIdx.x];  // (read with the count, as k_finish_blocks does)
+    const uint32_t nd = e.ctl->ndirty[par];
+    for (uint32_t w = blockIdx.x; w < nd; w += gridDim.x) {
+        if (w != blockIdx.x) b = dl[3 * w];
+        __syncthreads();  // red of the previous block has been read
+        const double m = block_tmin(s, b, red);
+        if (threadIdx.x == 0) e.bmin[b] = m;
     }
 }
 
@@ -3660,7 +3715,8 @@ int ensure_blockmin(h4h_ctx *ctx) {
 // by the next launch that needs its next block time (the next step's
 // selection, k_small_run, or k_tail after h4h_step), so in a device loop
 // that ends, the step after the last one finds the loop stopped.  One
-// system: three launches (its update makes its own plan); an ensemble: four.
+// system: three launches (its update makes its own plan); an ensemble: four,
+// or five (finish_by_blocks).
 // par: the step's slot in its captured chunk, mod 2 (its dirty list); select
 // false: k_small_run has made the selection.  Optional HIP events bracket the update kernel.
 int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par, bool select = true) {
@@ -3676,9 +3732,18 @@ int enqueue_step(h4h_ctx *ctx, bool events, uint32_t par, bool select = true) {
     if (events) H4H_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
     if ((rc = launch_update(ctx, true))) return rc;
     if (events) H4H_HIP(hipEventRecord(ctx->ev[1], ctx->stream));
-    hipLaunchKernelGGL(ctx->K == 1 ? k_finish_blocks<true> : k_finish_blocks<false>,
-                       dim3(std::min<uint32_t>(ctx->nblk, 1024)), dim3(BS), 0, ctx->stream, ctx->s,
-                       ctx->e, ctx->move, ctx->partial, ctx->eta, ctx->dt_min, ctx->dt_max, par);
+    const dim3 grid(std::min<uint32_t>(ctx->nblk, 1024));
+    if (!finish_by_blocks(ctx->K, ctx->nblk)) {
+        hipLaunchKernelGGL(k_finish_correct, dim3(finish_grid(ctx)), dim3(BS), 0, ctx->stream,
+                           ctx->s, ctx->e, ctx->move, ctx->partial, ctx->eta, ctx->dt_min,
+                           ctx->dt_max);
+        H4H_LAUNCHED();
+        hipLaunchKernelGGL(k_blockmin_dirty, grid, dim3(BS), 0, ctx->stream, ctx->s, ctx->e, par);
+    } else {
+        hipLaunchKernelGGL(ctx->K == 1 ? k_finish_blocks<true> : k_finish_blocks<false>, grid,
+                           dim3(BS), 0, ctx->stream, ctx->s, ctx->e, ctx->move, ctx->partial,
+                           ctx->eta, ctx->dt_min, ctx->dt_max, par);
+    }
     H4H_LAUNCHED();
     return H4H_OK;
 }

@@ -76,8 +76,16 @@ static void check_exact() {
     }
 }
 
+// A block step's finish: one pass up to 2048 blocks, two for larger ensembles.
+static void check_finish() {
+    CHECK(finish_by_blocks(1, 1) && finish_by_blocks(1, 100000), "one system");
+    CHECK(finish_by_blocks(2, 2048) && !finish_by_blocks(2, 2049), "two clusters");
+    CHECK(!finish_by_blocks(512, 4096), "512 clusters of 2048");
+}
+
 int main() {
     check_exact();
+    check_finish();
     if (failures) {
         std::printf("%d failures\n", failures);
         return 1;
