@@ -184,10 +184,8 @@ __host__ __device__ inline double dkey_inv(unsigned long long k) {
 // chunk of a narrow group (IW 4 or 16) holds at least 4 tiles, 4K or 16K
 // pairs: shorter items cost more in partial sums than they gain (IW 16),
 // longer ones leave small steps waiting on one item's tile copies (IW 4).
-// (Systems of 5 to TEAM_TILES tiles take one tile per chunk at any width:
-// their small steps are made by one workgroup per tile, k_team_run, with
-// these chunks' sums; so do the larger steps, nact > NARROW_ACT, of single
-// systems of up to 4.)
+// (Fewer in single systems of up to TEAM_TILES tiles and small ensembles of
+// them: one_tile_chunks.)
 // Large active sets of large systems (nact >= 8192 over more than 256
 // tiles) keep chunks of CHUNK_TILES_LARGE tiles: 8 to 32 items per resident
 // workgroup even out the end of the launch, and their finish pass reads
@@ -207,14 +205,32 @@ struct Decomp {
     uint32_t rows;             // n_it * IW: stride of one chunk in partials
 };
 
+// Whether a chunk of a narrow group may be one tile.  In single systems of 5 to
+// TEAM_TILES tiles at any width: their small steps are made by one workgroup
+// per tile, k_team_run, with these chunks' sums, and the launches gain as well
+// (n = 10007 with a tuning table, so without a team: 22.8 -> 21.4 us a step).  In
+// those of up to 4 for the larger steps, nact > NARROW_ACT.  Of an ensemble (share: the cluster's
+// part of its pairs) in clusters of 5 to TEAM_TILES tiles as long as chunks of 4
+// would give all clusters fewer than 256 items, one per CU; more items than
+// that cost in partial sums what they gain.  Block steps, us, chunks of 4 | 1 |
+// by this rule, FP64:
+//   2 clusters of 10000  32.0 | 29.6 | 29.8     64 of 128 to 4096  48.8 |  52.2 |  49.2
+//   8 of 4096            34.5 | 32.7 | 32.2    512 of 1100        129.8 | 139.4 | 130.2
+constexpr uint32_t ITEMS_ONE = 256;
+__host__ __device__ inline bool one_tile_chunks(uint32_t nact, uint32_t iw, uint32_t n_jt,
+                                                bool ensemble, double share) {
+    if (n_jt > TEAM_TILES) return false;
+    if (!ensemble) return n_jt > 4 || nact > NARROW_ACT;
+    return n_jt > 4 && (double)((nact + iw - 1) / iw) * ((n_jt + 3) / 4) < share * ITEMS_ONE;
+}
+
 __host__ __device__ inline Decomp decompose(uint32_t nact, uint32_t iw,
                                             uint32_t n_jt, uint32_t grid,
-                                            uint32_t max_split, bool ensemble = false) {
+                                            uint32_t max_split, bool ensemble = false,
+                                            double share = 1.0) {
     Decomp d;
     d.n_it = (nact + iw - 1) / iw;
-    const bool one_tile =
-        n_jt <= TEAM_TILES && (n_jt > 4 || (!ensemble && nact > NARROW_ACT));
-    uint32_t min_tiles = iw >= 64 || one_tile ? 1u : 4u;
+    uint32_t min_tiles = iw >= 64 || one_tile_chunks(nact, iw, n_jt, ensemble, share) ? 1u : 4u;
     uint32_t S = 1;
     const uint32_t target = grid * QUEUE_FACTOR;
     if (d.n_it > 0 && d.n_it < target) {
@@ -456,7 +472,7 @@ __host__ __device__ __forceinline__ ClPlan plan_cluster(const Ens &e, uint32_t c
                 pl.jrun = 0;
             }
         }
-        Decomp d = decompose(nact, pl.iw, nt, pl.grid, e.max_split, e.K > 1);
+        Decomp d = decompose(nact, pl.iw, nt, pl.grid, e.max_split, e.K > 1, share);
         pl.S = d.S;
         pl.tpc = d.tiles_per_chunk;
         pl.n_it = d.n_it;

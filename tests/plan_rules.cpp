@@ -83,8 +83,27 @@ static void check_finish() {
     CHECK(!finish_by_blocks(512, 4096), "512 clusters of 2048");
 }
 
+// Chunks of one tile in ensembles: only where chunks of four make few items.
+static void check_chunks() {
+    const struct {
+        uint32_t K, n, nact;
+        bool mixed;
+        uint32_t S;
+    } all[] = {{2, 10000, 78, false, 40}, {2, 10000, 78, true, 40},   {8, 4096, 32, false, 16},
+               {512, 1100, 9, false, 2},  {512, 1100, 9, true, 2},    {256, 2048, 16, false, 2},
+               {8, 1000, 8, false, 1},    {2, 70000, 40, false, 69}, {64, 4096, 32, false, 4}};
+    for (const auto &a : all) {
+        const Clusters c(std::vector<uint32_t>(a.K, a.n));
+        const ClPlan pl =
+            plan_cluster(c.e, 0, a.nact, (double)a.K * a.nact * a.n, false, a.mixed, false);
+        CHECK(pl.S == a.S, "%u clusters of %u, %u active: %u chunks of %u, %u slots", a.K, a.n, a.nact,
+              pl.S, pl.tpc, pl.iw);
+    }
+}
+
 int main() {
     check_exact();
+    check_chunks();
     check_finish();
     if (failures) {
         std::printf("%d failures\n", failures);
