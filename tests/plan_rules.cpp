@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <random>
 #include <vector>
 
 using namespace h4;
@@ -101,8 +102,53 @@ static void check_chunks() {
     }
 }
 
+// The plans of random ensembles, as the device makes them, cover their tiles and
+// fit the buffer that their partial sums share (ensemble_partial_bound, or the
+// clusters' own bounds).
+static void check_partials(uint32_t trials, uint32_t grid, uint32_t max_split, bool mixed) {
+    const uint32_t target = grid * QUEUE_FACTOR;
+    std::mt19937_64 rng(20261205 + grid + mixed);
+    for (uint32_t t = 0; t < trials; ++t) {
+        const uint32_t K = 2 + rng() % 80, spread = 1 + rng() % 40000;
+        std::vector<uint32_t> n(K), nact(K);
+        unsigned long long n_total = 0, per_cluster = 0;
+        double W = 0.0;
+        for (uint32_t c = 0; c < K; ++c) {
+            n[c] = 1 + rng() % spread;
+            nact[c] = rng() % 4 == 0 ? 0 : 1 + rng() % (rng() % 2 ? n[c] : std::min(n[c], 600u));
+            n_total += n[c];
+            per_cluster += partial_bound(n[c], target);
+            W += (double)nact[c] * (double)n[c];
+        }
+        Clusters cl(n);
+        cl.e.grid = grid;
+        cl.e.max_split = max_split;
+        unsigned long long used = 0;
+        for (uint32_t c = 0; c < K; ++c) {
+            if (!nact[c]) continue;
+            const ClPlan pl = plan_cluster(cl.e, c, nact[c], W, false, mixed, false);
+            const uint32_t nt = ntiles(cl.e, c);
+            CHECK((unsigned long long)pl.n_it * pl.iw >= nact[c] && pl.rows == pl.n_it * pl.iw &&
+                      (unsigned long long)pl.S * pl.tpc >= nt && (pl.S - 1) * pl.tpc < nt &&
+                      pl.S <= max_split,
+                  "n %u, %u active: %u x %u slots, %u chunks of %u tiles", n[c], nact[c], pl.n_it,
+                  pl.iw, pl.S, pl.tpc);
+            CHECK(!pl.jrun || (mixed && pl.iw == 64), "jrun with %u slots", pl.iw);
+            if (pl.S > 1) used += 6ull * pl.S * pl.rows;
+        }
+        const unsigned long long sum = ensemble_partial_bound(K, n_total, target);
+        CHECK(used <= std::min(per_cluster, sum), "trial %u, K %u: %llu doubles", t, K, used);
+    }
+}
+
 int main() {
     check_exact();
+    for (int mixed = 0; mixed < 2; ++mixed) {
+        check_partials(4000, 4096, 1024, mixed);
+        check_partials(4000, 2048, 1024, mixed);
+        check_partials(2000, 256, 16, mixed);
+        check_partials(2000, 1, 1u << 30, mixed);
+    }
     check_chunks();
     check_finish();
     if (failures) {
