@@ -4788,12 +4788,12 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     if (!large && (small || team_path(ctx))) {
         const OneStep one{itime, ctx->cs_host};
         if ((rc = small ? launch_small(ctx, 1, 0, one) : launch_team(ctx, 1, one))) return rc;
-        if (ctx->timing)
-            for (int k : {0, 1, 3}) H4H_HIP(hipEventRecord(ctx->ev[k], ctx->stream));
+        if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
         if ((rc = await_step(ctx))) return rc;
         if ((rc = check_team(ctx, ctx->cs_host[0].done == STEP_FAILED))) return rc;
     }
-    if (ctx->cs_host[0].done != STEP_DONE) {
+    const bool launches = ctx->cs_host[0].done != STEP_DONE;
+    if (launches) {
         ctx->cs_host[0].done = 0;
         // One-step loop: ATIME = itime, stop after the step.
         hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, (double)INFINITY,
@@ -4809,9 +4809,11 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
         float ms = 0.f;
         H4H_HIP(hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[3]));
         ctx->stats.step_ms += ms;
-        H4H_HIP(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
-        ctx->stats.update_ms += ms;
-        ctx->stats.update_launches += 1;
+        if (launches) {
+            H4H_HIP(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
+            ctx->stats.update_ms += ms;
+            ctx->stats.update_launches += 1;
+        }
     }
     const ClState &cs = ctx->cs_host[0];
     uint32_t k = (uint32_t)cs.nsteps;  // the step's nact (counters were reset)

@@ -57,7 +57,8 @@ typedef struct h4h_stats {
     uint64_t block_steps;      /* h4h_step / update calls               */
     uint64_t interactions;     /* sum of nact * n over updates          */
     uint64_t nsteps;           /* sum of nact                           */
-    uint64_t update_launches;  /* timed update passes                   */
+    uint64_t update_launches;  /* timed update passes (none in a step
+                                  that one kernel makes by itself)      */
     double   update_ms;        /* HIP-event time of the timed passes    */
     double   step_ms;          /* HIP-event time of timed h4h_step calls */
     uint64_t small_steps;      /* block steps made in one workgroup     */
