@@ -1860,6 +1860,7 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
         ctl.ndirty[0] = ctl.ndirty[1] = 0;
         ctl.ndone = t;
         ctl.team_retry = 0;
+        ctl.team_steps = 0;
         ctl.team_err = 0;
         ctl.items = 0;
         ctl.fin_units = 0;
@@ -3082,6 +3083,7 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             cs->steps = steps;
             cs->interactions = inter;
             cs->nsteps = nst;
+            ctl->team_steps += it;
             if (stop) {
                 cs->done = 1;
                 atomicAdd(&ctl->ndone, 1u);
@@ -3457,6 +3459,7 @@ struct h4h_ctx {
     Soa s{};
     Ens e{};
     h4h_stats stats{};
+    uint64_t team_steps = 0;     // block steps made by k_team_run
 };
 
 namespace {
@@ -4793,6 +4796,7 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
         if ((rc = check_team(ctx, ctx->cs_host[0].done == STEP_FAILED))) return rc;
     }
     const bool launches = ctx->cs_host[0].done != STEP_DONE;
+    if (!launches && !small) ctx->team_steps += 1;
     if (launches) {
         ctx->cs_host[0].done = 0;
         // One-step loop: ATIME = itime, stop after the step.
@@ -4877,7 +4881,9 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
         H4H_HIP(hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[3]));
         ctx->stats.step_ms += ms;
     }
-    return read_state(ctx);
+    if ((rc = read_state(ctx))) return rc;
+    ctx->team_steps += ctx->ctl_host->team_steps;
+    return H4H_OK;
 }
 
 int h4h_run(h4h_ctx *ctx, double t_end, double t_stop, uint64_t max_steps, h4h_run_info *io,
@@ -5082,6 +5088,7 @@ int h4h_tune_launch(h4h_ctx *ctx, uint32_t steps, h4h_launch_choice *choice) {
         return H4H_OK;
     };
     const h4h_stats stats0 = ctx->stats;
+    const uint64_t team0 = ctx->team_steps;
     const uint32_t g0 = ctx->grid, s0 = ctx->max_split, f0 = ctx->iw_fill;
     const uint32_t grids[5] = {256, 512, 1024, 2048, 4096};
     const uint32_t splits[4] = {16, 64, 256, 1024};
@@ -5126,6 +5133,7 @@ int h4h_tune_launch(h4h_ctx *ctx, uint32_t steps, h4h_launch_choice *choice) {
     if (!rc2 && hipStreamSynchronize(ctx->stream) != hipSuccess) rc2 = fail(H4H_EHIP, "sync");
     (void)hipFree(save);
     ctx->stats = stats0;
+    ctx->team_steps = team0;
     if (rc) return rc;
     if (rc2) return rc2;
     if (choice) {
@@ -5180,6 +5188,14 @@ int h4h_get_stats(h4h_ctx *ctx, h4h_stats *out, int reset) {
     if (rc) return rc;
     if (out) *out = ctx->stats;
     if (reset) ctx->stats = h4h_stats{};
+    return H4H_OK;
+}
+
+int h4h_team_steps(h4h_ctx *ctx, uint64_t *steps, int reset) {
+    int rc = check_ctx(ctx, false);
+    if (rc) return rc;
+    if (steps) *steps = ctx->team_steps;
+    if (reset) ctx->team_steps = 0;
     return H4H_OK;
 }
 

@@ -154,6 +154,12 @@ class Hermite4HIP:
         check("h4h_get_stats", self.lib.h4h_get_stats(self._ctx, ctypes.byref(s), int(reset)))
         return {k: getattr(s, k) for k, _ in s._fields_}
 
+    def team_steps(self, reset=False):
+        """Block steps made by one workgroup per j tile or two (h4h_team_steps)."""
+        k = ctypes.c_uint64()
+        check("h4h_team_steps", self.lib.h4h_team_steps(self._ctx, ctypes.byref(k), int(reset)))
+        return k.value
+
     # -- transfers -------------------------------------------------------
     def upload(self, r, v, f=None, t=None, dt=None):
         n = self.n

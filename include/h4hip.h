@@ -325,6 +325,16 @@ int h4h_set_graphs(h4h_ctx *ctx, int enable);
 /* Reads and optionally resets the counters. */
 int h4h_get_stats(h4h_ctx *ctx, h4h_stats *out, int reset);
 
+/* Single systems of 1025 to 65536 particles make their small block steps in
+ * one launch of a workgroup per 256 particles (512 beyond 32768), which
+ * exchange through device memory: steps of up to 256 active particles in the
+ * loops up to n = 32768, of up to 128 beyond and in h4h_step; in mixed
+ * precision of up to 191.  Not in exact precision and not with a tuning table.
+ * If the workgroups are not all running at once (other work holds the GPU),
+ * the steps go through the multi-workgroup kernels, with the same results.
+ * Reads and optionally resets the number of steps made so. */
+int h4h_team_steps(h4h_ctx *ctx, uint64_t *steps, int reset);
+
 /* Blocks until all work queued on the context's stream is done. */
 int h4h_synchronize(h4h_ctx *ctx);
 
