@@ -36,6 +36,7 @@ EXPORTS = (
     "h4h_set_tuning", "h4h_autotune", "h4h_set_graphs", "h4h_set_small_path",
     "h4h_tune_launch",
     "h4h_set_launch_choice", "h4h_update_acc_jrk_static", "h4h_team_steps",
+    "h4h_refuse_team",
 )
 
 # Limits of h4h_update_acc_jrk_static (include/h4hip.h).
@@ -144,6 +145,7 @@ def load():
         "h4h_set_timing": ([P, i32], i32),
         "h4h_get_stats": ([P, ctypes.POINTER(H4HStats), i32], i32),
         "h4h_team_steps": ([P, ctypes.POINTER(ctypes.c_uint64), i32], i32),
+        "h4h_refuse_team": ([P], i32),
         "h4h_synchronize": ([P], i32),
         "h4h_create_ensemble": ([pp, u32, pu, dbl, flt, dbl, dbl, i32], i32),
         "h4h_ensemble_sizes": ([P, pu, pu], i32),

@@ -1827,9 +1827,11 @@ __global__ __launch_bounds__(BS) void k_init_dt(Soa s, Ens e, float eta, double 
 // Arms the device step loop of every cluster.  set0: cluster 0 takes
 // (itime0, atime0) first.  A cluster whose ITIME is not < t_end is done
 // at once (the reference's loop test, Hermite4CPU_integration.cpp:81).
+// team_rest: k_team_run leaves that many steps alone first.
 __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_stop,
                                                  unsigned long long max_steps, uint32_t set0,
-                                                 double itime0, double atime0) {
+                                                 double itime0, double atime0,
+                                                 unsigned long long team_rest) {
     __shared__ uint32_t cnt[BS / 64];
     uint32_t nd = 0;
     for (uint32_t c = threadIdx.x; c < e.K; c += BS) {
@@ -1859,7 +1861,7 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
         ctl.max_steps = max_steps;
         ctl.ndirty[0] = ctl.ndirty[1] = 0;
         ctl.ndone = t;
-        ctl.team_retry = 0;
+        ctl.team_retry = team_rest;
         ctl.team_steps = 0;
         ctl.team_err = 0;
         ctl.items = 0;
@@ -1892,7 +1894,7 @@ __device__ __forceinline__ void step_state(ClState *cs, double itime, double ati
 // fields, and when they are there `done`.  (Waiting for the launch itself
 // takes 5 us more, of a step of 18 to 28.)  next: the next block step's
 // active count (tail_nact there; BCNT_MANY or more: not known).
-enum : uint32_t { STEP_DONE = 1, STEP_LEFT = 2, STEP_FAILED = 3 };
+enum : uint32_t { STEP_DONE = 1, STEP_LEFT = 2, STEP_FAILED = 3, STEP_ALONE = 4 };
 template <class T>
 __device__ __forceinline__ void host_store(T *p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -2067,7 +2069,8 @@ __device__ __forceinline__ void small_pairs(const double pi[6], uint32_t i, uint
 // One block step at `itime` without a device loop (h4h_step): the kernels
 // that make whole steps take the loop's state from here instead of the loop
 // control and the cluster record, and write the step's result to the pinned
-// record `host` (STEP_LEFT if they leave the step to others), so that such a
+// record `host` (STEP_LEFT if they leave the step to others, STEP_ALONE if the
+// workgroups of a team did not come together), so that such a
 // step is one launch and no copy.
 struct OneStep {
     double itime;
@@ -3172,9 +3175,12 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
         step_result(one.host, mn, (uint32_t)nst, n, 0, lact[0]);
         step_state(cs, one.itime, mn, (uint32_t)nst, n, 0);
     } else {
-        host_store(&one.host->done, (uint32_t)STEP_LEFT);
+        host_store(&one.host->done, (uint32_t)(go ? STEP_LEFT : STEP_ALONE));
     }
 }
+
+// The decision of the next team made ahead (h4h_refuse_team).
+__global__ void k_team_refuse(Team tm) { agent_store(&tm.sync[TS_DECISION], (uint32_t)TEAM_NO); }
 
 // Every word of a team's buffers waiting (context creation).
 __global__ __launch_bounds__(BS) void k_team_clear(Team tm, size_t words) {
@@ -3438,7 +3444,7 @@ struct h4h_ctx {
     uint32_t *d_dirty = nullptr;
     double *d_bmin = nullptr;    // [nblk], then u32 x nblk counts
     Team team{};                 // exchange buffers of k_team_run (behind d_arec)
-    bool team_ok = false;        // the system has a team's number of tiles
+    bool team_ok = false;        // the system has a team's number of tiles, and the device room
     double4 *d_arec = nullptr;   // the step's active particles' records (Ens::arec)
     uint32_t *d_tune = nullptr;  // [64] tuning table
     // pinned host memory: energy per-workgroup sums, mirrors
@@ -3460,6 +3466,8 @@ struct h4h_ctx {
     Ens e{};
     h4h_stats stats{};
     uint64_t team_steps = 0;     // block steps made by k_team_run
+    uint64_t team_rest = 0;      // coming steps it leaves alone, since its workgroups were
+                                 // not all running
 };
 
 namespace {
@@ -3511,6 +3519,33 @@ void drop_graph(h4h_ctx *ctx) {
 bool team_size(const h4h_ctx *ctx) { return ctx->K == 1 && ctx->nblk > 4 && ctx->nblk <= TEAM_TILES; }
 
 uint32_t team_act(const h4h_ctx *ctx) { return team_act(ctx->nblk > TEAM_ONE ? 2u : 1u); }
+
+auto *team_kernel(bool two, bool mixed, bool one) {
+    return one ? (two ? (mixed ? k_team_run<true, 2, true> : k_team_run<false, 2, true>)
+                      : (mixed ? k_team_run<true, 1, true> : k_team_run<false, 1, true>))
+               : (two ? (mixed ? k_team_run<true, 2, false> : k_team_run<false, 2, false>)
+                      : (mixed ? k_team_run<true, 1, false> : k_team_run<false, 1, false>));
+}
+uint32_t team_wgs(uint32_t nblk) { return nblk > TEAM_ONE ? (nblk + 1) / 2 : nblk; }
+
+// Whether all workgroups of a team of the context's size can run at once on
+// the device (one per CU at least, so a full MI355X holds any; a partition
+// of it may not).
+bool team_fits(const h4h_ctx *ctx) {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess)
+        return false;
+    for (uint32_t k = 0; k < 4; ++k) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, team_kernel(ctx->nblk > TEAM_ONE, k & 1, k & 2), TB, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if ((uint64_t)per_cu * cus < team_wgs(ctx->nblk)) return false;
+    }
+    return true;
+}
 
 // The plans of the active counts a team takes (0: not one chunk per tile,
 // or a tuning table is set).
@@ -3663,13 +3698,8 @@ bool team_path(const h4h_ctx *ctx) {
 }
 
 int launch_team(h4h_ctx *ctx, uint32_t max_run, OneStep one = {}) {
-    const bool two = ctx->nblk > TEAM_ONE, mixed = ctx->precision == H4H_MIXED;
-    auto *kern = one.host
-                     ? (two ? (mixed ? k_team_run<true, 2, true> : k_team_run<false, 2, true>)
-                            : (mixed ? k_team_run<true, 1, true> : k_team_run<false, 1, true>))
-                     : (two ? (mixed ? k_team_run<true, 2, false> : k_team_run<false, 2, false>)
-                            : (mixed ? k_team_run<true, 1, false> : k_team_run<false, 1, false>));
-    hipLaunchKernelGGL(kern, dim3(two ? (ctx->nblk + 1) / 2 : ctx->nblk), dim3(TB), 0, ctx->stream,
+    auto *kern = team_kernel(ctx->nblk > TEAM_ONE, ctx->precision == H4H_MIXED, one.host != nullptr);
+    hipLaunchKernelGGL(kern, dim3(team_wgs(ctx->nblk)), dim3(TB), 0, ctx->stream,
                        ctx->s, ctx->e, ctx->team, max_run, ctx->e2, (double)ctx->eta, ctx->dt_min,
                        ctx->dt_max, one);
     H4H_LAUNCHED();
@@ -4047,7 +4077,7 @@ int create_impl(h4h_ctx **out, uint32_t K, const uint32_t *sizes, double e2, flo
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
         return cleanup(fail(H4H_EHIP, "hipStreamCreate failed"));
     size_t np = ctx->n_dev;
-    ctx->team_ok = team_size(ctx);
+    ctx->team_ok = team_size(ctx) && team_fits(ctx);
     const size_t tm_hdr = 3 * (size_t)ctx->nblk * 8,
                  tm_rec = 3 * (size_t)ctx->nblk * 8 * team_act(ctx),
                  tm_part = (size_t)ctx->nblk * team_act(ctx) * 6, tm_words = tm_hdr + tm_rec + tm_part,
@@ -4784,16 +4814,20 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
     const bool small = small_path(ctx);
     const bool large = ctx->bm_valid && itime == ctx->next_time && ctx->next_nact < BCNT_MANY &&
                        ctx->next_nact > (small ? std::min(ctx->small_act, SMALL_MAX_ACT) : ONE_ACT);
+    const bool team = team_path(ctx) && !ctx->team_rest;
+    if (ctx->team_rest) --ctx->team_rest;
     ctx->next_nact = 0;
     if ((rc = ensure_blockmin(ctx))) return rc;
     if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
     ctx->cs_host[0] = ClState{};
-    if (!large && (small || team_path(ctx))) {
+    if (!large && (small || team)) {
         const OneStep one{itime, ctx->cs_host};
         if ((rc = small ? launch_small(ctx, 1, 0, one) : launch_team(ctx, 1, one))) return rc;
         if (ctx->timing) H4H_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
         if ((rc = await_step(ctx))) return rc;
         if ((rc = check_team(ctx, ctx->cs_host[0].done == STEP_FAILED))) return rc;
+        // (this step and the ones after it, as in a loop)
+        if (ctx->cs_host[0].done == STEP_ALONE) ctx->team_rest = TEAM_BACKOFF - 1;
     }
     const bool launches = ctx->cs_host[0].done != STEP_DONE;
     if (!launches && !small) ctx->team_steps += 1;
@@ -4801,7 +4835,7 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
         ctx->cs_host[0].done = 0;
         // One-step loop: ATIME = itime, stop after the step.
         hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, (double)INFINITY,
-                           -INFINITY, 1ull, 1u, -INFINITY, itime);
+                           -INFINITY, 1ull, 1u, -INFINITY, itime, 0ull);
         H4H_LAUNCHED();
         if ((rc = enqueue_step(ctx, ctx->timing, 0))) return rc;
         hipLaunchKernelGGL(k_tail, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, ctx->cs_host);
@@ -4882,7 +4916,10 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
         ctx->stats.step_ms += ms;
     }
     if ((rc = read_state(ctx))) return rc;
-    ctx->team_steps += ctx->ctl_host->team_steps;
+    const RunCtl &ctl = *ctx->ctl_host;
+    const uint64_t steps = ctx->cs_host[0].steps;
+    ctx->team_steps += ctl.team_steps;
+    ctx->team_rest = ctl.team_retry > steps ? ctl.team_retry - steps : 0;
     return H4H_OK;
 }
 
@@ -4894,7 +4931,8 @@ int h4h_run(h4h_ctx *ctx, double t_end, double t_stop, uint64_t max_steps, h4h_r
     if (max_steps == 0) return fail(H4H_EINVAL, "max_steps must be >= 1");
     if ((rc = ensure_blockmin(ctx))) return rc;
     hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, t_end, t_stop,
-                       (unsigned long long)max_steps, 1u, io->itime, io->atime);
+                       (unsigned long long)max_steps, 1u, io->itime, io->atime,
+                       (unsigned long long)ctx->team_rest);
     H4H_LAUNCHED();
     if ((rc = run_chunks(ctx, step_time, step_nact, max_steps))) return rc;
     const ClState &d = ctx->cs_host[0];
@@ -4939,7 +4977,7 @@ int h4h_ensemble_run(h4h_ctx *ctx, double t_end, double t_stop, uint64_t max_ste
     if (max_steps == 0) return fail(H4H_EINVAL, "max_steps must be >= 1");
     if ((rc = ensure_blockmin(ctx))) return rc;
     hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, t_end, t_stop,
-                       (unsigned long long)max_steps, 0u, 0.0, 0.0);
+                       (unsigned long long)max_steps, 0u, 0.0, 0.0, (unsigned long long)ctx->team_rest);
     H4H_LAUNCHED();
     if ((rc = run_chunks(ctx, nullptr, nullptr, 0))) return rc;
     for (uint32_t c = 0; c < ctx->K; ++c) {
@@ -5188,6 +5226,15 @@ int h4h_get_stats(h4h_ctx *ctx, h4h_stats *out, int reset) {
     if (rc) return rc;
     if (out) *out = ctx->stats;
     if (reset) ctx->stats = h4h_stats{};
+    return H4H_OK;
+}
+
+int h4h_refuse_team(h4h_ctx *ctx) {
+    int rc = check_ctx(ctx, false);
+    if (rc) return rc;
+    if (!ctx->team_ok) return H4H_OK;
+    hipLaunchKernelGGL(k_team_refuse, dim3(1), dim3(1), 0, ctx->stream, ctx->team);
+    H4H_LAUNCHED();
     return H4H_OK;
 }
 

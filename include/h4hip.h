@@ -331,9 +331,14 @@ int h4h_get_stats(h4h_ctx *ctx, h4h_stats *out, int reset);
  * loops up to n = 32768, of up to 128 beyond and in h4h_step; in mixed
  * precision of up to 191.  Not in exact precision and not with a tuning table.
  * If the workgroups are not all running at once (other work holds the GPU),
- * the steps go through the multi-workgroup kernels, with the same results.
+ * that step and the 63 after it go through the multi-workgroup kernels, with
+ * the same results.
  * Reads and optionally resets the number of steps made so. */
 int h4h_team_steps(h4h_ctx *ctx, uint64_t *steps, int reset);
+
+/* Has the next such launch do what it does when its workgroups are not all
+ * running (for tests of that case). */
+int h4h_refuse_team(h4h_ctx *ctx);
 
 /* Blocks until all work queued on the context's stream is done. */
 int h4h_synchronize(h4h_ctx *ctx);
