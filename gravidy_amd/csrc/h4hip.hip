@@ -5276,7 +5276,15 @@ int h4h_update_acc_jrk_static(const double *d_p6, const float *d_pm, uint32_t n,
     const uint32_t n_jt = n_pad / JT;
     const LaneGroup lg =
         lane_group(nact, DEFAULT_IW_FILL, std::min(n_jt, DEFAULT_MAX_SPLIT), mixed);
-    if (precision != H4H_FP64_EXACT && n_jt <= ONE_TILES && nact <= BS && lg.iw <= 64 && !lg.jrun) {
+    // The forces may be written over the particles (d_f6 on d_p6 or d_pm): the one
+    // launch reads those while it writes.
+    auto over = [&](const void *p, size_t bytes) {
+        const uintptr_t f = (uintptr_t)d_f6, x = (uintptr_t)p;
+        return f < x + bytes && x < f + (size_t)n * 48;
+    };
+    const bool apart = !over(d_p6, (size_t)n * 48) && !over(d_pm, (size_t)n * 4);
+    if (precision != H4H_FP64_EXACT && n_jt <= ONE_TILES && nact <= BS && lg.iw <= 64 && !lg.jrun &&
+        apart) {
         const Decomp d = decompose(nact, lg.iw, n_jt, DEFAULT_GRID, DEFAULT_MAX_SPLIT);
         if (d.S == 1) {
             hipLaunchKernelGGL(mixed ? k_static_one<true> : k_static_one<false>, dim3(d.n_it),

@@ -364,6 +364,7 @@ int h4h_synchronize(h4h_ctx *ctx);
  *   d_move : nact uint32 indices < n
  *   d_f6   : n x 6 double (Forces, common.hpp:228-231): rows d_move[k]
  *            receive a[3], a1[3]; other rows are left as they are
+ *            (it may lie over d_p6 or d_pm)
  * e2 and precision as h4h_create; n <= H4H_STATIC_MAX_N, nact <= n (larger
  * sizes are refused with H4H_EINVAL).  The work is queued on `stream` (a
  * hipStream_t; NULL is the null stream) and not waited for.  The results
