@@ -3396,12 +3396,14 @@ constexpr int N_SOA = 35;           // doubles per particle in `state`
 // touched before take longer than the bus: 28 doubles of 262144 particles 8.1
 // -> 3.9 ms into new arrays, 3.4 -> 1.8 ms into used ones (the pieces alone: 2
 // threads 3.2 and 1.7 ms, 4 2.4 and 1.6, 8 1.8 and 1.7; slots of 256 KB: 2.7).
-// Below: 2 threads at most and 256 KB slots, 1 MB in all, which is had in 15 to
-// 40 us (2 MB: 270); a gather, a copy and a wait per array took 0.30 ms at n =
-// 1024 and 0.67 at n = 4096.
+// Below: 256 KB slots, 1 MB in all, which is had in 15 to 40 us (2 MB: 270); a
+// gather, a copy and a wait per array took 0.30 ms at n = 1024 and 0.67 at n =
+// 4096.  From DL_TWO doubles (1 MB) 2 threads, whose start takes as long as one
+// copies 0.5 MB: r of 25000 particles (0.8 MB) 54 us with one, 72 with two, r of
+// 50000 91 and 98, all of 15000 (3.4 MB) into new arrays 0.20 and 0.19 ms.
 constexpr uint32_t DL_THREADS = 4, DL_SLOTS = 2 * DL_THREADS;
 constexpr uint32_t DL_SLOT = 1u << 16, DL_SLOT_SMALL = 1u << 15;  // doubles
-constexpr size_t DL_MIN = 8 * (size_t)DL_SLOT;
+constexpr size_t DL_MIN = 8 * (size_t)DL_SLOT, DL_TWO = 4 * (size_t)DL_SLOT_SMALL;
 }  // namespace
 
 struct h4h_ctx {
@@ -4566,8 +4568,8 @@ int h4h_download(h4h_ctx *ctx, double *r4, double *v4, double *f6, double *time,
         const bool large = t.at[t.n] >= DL_MIN;
         const uint32_t size = large ? DL_SLOT : DL_SLOT_SMALL;
         const uint32_t threads =
-            std::min({large ? DL_THREADS : 2u, (uint32_t)(t.at[t.n] / (2 * (size_t)size)) + 1u,
-                      std::max(1u, std::thread::hardware_concurrency())});
+            std::min(large ? DL_THREADS : t.at[t.n] >= DL_TWO ? 2u : 1u,
+                     std::max(1u, std::thread::hardware_concurrency()));
         const bool slots = make_slots(ctx, 2 * threads, size);
         rc = slots ? download_rows(ctx, t, to, threads, size) : H4H_OK;
         if (current != ctx->device) H4H_HIP(hipSetDevice(current));

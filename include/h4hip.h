@@ -109,7 +109,7 @@ int h4h_upload(h4h_ctx *ctx, const double *r4, const double *v4,
  * old6 is Hermite4::save_old_acc_jrk's h_old, a2/a3 the corrector's
  * h_a2/h_a3.  Call before any Logger / NbodyUtils use of the host arrays
  * (Hermite4CPU_integration.cpp:102-117 reads them at output times).
- * 0.5 MB or more are copied by 2 threads, 4 MB or more by 4, which end before
+ * 1 MB or more are copied by 2 threads, 4 MB or more by 4, which end before
  * the call. */
 int h4h_download(h4h_ctx *ctx, double *r4, double *v4, double *f6,
                  double *t, double *dt, double *old6, double *a2,
