@@ -343,9 +343,12 @@ __host__ __device__ inline uint32_t pick_iw(uint32_t nact, uint32_t fill16 = DEF
 // jrun = 1: each j sub-group then takes 64 consecutive j, so that the FP32
 // runs are the 32 consecutive pairs that 256 slots sum; with 16 slots they
 // would be others.
-// share: of the part, in an ensemble.  (Its clusters of up to 4 tiles keep
-// pick_iw's width: a few steps beside the thousands of k_small_run, 17.0 ms
-// with and without for 256 clusters of 128 to 1024.)
+// share: of the part, in an ensemble.  Its clusters of up to 4 tiles keep
+// pick_iw's width, and with it the order of their sums over the thousands of
+// steps that k_small_run leaves to the launches a few of (256 clusters of 128 to
+// 1024: 50.5 us a step with it, 50.0 narrowed).  Beside a larger cluster, where
+// all their steps are launches, narrower groups would gain: with one of 4096
+// 65.2 us a step, 49.6 narrowed.
 constexpr uint32_t ITEMS_256 = 1024, ITEMS_64 = 512;
 struct LaneGroup {
     uint32_t iw, jrun;
@@ -538,7 +541,7 @@ __device__ __forceinline__ double rsqrt3_fp64(double x) {
     return y * fma(e, 0.8660254037844386, 1.7320508075688772);  // sqrt3 / 2, sqrt3
 }
 
-// Same pair as pair_exact with FMA contraction and rsqrt3_fp64, scaled by
+// Same pair as terms_exact with FMA contraction and rsqrt3_fp64, scaled by
 // 3 sqrt(3) (see PAIR_SCALE):
 //   a  += m r / |r|^3
 //   j  += m/|r|^3 (v - 3 (r.v)/|r|^2 r)

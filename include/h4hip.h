@@ -270,7 +270,9 @@ int h4h_set_tuning(h4h_ctx *ctx, const uint32_t *grid32, const uint32_t *iw32);
  * bucket (nact = 2^b, evenly spaced active particles) over the candidate
  * workgroup shares and lane-group widths, installs the fastest per bucket
  * and returns the table (grid32, iw32: 32 entries each, may be NULL).
- * Leaves the active list empty; call before the integration starts. */
+ * Leaves the active list empty; call before the integration starts.  A table
+ * turns off the steps of h4h_team_steps, which are faster than any table's (n =
+ * 10007: 14.9 us a step without a table, 21.4 with the autotuner's). */
 int h4h_autotune(h4h_ctx *ctx, uint32_t reps, uint32_t *grid32, uint32_t *iw32);
 
 /* Result of h4h_tune_launch. */
