@@ -114,7 +114,8 @@ struct RunCtl {
     unsigned long long fin_units;  // finish workgroup units this step
     unsigned long long team_retry; // k_team_run leaves the steps before this one alone
     unsigned long long team_steps; // block steps made by k_team_run
-    uint32_t team_err, pad_;       // 1: a wait inside k_team_run ran out
+    uint32_t team_err;             // 1: a wait inside k_team_run ran out
+    uint32_t team_fails;           // teams in a row that did not form
     unsigned long long qnext;      // update work queue: items claimed beyond the
                                    // first gridDim.x (zero between launches)
 };

@@ -1827,11 +1827,13 @@ __global__ __launch_bounds__(BS) void k_init_dt(Soa s, Ens e, float eta, double 
 // Arms the device step loop of every cluster.  set0: cluster 0 takes
 // (itime0, atime0) first.  A cluster whose ITIME is not < t_end is done
 // at once (the reference's loop test, Hermite4CPU_integration.cpp:81).
-// team_rest: k_team_run leaves that many steps alone first.
+// team_rest: k_team_run leaves that many steps alone first, team_fails teams in
+// a row not having formed.
 __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_stop,
                                                  unsigned long long max_steps, uint32_t set0,
                                                  double itime0, double atime0,
-                                                 unsigned long long team_rest) {
+                                                 unsigned long long team_rest,
+                                                 uint32_t team_fails) {
     __shared__ uint32_t cnt[BS / 64];
     uint32_t nd = 0;
     for (uint32_t c = threadIdx.x; c < e.K; c += BS) {
@@ -1862,6 +1864,7 @@ __global__ __launch_bounds__(BS) void k_run_setup(Ens e, double t_end, double t_
         ctl.ndirty[0] = ctl.ndirty[1] = 0;
         ctl.ndone = t;
         ctl.team_retry = team_rest;
+        ctl.team_fails = team_fails;
         ctl.team_steps = 0;
         ctl.team_err = 0;
         ctl.items = 0;
@@ -2544,7 +2547,12 @@ constexpr uint32_t team_act(uint32_t tpw) { return tpw == 1 ? 256u : 128u; }
 constexpr uint32_t ONE_ACT = 128;       // of a single step (h4h_step)
 constexpr uint32_t TEAM_ONE = 128;      // tiles up to which a workgroup has one (else two)
 constexpr uint32_t TEAM_WGS = TEAM_TILES / 2;
-constexpr uint32_t TEAM_BACKOFF = 64;   // steps left alone after a team did not form
+// Steps left to the launches after a team did not form: that one, and twice as
+// many each time in a row, up to 64.  (One launch in some thousand after the GPU
+// was idle, and now and then a kernel's first, starts its last workgroup too
+// late; that step takes 80 to 140 us.  With the CUs held by other work every
+// launch does.)
+__host__ __device__ inline uint64_t team_backoff(uint32_t fails) { return 1ull << (fails < 6 ? fails : 6); }
 static_assert(TEAM_ONE <= TEAM_WGS && TEAM_WGS == 128, "workgroups of a team");
 
 // What the workgroups of a team exchange, in device memory.  Every 64-bit
@@ -3087,6 +3095,7 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
             cs->interactions = inter;
             cs->nsteps = nst;
             ctl->team_steps += it;
+            ctl->team_fails = 0;
             if (stop) {
                 cs->done = 1;
                 atomicAdd(&ctl->ndone, 1u);
@@ -3141,8 +3150,11 @@ __global__ __launch_bounds__(TB) void k_team_run(Soa s, Ens e, Team tm, uint32_t
     if (go)
         for (uint32_t k = tid; k < 8 * M; k += TB)
             agent_store(tm.hdr + (size_t)slot * M * 8 + k, SENT);
-    else if (tid == 0)
-        ctl->team_retry = steps + TEAM_BACKOFF;
+    else if (tid == 0 && loop) {
+        const uint32_t fails = ctl->team_fails;
+        ctl->team_retry = steps + team_backoff(fails);
+        ctl->team_fails = fails + 1;
+    }
     if (tid == 0) {
         agent_store(&tm.sync[TS_DECISION], 0u);
         agent_store(&tm.sync[TS_LEFT], 0u);
@@ -3469,7 +3481,8 @@ struct h4h_ctx {
     h4h_stats stats{};
     uint64_t team_steps = 0;     // block steps made by k_team_run
     uint64_t team_rest = 0;      // coming steps it leaves alone, since its workgroups were
-                                 // not all running
+                                 // not all running,
+    uint32_t team_fails = 0;     // so many times in a row (team_backoff)
 };
 
 namespace {
@@ -4829,15 +4842,19 @@ int h4h_step(h4h_ctx *ctx, double itime, uint32_t *nact, double *atime) {
         if ((rc = await_step(ctx))) return rc;
         if ((rc = check_team(ctx, ctx->cs_host[0].done == STEP_FAILED))) return rc;
         // (this step and the ones after it, as in a loop)
-        if (ctx->cs_host[0].done == STEP_ALONE) ctx->team_rest = TEAM_BACKOFF - 1;
+        if (ctx->cs_host[0].done == STEP_ALONE)
+            ctx->team_rest = team_backoff(ctx->team_fails++) - 1;
     }
     const bool launches = ctx->cs_host[0].done != STEP_DONE;
-    if (!launches && !small) ctx->team_steps += 1;
+    if (!launches && !small) {
+        ctx->team_steps += 1;
+        ctx->team_fails = 0;
+    }
     if (launches) {
         ctx->cs_host[0].done = 0;
         // One-step loop: ATIME = itime, stop after the step.
         hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, (double)INFINITY,
-                           -INFINITY, 1ull, 1u, -INFINITY, itime, 0ull);
+                           -INFINITY, 1ull, 1u, -INFINITY, itime, 0ull, 0u);
         H4H_LAUNCHED();
         if ((rc = enqueue_step(ctx, ctx->timing, 0))) return rc;
         hipLaunchKernelGGL(k_tail, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, ctx->cs_host);
@@ -4922,6 +4939,7 @@ static int run_chunks(h4h_ctx *ctx, double *step_time, uint32_t *step_nact, uint
     const uint64_t steps = ctx->cs_host[0].steps;
     ctx->team_steps += ctl.team_steps;
     ctx->team_rest = ctl.team_retry > steps ? ctl.team_retry - steps : 0;
+    ctx->team_fails = ctl.team_fails;
     return H4H_OK;
 }
 
@@ -4934,7 +4952,7 @@ int h4h_run(h4h_ctx *ctx, double t_end, double t_stop, uint64_t max_steps, h4h_r
     if ((rc = ensure_blockmin(ctx))) return rc;
     hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, t_end, t_stop,
                        (unsigned long long)max_steps, 1u, io->itime, io->atime,
-                       (unsigned long long)ctx->team_rest);
+                       (unsigned long long)ctx->team_rest, ctx->team_fails);
     H4H_LAUNCHED();
     if ((rc = run_chunks(ctx, step_time, step_nact, max_steps))) return rc;
     const ClState &d = ctx->cs_host[0];
@@ -4979,7 +4997,8 @@ int h4h_ensemble_run(h4h_ctx *ctx, double t_end, double t_stop, uint64_t max_ste
     if (max_steps == 0) return fail(H4H_EINVAL, "max_steps must be >= 1");
     if ((rc = ensure_blockmin(ctx))) return rc;
     hipLaunchKernelGGL(k_run_setup, dim3(1), dim3(BS), 0, ctx->stream, ctx->e, t_end, t_stop,
-                       (unsigned long long)max_steps, 0u, 0.0, 0.0, (unsigned long long)ctx->team_rest);
+                       (unsigned long long)max_steps, 0u, 0.0, 0.0, (unsigned long long)ctx->team_rest,
+                       ctx->team_fails);
     H4H_LAUNCHED();
     if ((rc = run_chunks(ctx, nullptr, nullptr, 0))) return rc;
     for (uint32_t c = 0; c < ctx->K; ++c) {

@@ -333,8 +333,8 @@ int h4h_get_stats(h4h_ctx *ctx, h4h_stats *out, int reset);
  * loops up to n = 32768, of up to 128 beyond and in h4h_step; in mixed
  * precision of up to 191.  Not in exact precision and not with a tuning table.
  * If the workgroups are not all running at once (other work holds the GPU),
- * that step and the 63 after it go through the multi-workgroup kernels, with
- * the same results.
+ * that step goes through the multi-workgroup kernels, and if it happens again
+ * and again up to 63 steps after it, with the same results.
  * Reads and optionally resets the number of steps made so. */
 int h4h_team_steps(h4h_ctx *ctx, uint64_t *steps, int reset);
 

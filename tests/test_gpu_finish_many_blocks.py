@@ -48,3 +48,24 @@ def test_steps_are_the_clusters(precision, dt_max, steps, pairs):
                 # a step, 2^-24 of it in the FP32 runs
                 tol = 1e-10 if precision == "fp64" else 1e-6
                 assert np.abs(x - y).max() <= tol * max(1.0, np.abs(y).max()), (c, k)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_small_clusters_are_the_same_in_more_company(precision):
+    """Clusters with a workgroup of their own, 2000 blocks and 2200: the plan of
+    a cluster of two tiles does not depend on the others, so the bits agree."""
+    small = [ic.plummer(300, k) for k in range(5)]
+    out = []
+    for count in (1000, 1100):
+        with EnsembleHIP([small[k % 5] for k in range(count)], E2, precision=precision) as e:
+            e.init()
+            info = e.run(2.0 ** -7, 2.0 ** -7)
+            assert e.stats()["small_steps"] > 0
+            out.append((info, e.download()))
+    (a, s), (b, t) = out
+    assert sum(x["steps"] for x in a) > 0
+    for c in (0, 1, 2, 3, 4, 999):
+        assert a[c] == b[c] == b[1000 + c % 5]
+        for k in s[c]:
+            assert bits_equal(s[c][k], t[c][k]), (c, k)
+            assert bits_equal(s[c][k], t[1000 + c % 5][k]), (c, k)

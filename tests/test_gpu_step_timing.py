@@ -30,8 +30,13 @@ def test_update_passes_of_steps(n, largest):
     r, v = ic.plummer(n, 5 * n)
     with Hermite4HIP(r, v, E2) as h:
         _steps(h, r, v, 40)  # (first launches)
-        sizes, st = _steps(h, r, v, 120)
-        assert st["block_steps"] == 120
+        for _ in range(6):
+            sizes, st = _steps(h, r, v, 120)
+            assert st["block_steps"] == 120
+            assert st["update_launches"] >= sum(k > largest for k in sizes)
+            # (workgroups that do not come together leave their step to the launches)
+            if st["update_launches"] == sum(k > largest for k in sizes):
+                break
         assert st["update_launches"] == sum(k > largest for k in sizes)
         assert 0 < st["update_launches"]
         assert (largest == 0) or st["update_launches"] < 120
